@@ -46,7 +46,7 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, vendor figure
 # (the prefill figures are k_gemm_w2's alone, which is built from sx8_gemm.hip and the device
 # headers; the Z/pack pass in sx8_gemv.hip is a kernel of its own)
 SRC_FILES = {"gemv": ("sx8_gemv.hip", "sx8_device.h", "sx8_buffer.h"),
-             "gemm": ("sx8_gemm.hip", "sx8_device.h", "sx8_buffer.h")}
+             "gemm": ("sx8_gemm.hip", "sx8_gemm_ops.h", "sx8_device.h", "sx8_buffer.h")}
 MEASURED = {
     # k_gemv_panel over the layer sweep: mean 6820.9 KiB fetched, 17.1 KiB written per launch
     "gemv_traffic": {"value": (6820.9 * 2.0 + 17.1) * 1024, "src": "gemv", "src_sha16": "81981aeb00e8fc2a",

@@ -28,6 +28,7 @@
 
 #include "sx8_buffer.h"
 #include "sx8_device.h"
+#include "sx8_gemm_ops.h"
 #include "sx8_host.h"
 
 namespace {
@@ -36,19 +37,8 @@ constexpr int kBN = 128;
 constexpr int kThreads = 512;   // waves 0-3 run the MFMAs, waves 4-7 decode weights
 
 typedef float sx8_float16v __attribute__((ext_vector_type(16)));
-typedef uint32_t sx8_u32x4 __attribute__((ext_vector_type(4)));
 
-// Weight sources: the v4.4 layout (hdr + levels) or the kb-major split arrays.
-struct WeightSrc {
-    const uint8_t* hdr;
-    const uint8_t* levels;
-    const uint16_t* dmin;
-    const uint16_t* dmax;
-    const uint8_t* config;
-    const uint8_t* coeff;
-    const uint8_t* hi;
-    const uint8_t* lo;
-};
+using sx8::WeightSrc;
 
 // Matrices of one launch that multiply the same X (q/k/v, gate/up): column tiles are
 // numbered across the group, matrix after matrix; each matrix has its own weights, Zhl
@@ -104,14 +94,14 @@ __device__ __forceinline__ void rec_unpack(const LaneRec& r, uint32_t& lohi, uin
 
 // Range of sub-block sb: rlo = lo + q k1[s], step = max(0.015873 (rhi - rlo), 1e-10) in the
 // reference's float32 form (cuda/sx8_fused_wmma.cu:70-94); the floor binds only for
-// hi <= lo, where every sub-block's step is 1e-10.
+// hi <= lo, where every sub-block's step is 1e-10.  step24 = 2^24 step (sx8_dec_weights).
 __device__ __forceinline__ void sub_range(float lo, float d, float q, float m, uint32_t cfg, int sb,
-                                          float& rlo, float& step) {
+                                          float& rlo, float& step24) {
     const uint32_t s = (cfg >> (2 * sb)) & 3u;
     const float k1 = (float)((0x1300u >> (4 * s)) & 0xFu);        // 0, 0, 3, 1
     const int e = (int)((0x1220u >> (4 * s)) & 0xFu);             // 0, 2, 2, 1
     rlo = __builtin_fmaf(q, k1, lo);
-    step = d > 0.f ? __builtin_ldexpf(m, -e) : 1e-10f;
+    step24 = d > 0.f ? __builtin_ldexpf(m, kStepExp - e) : kStepFloor;
 }
 
 // LDS of one work-group: B operands in lane order, so every MFMA operand read is one
@@ -276,36 +266,14 @@ __device__ __forceinline__ void lds_barrier_keep4() {
     asm volatile("s_barrier" ::: "memory");
 }
 
-__device__ __forceinline__ uint32_t coeff_pair_f16(int c) {
-    const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)(float)c);
-    return h | (h << 16);
-}
-
-// levels of the even (le) and odd (lo) weights of a sub-block, one byte each
-__device__ __forceinline__ void dec_unpack(uint32_t H, uint32_t P, uint32_t& le, uint32_t& lo) {
-    const uint32_t x = __builtin_amdgcn_perm(0u, P, 0x01010000u);        // P0, P0, P1, P1
-    const uint32_t qe = ((x >> 6) & 0x00030003u) | ((x >> 2) & 0x03000300u);   // q0 q2 q4 q6
-    const uint32_t qo = ((x >> 4) & 0x00030003u) | (x & 0x03000300u);          // q1 q3 q5 q7
-    le = ((H & 0x0F0F0F0Fu) << 2) | qe;
-    lo = (((H >> 4) & 0x0F0F0F0Fu) << 2) | qo;
-}
-
-// weights 2j, 2j + 1 of a sub-block as a packed fp16 pair
-__device__ __forceinline__ uint32_t dec_pair(uint32_t le, uint32_t lo, int j, float rlo, float step) {
-    const float we = __builtin_fmaf(step, (float)((le >> (8 * j)) & 0xFFu), rlo);
-    const float wo = __builtin_fmaf(step, (float)((lo >> (8 * j)) & 0xFFu), rlo);
-    const sx8_half2 v = {(_Float16)we, (_Float16)wo};
-    return __builtin_bit_cast(uint32_t, v);
-}
-
 // Decode of this thread's two sub-blocks of a block, in two halves so the decode waves can
 // overlap the second half of block kb with the first half of block kb + 1 (one decode wave
 // per SIMD has no other wave to hide its dependency chains behind).
-// dec_prep: sub-block ranges, level bytes and the PCA coefficient (h = 0: c0, h = 1: c1)
+// dec_prep: sub-block ranges, level words and the PCA coefficient (h = 0: c0, h = 1: c1)
 // as an fp16 pair.
 struct DecPrep {
     float rlo[2], step[2];
-    uint32_t le[2], lv[2];
+    uint32_t H[2], P;
     uint32_t cpair;
 };
 
@@ -317,16 +285,12 @@ __device__ __forceinline__ DecPrep dec_prep(const LaneRec& rec, int h) {
     const float d = hi - lo;
     const float q = d * 0.25f;
     const float mstep = d * 0.015873f;
-    uint32_t Hx, Hy, P;
-    rec_levels<kSplit>(rec, h, Hx, Hy, P);
     DecPrep p;
+    rec_levels<kSplit>(rec, h, p.H[0], p.H[1], p.P);
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
-        sub_range(lo, d, q, mstep, cfg, 2 * h + st, p.rlo[st], p.step[st]);
-        dec_unpack(st ? Hy : Hx, st ? (P >> 16) : P, p.le[st], p.lv[st]);
-    }
+    for (int st = 0; st < 2; ++st) sub_range(lo, d, q, mstep, cfg, 2 * h + st, p.rlo[st], p.step[st]);
     const uint32_t cf = kSplit ? rec.cf : (rec.cc >> 8);
-    p.cpair = coeff_pair_f16(sx8_sext4(cf >> (4 * h)));
+    p.cpair = sx8_coeff_pair_f16(sx8_sext4(cf >> (4 * h)));
     return p;
 }
 
@@ -336,11 +300,11 @@ template <bool kPca>
 __device__ __forceinline__ void dec_finish(GemmSmem& sm, const DecPrep& p, int kb, int b, int wj, int wl,
                                            int h) {
 #pragma unroll
-    for (int st = 0; st < 2; ++st)
-        sm.wt[b][wj][st][wl] = sx8_u32x4{dec_pair(p.le[st], p.lv[st], 0, p.rlo[st], p.step[st]),
-                                         dec_pair(p.le[st], p.lv[st], 1, p.rlo[st], p.step[st]),
-                                         dec_pair(p.le[st], p.lv[st], 2, p.rlo[st], p.step[st]),
-                                         dec_pair(p.le[st], p.lv[st], 3, p.rlo[st], p.step[st])};
+    for (int st = 0; st < 2; ++st) {
+        uint32_t lv[4];
+        sx8_dec_levels(p.H[st], p.P, st ? kQuadHi : kQuadLo, lv);
+        sm.wt[b][wj][st][wl] = sx8_dec_weights(lv, p.rlo[st], p.step[st]);
+    }
     if constexpr (kPca) {
         const int t4 = kb & 3;
         uint32_t* dst = reinterpret_cast<uint32_t*>(&sm.pt[(kb >> 2) & 1][wj][(t4 >> 1) * 32 + (wl & 31)]);
@@ -897,7 +861,7 @@ __device__ __forceinline__ void load_rec1(LaneRec1& r, const LoopSrc<kW2MF>& ls,
 // the arithmetic of dec_prep
 struct DecPrep1 {
     float rlo, step;
-    uint32_t le, lv;
+    uint32_t H, P;
     uint32_t cpair;
 };
 
@@ -909,9 +873,10 @@ __device__ __forceinline__ DecPrep1 dec1_prep(const LaneRec1& rec, int sb) {
     const float d = hi - lo;
     DecPrep1 p;
     sub_range(lo, d, d * 0.25f, d * 0.015873f, cfg, sb, p.rlo, p.step);
-    dec_unpack(rec.qh, rec.ql, p.le, p.lv);
+    p.H = rec.qh;
+    p.P = rec.ql;
     const uint32_t cf = kSplit ? rec.cf : (rec.cc >> 8);
-    p.cpair = coeff_pair_f16(sx8_sext4(cf >> (4 * (sb >> 1))));
+    p.cpair = sx8_coeff_pair_f16(sx8_sext4(cf >> (4 * (sb >> 1))));
     return p;
 }
 
@@ -919,9 +884,9 @@ __device__ __forceinline__ DecPrep1 dec1_prep(const LaneRec1& rec, int sb) {
 // 32 (sb / 2) + c % 32); the even sub-block of a pair stores the coefficient pair
 template <bool kPca>
 __device__ __forceinline__ void dec1_finish(GemmSmem& sm, const DecPrep1& p, int kb, int b, int c, int sb) {
-    sm.wt[b][c >> 5][sb & 1][32 * (sb >> 1) + (c & 31)] =
-        sx8_u32x4{dec_pair(p.le, p.lv, 0, p.rlo, p.step), dec_pair(p.le, p.lv, 1, p.rlo, p.step),
-                  dec_pair(p.le, p.lv, 2, p.rlo, p.step), dec_pair(p.le, p.lv, 3, p.rlo, p.step)};
+    uint32_t lv[4];
+    sx8_dec_levels(p.H, p.P, kQuadLo, lv);
+    sm.wt[b][c >> 5][sb & 1][32 * (sb >> 1) + (c & 31)] = sx8_dec_weights(lv, p.rlo, p.step);
     if constexpr (kPca) {
         if ((sb & 1) == 0) {
             const int t4 = kb & 3;
@@ -1084,7 +1049,11 @@ __global__ __launch_bounds__(kW2Threads) __attribute__((amdgpu_waves_per_eu(2, 2
     read_b(kb0, 0);
 
     // iteration kb (as k_gemm_w1 with 8 MFMAs per k-step): k-step 0 prepares block kb + 3,
-    // k-step 1 finishes block kb + 2 into the ring; PCA k-step at the end of a 4-block group
+    // k-step 1 finishes block kb + 2 into the ring; PCA k-step at the end of a 4-block group.
+    // The preparation is the range arithmetic (~18 instructions) and the finish the level
+    // words and the products (~28): two and four VALU per MFMA.  Measured on gate / down at M =
+    // 2048: 147.1 / 147.7 us a call against 148.5 / 147.7 with four and three, 152 / 151 with
+    // two and six; every lane pair storing its coefficients without the branch cost 4%.
     auto body = [&](int kb, sx8_u32x4 (&acur)[MF][2], sx8_u32x4 (&aprev)[MF][2], LaneRec1& rx,
                     const DecPrep1& pcur, DecPrep1& pnext, const bool pca) __attribute__((always_inline)) {
         const int ka = min(kb + 2, kb1 - 1);
@@ -1102,7 +1071,7 @@ __global__ __launch_bounds__(kW2Threads) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // up to four VALU
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);   // up to two VALU
             if (i < 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);           // a B read
             else if (i < 6) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);      // an A load
         }
@@ -1121,7 +1090,7 @@ __global__ __launch_bounds__(kW2Threads) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);   // up to three VALU
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // up to four VALU
             if (i < 2) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);           // ring writes
             else if (i < 8) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);      // A / record loads
             if (i >= 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);          // B reads
