@@ -155,6 +155,18 @@ int32_t sx8_gemv_group(const uint16_t* X, int32_t n_mats, const uint8_t* const* 
 /* Workspace bytes sx8_gemv needs for n_cb K blocks (112 per block). */
 int64_t sx8_gemv_workspace_bytes(int64_t n_cb);
 
+/* A linear layer on up to 32 rows in one launch: Y (M, N) fp16 = fp16(X . W^T), plus bias (N)
+ * fp16 as an fp16 sum when bias is not NULL.  X (M, K) fp16 with row stride ldx >= K; K and ldx
+ * may be odd, the tail of the last K block counts as zero.  Z is computed inside (its bases
+ * split into two fp16 parts, about 22 bits), the core weights are those of sx8_gemm_prefill;
+ * no workspace.  SX8_ERR_UNSUPPORTED past 32 rows or 2 GiB operands.  Replaces
+ * gemm_compact's call plus the .half() and the bias add of SX8LinearV44.forward
+ * (scripts/integrate_fused_v44.py:43-77). */
+int32_t sx8_linear_f16(const uint16_t* X, int64_t M, int64_t ldx, int64_t K, const uint8_t* hdr,
+                       const uint8_t* levels, int32_t hdr_bytes, const float* basis,
+                       const float* scales, const uint16_t* bias, int64_t N, int64_t n_cb,
+                       uint16_t* Y, void* stream);
+
 /* Workspace bytes of a prefill call over n_mats (1..4) matrices of Ns[i] output columns
  * that share an (M, K) X with n_cb = ceil(K / 32): the PCA operand of every matrix, the
  * packed copy of X and the split-K partials of the plan the call will run.  The same value
@@ -179,7 +191,9 @@ int32_t sx8_gemm_reload_tuning(void);
 /* The plan a prefill call with these sizes runs (for logs and tests): desc[0] tile rows
  * (128, 256 or 512), desc[1] work-groups, desc[2] K ranges, desc[3] K blocks per range,
  * desc[4] whole 512-row tiles before the split tail, desc[5] tiles of the split tail,
- * desc[6] workspace bytes, desc[7] 0.  No counterpart in the reference. */
+ * desc[6] workspace bytes, desc[7] 0.  Calls of at most 128 rows run a wave-level kernel
+ * without tiles or split-K partials (sx8_gemm_small.hip) where its estimated time is below
+ * this plan's; the workspace is the plan's either way.  No counterpart in the reference. */
 int32_t sx8_gemm_prefill_plan(int64_t M, int32_t n_mats, const int64_t* Ns, int64_t n_cb,
                               int64_t* desc);
 

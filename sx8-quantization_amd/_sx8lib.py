@@ -19,7 +19,7 @@ INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 LIB_NAME = "libsx8_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = ["sx8_abi.hip", "sx8_dequant.hip", "sx8_layout.hip", "sx8_quant.hip", "sx8_gemv.hip",
-           "sx8_gemm.hip", "sx8_decoder.hip"]
+           "sx8_gemm.hip", "sx8_gemm_small.hip", "sx8_decoder.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # hipcc flags: gfx950 only, no packed-fp32 instruction selection (those forms have
@@ -54,6 +54,7 @@ SIGNATURES = [
     ("sx8_gemv", _I32, [_P, _P, _P, _I32, _P, _P, _P, _P, _I64, _I64, _P, _P, _I64, _P]),
     ("sx8_gemv_group", _I32, [_P, _I32, _P, _P, _I32, _P, _P, _P, _P, _I64, _P, _P, _I64, _P]),
     ("sx8_gemv_workspace_bytes", _I64, [_I64]),
+    ("sx8_linear_f16", _I32, [_P, _I64, _I64, _I64, _P, _P, _I32, _P, _P, _P, _I64, _I64, _P, _P]),
     ("sx8_gemm_prefill_workspace_bytes", _I64, [_I64, _I32, _P, _I64]),
     ("sx8_gemm_prefill_plan", _I32, [_I64, _I32, _P, _I64, _P]),
     ("sx8_gemm_reload_tuning", _I32, []),
@@ -194,10 +195,16 @@ def lib():
 
 def call(name: str, *args) -> None:
     """Call an entry point and raise RuntimeError with the library's message on error."""
-    L = lib()
-    rc = getattr(L, name)(*args)
+    check(name, getattr(lib(), name)(*args))
+
+
+ERR_UNSUPPORTED = 3
+
+
+def check(name: str, rc: int) -> None:
+    """Raise RuntimeError with the library's message for a non-zero status of `name`."""
     if rc != 0:
-        msg = L.sx8_last_error().decode(errors="replace")
+        msg = lib().sx8_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed (code {rc}): {msg}")
 
 

@@ -1578,6 +1578,7 @@ int32_t run_gemm(const char* what, const uint16_t* X, int64_t M, int64_t ldx, in
     int64_t Ntot = 0, NB = 0;
     if (!group_width(n_mats, Ns, Ntot, NB)) return fail(SX8_ERR_UNSUPPORTED, "%s: group too wide", what);
     const Plan p = plan_gemm(M, Ntot, NB, n_cb, part_cap);
+    const Tuning tu = tuning();
     if (p.G > 0x7FFFFFFF) return fail(SX8_ERR_UNSUPPORTED, "%s: grid too large", what);
     const bool staged = zm != ZMode::kPacked;
     const WsLayout lay = ws_layout(p, M, Ntot, n_cb, n_mats, zm != ZMode::kNone, staged);
@@ -1627,6 +1628,17 @@ int32_t run_gemm(const char* what, const uint16_t* X, int64_t M, int64_t ldx, in
         const int32_t rc = silu_g ? compute_z_silu(silu_g, silu_u, M, ldx, K, zs, n_cb, xp_ws, st)
                                   : compute_z_sets(X, M, ldx, K, zs, n_cb, true, xp_ws, st);
         if (rc != SX8_OK) return rc;
+    }
+    // few rows: the wave-level kernel of sx8_gemm_small.hip where its estimate beats the plan's.
+    // Plan units against measured k_gemm + k_reduce times at 64-128 rows: 6 + 0.65 cost us
+    // (9728 x 2560 20.7, 1024 x 2560 11.6, 2560 x 9728 24.2, 512 x 512 8.0, within 1 us).  It wins up
+    // to 128 rows at K = 2560 and N <= 4096 (14.5 against 18.7 us), up to 64 at N = 9728 (18.4
+    // against 20.7; 80 rows 20.9 against 21.4) or K = 9728 (23.7 against 24.2; 80 rows 28.6 / 24.8)
+    if (zm != ZMode::kNone && !tu.plan && tu.tile == 0 &&
+        gemm_small_us(M, n_mats, Ns, n_cb) < 6.0 + 0.65 * p.cost) {
+        const uint32_t* zh[kMaxGemmGroup];
+        for (int i = 0; i < n_mats; ++i) zh[i] = g.m[i].Zhl;
+        return gemm_small_packed(what, kSplit, hdr_bytes, Xp, M, n_cb, n_mats, ws_in, zh, Ns, Ys, st);
     }
     if constexpr (kSplit) {
         launch_hb<true, true, 6>(p, st, Xp, M, g, n_cb, part);

@@ -3,6 +3,7 @@
 Interface of scripts/integrate_fused_v44.py (reference): ``SX8LinearV44`` and
 ``clone_model_fused_v44``.  Dispatch follows integrate_fused_v44.py:43-77:
   * M == 1                -> decode1_v44 (HIP GEMV, kb-major v4.4 tensors);
+  * 1 < M <= 32           -> linear_sx8 (one HIP launch with the fp16 output and the bias);
   * M > 1                 -> gemm_sx8_compact (HIP MFMA prefill on the same tensors),
                              or gemm_sx8_wmma_cached on kb-major split arrays when
                              SX8_USE_WMMA=1;
@@ -19,7 +20,7 @@ import torch.nn as nn
 from sx8_decode1_v3 import decode1_v44, best_split_k, make_tensors_v44
 from sx8_embed_v44 import SX8EmbeddingV44
 from sx8_fused_wmma import gemm_sx8_wmma_cached, make_tensors, to_kbmajor
-from sx8_gemm_compact import gemm_sx8_compact
+from sx8_gemm_compact import LINEAR_ROWS, gemm_sx8_compact, linear_sx8
 
 DEV = torch.device("cuda")
 
@@ -49,6 +50,11 @@ class SX8LinearV44(nn.Module):
         if x.dim() != 2:
             x = x.reshape(-1, x.shape[-1])
         M = x.shape[0]
+        if 1 < M <= LINEAR_ROWS and self.qt["shape"][0] >= 64 and os.environ.get("SX8_USE_WMMA") != "1":
+            self._load_t44()
+            y = linear_sx8(x, self.qt, *self._t44, self.hdr_bytes, self.bias)
+            if y is not None:
+                return y.reshape(*orig_shape[:-1], self.out_f)
         if M == 1:
             self._load_t44()
             hdr_t, lvl_t, bas_t, sca_t = self._t44

@@ -103,3 +103,30 @@ def gemm_sx8_compact(X, qt, bases_info, hdr_t=None, lvl_t=None, bas_t=None, sca_
             int(hdr_bytes), _L.ptr(bas_t), _L.ptr(sca_t), out_f, int(n_cb), _L.ptr(Y), _L.ptr(ws), nb,
             _L.stream(Xc.device))
     return Y
+
+
+# rows that sx8_linear_f16 takes
+LINEAR_ROWS = 32
+
+
+def linear_sx8(X, qt, hdr_t, lvl_t, bas_t, sca_t, hdr_bytes=6, bias=None):
+    """fp16(X @ W^T) (+ bias) for up to LINEAR_ROWS rows X (M, K) CUDA in one launch
+    (sx8_linear_f16; no counterpart upstream, whose module runs the GEMM, .half() and the bias
+    add).  None when the call is not one it takes: a bias that is not a contiguous fp16 (N,)
+    tensor on X's device or that autograd tracks, or operands past 2 GiB."""
+    out_f, in_f = qt["shape"]
+    if bias is not None and (bias.dtype != torch.float16 or bias.device != X.device or bias.shape != (out_f,)
+                             or not bias.is_contiguous() or (bias.requires_grad and torch.is_grad_enabled())):
+        return None
+    Xc = _x2d(X)
+    M, K = Xc.shape
+    if K < in_f:
+        raise ValueError(f"X has {K} columns, weight needs {in_f}")
+    Y = torch.empty((M, out_f), dtype=torch.float16, device=Xc.device)
+    rc = _L.lib().sx8_linear_f16(_L.ptr(Xc), M, K, int(in_f), _L.ptr(hdr_t), _L.ptr(lvl_t), int(hdr_bytes),
+                                 _L.ptr(bas_t), _L.ptr(sca_t), _L.ptr(bias), out_f, int(qt["n_cb"]), _L.ptr(Y),
+                                 _L.stream(Xc.device))
+    if rc == _L.ERR_UNSUPPORTED:
+        return None
+    _L.check("sx8_linear_f16", rc)
+    return Y

@@ -1,0 +1,138 @@
+"""Few-row GEMMs (sx8_gemm_small.hip): sx8_linear_f16 and the packed form behind the prefill
+entry points at up to 128 rows.  Sizes at the edges of the kernel's tiles: 16-row fragments,
+16 / 32 / 48-column tiles, four-block groups, K tails inside a block and odd rows (whose last
+element shares a word with the next row).  W16 is the oracle's R64 dequant; the bar against its
+float64 product is the other GEMM tests' 1e-3 of max |Y| (weights rounded to fp16), and the
+tiled kernels, forced by SX8_GEMM_TILE, multiply the same fp16 operands, so the two differ by
+the order of float32 sums: at most K 2^-24 sum |x w| / max |Y|, below 1e-5 here."""
+import ctypes
+
+import numpy as np
+import pytest
+
+
+def _quantized(N, K, seed, cuda):
+    import torch
+    from quantize_sx8 import quantize_tensor
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    W = (torch.randn(N, K, generator=g) * 0.02).half()
+    return quantize_tensor(W, device=cuda, degenerate_frac=0.01, seed=seed + 1)
+
+
+def _rel(a, b):
+    return (a.double() - b.double()).abs().max().item() / b.double().abs().max().item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,hb,bias", [
+    (2, 64, 32, 6, False), (3, 80, 31, 8, True), (15, 1000, 1333, 6, True), (16, 2560, 4096, 8, False),
+    (17, 1024, 2560, 6, True), (31, 9728, 515, 6, False), (32, 305, 2081, 8, True), (1, 129, 97, 6, False),
+    (8, 4099, 640, 6, True),
+])
+def test_linear_f16(hiplib, oracle, cuda, M, N, K, hb, bias):
+    """fp16 outputs against the oracle (fp16 rounding on top of the GEMM bar), the bias as an
+    fp16 sum on top, a row stride past K, and the module that calls it."""
+    import torch
+    import _sx8lib as L
+    from integrate_fused_v44 import SX8LinearV44
+    from sx8_decode1_v3 import make_tensors_v44
+    print("linear", M, N, K, hb, flush=True)
+    qt, bi = _quantized(N, K, 31 * M + N, cuda)
+    t = make_tensors_v44(qt, bi, hdr_aligned=(hb == 8))
+    g = torch.Generator(device="cpu").manual_seed(M)
+    wide = torch.randn(M, K + 5, generator=g).half().to(cuda)
+    wide[:, K:] = float("nan")                       # outside the rows: never part of a product
+    X = wide[:, :K].contiguous()
+    b = torch.randn(N, generator=g).half().to(cuda) if bias else None
+    P = L.ptr
+
+    def call(x, ld, bb):
+        Y = torch.full((M, N), 7.0, dtype=torch.float16, device=cuda)
+        L.call("sx8_linear_f16", P(x), M, ld, K, P(t[0]), P(t[1]), hb, P(t[2]), P(t[3]), P(bb), N, qt["n_cb"], P(Y),
+               L.stream(cuda))
+        return Y
+
+    Y = call(X, K, None)
+    ref = oracle.gemm_f64(X.cpu().numpy(), oracle.dequant_r64(qt, bi))
+    err = np.abs(Y.cpu().numpy().astype(np.float64) - ref)
+    assert (err <= 1e-3 * np.abs(ref).max() + 2.0 ** -11 * np.abs(ref)).all()
+    assert torch.equal(call(wide, K + 5, None), Y)
+    if bias:
+        assert torch.equal(call(X, K, b), Y + b)
+    lin = SX8LinearV44(qt, bi, b, hdr_bytes=hb)
+    lin._t44 = t
+    y = lin(X.reshape(1, M, K))
+    assert y.shape == (1, M, N)
+    if M > 1:
+        assert torch.equal(y[0], Y + b if bias else Y)
+        fp32_bias = torch.zeros(N, device=cuda)      # promotes the sum: the unfused path
+        assert SX8LinearV44(qt, bi, fp32_bias, hdr_bytes=hb)(X).dtype == torch.float32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,Ns,K,hb", [
+    (1, [64], 96, 6), (16, [1000], 2560, 8), (17, [129, 300, 64, 700], 80, 6), (33, [4096, 1024, 1024], 2560, 6),
+    (48, [777], 1000, 6), (49, [513], 4096, 8), (64, [9728], 640, 6), (65, [640], 1333, 6), (80, [1001], 515, 8),
+    (96, [300, 500], 2081, 6), (97, [256], 129, 6), (128, [2560], 2560, 6),
+])
+def test_packed_forms_match_tiles(hiplib, oracle, cuda, gemm_tuning, M, Ns, K, hb):
+    """sx8_gemm_prefill_group against the oracle, against the tiled kernels, and against the
+    split-array and caller-Z contracts of the same product."""
+    import torch
+    import _sx8lib as L
+    from sx8_decode1_v3 import make_tensors_v44
+    from sx8_fused_wmma import gemm_sx8_wmma_cached, make_tensors, to_kbmajor
+    from sx8_gemm_compact import _ext
+    print("packed", M, Ns, K, hb, flush=True)
+    mats = [_quantized(N, K, 900 + 7 * i + M, cuda) for i, N in enumerate(Ns)]
+    ts = [make_tensors_v44(qt, bi, hdr_aligned=(hb == 8)) for qt, bi in mats]
+    n, n_cb = len(Ns), mats[0][0]["n_cb"]
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half().to(cuda)
+    arr = lambda i: (ctypes.c_void_p * n)(*[t[i].data_ptr() for t in ts])
+
+    def group():
+        ys = [torch.full((M, N), float("nan"), device=cuda) for N in Ns]
+        ws, nb = L.gemm_workspace(M, Ns, n_cb, cuda)
+        L.call("sx8_gemm_prefill_group", L.ptr(X), M, K, K, n, arr(0), arr(1), hb, arr(2), arr(3),
+               (ctypes.c_int64 * n)(*Ns), n_cb, (ctypes.c_void_p * n)(*[y.data_ptr() for y in ys]), L.ptr(ws), nb,
+               L.stream(cuda))
+        return ys
+
+    ys = group()
+    assert all(torch.equal(a, b) for a, b in zip(ys, group()))      # deterministic
+    gemm_tuning(TILE="256")
+    tiles = group()
+    gemm_tuning(TILE=None)
+    for (qt, bi), y, yt in zip(mats, ys, tiles):
+        ref = oracle.gemm_f64(X.cpu().numpy(), oracle.dequant_r64(qt, bi))
+        assert oracle.rel_err(y.cpu().numpy(), ref) <= 1e-3
+        assert _rel(y, yt) <= 1e-5
+    if n == 1:
+        qt, bi = mats[0]
+        assert torch.equal(gemm_sx8_wmma_cached(X, make_tensors(to_kbmajor(qt, bi)[0], bi, cuda), n_cb), ys[0])
+        Xp = torch.zeros(M, n_cb * 32, dtype=torch.float16, device=cuda)
+        Xp[:, :K] = X
+        Z = _ext().compute_z44_batch(Xp, ts[0][2], ts[0][3], n_cb)
+        assert torch.equal(_ext().gemm_compact(Xp, ts[0][0], ts[0][1], Z, n_cb, hb), ys[0])
+
+
+def test_linear_f16_refusals(hiplib):
+    """Bad arguments and sizes past the kernel's are turned into errors on the host."""
+    L, p = hiplib, ctypes.c_void_p(4096)
+    N0 = ctypes.c_void_p(None)
+    ok = [p, 4, 64, 64, p, p, 6, p, p, N0, 128, 2, p, N0]
+
+    def call(**kw):
+        a = list(ok)
+        for k, v in kw.items():
+            a[int(k[1:])] = v
+        return L.sx8_linear_f16(*a)
+
+    assert call(a0=N0) == 1 and call(a12=N0) == 1 and call(a7=N0) == 1
+    assert call(a6=7) == 1                            # header width
+    assert call(a2=63) == 1 and call(a11=3) == 1      # row stride below K; n_cb != ceil(K / 32)
+    assert call(a1=0) == 1 and call(a10=0) == 1
+    assert call(a5=ctypes.c_void_p(4100)) == 1        # levels misaligned
+    assert call(a1=33) == 3                           # rows
+    assert call(a10=1 << 27) == 3                     # levels past 2 GiB
+    assert b"at most 32 rows" in L.sx8_last_error()
