@@ -4,6 +4,8 @@
 // Hugging Face Qwen modules driven by scripts/infer_sx8.py:109-173.)  Each is one launch
 // that reads its position from device memory, so a whole decode step can be captured in
 // a HIP graph and replayed.
+#include <type_traits>
+
 #include "sx8_buffer.h"
 #include "sx8_device.h"
 #include "sx8_host.h"
@@ -723,7 +725,16 @@ __global__ __launch_bounds__(256) void k_qk_rope128(const float* __restrict__ q_
 // ms per token on one box: 8 chunks 1.589, 12 1.534, 16 1.534, 24 1.557, 32 1.569.  (A
 // chunk count derived from *pos on the device was slower, 1.66: the combine's loads then
 // wait for that read.)
-constexpr int kAttnChunks = 16;
+// Caches longer than kAttnLongL positions get as many chunks (16, 32 or 64) as fill the 256 CUs
+// with one work-group each, never shorter than kAttnMinT positions (one pass of the lane
+// groups); work-groups past the last chunk write an empty partial and stop.  With 16 chunks and
+// 8 KV heads only half the CUs stream the cache.  Split + combine, 32/8 heads of 128, us with 16
+// / 32 / 64 chunks: position 2000 8.5 / 7.7 / 10.2, 8000 17.1 / 12.9 / 14.4, 24000 42.8 / 26.6 /
+// 25.4 (the combine reads every chunk's partials); 4 KV heads at 8000 26.1 / 17.5 / 14.3, 16 KV
+// heads of 64 at 8000 10.2 / 10.7 / 10.8.  A long cache at an early position costs at most 0.3 us
+// (position 700 of 4096: 7.2 / 7.5 / 9.9).
+constexpr int kAttnChunks = 16, kAttnMaxChunks = 64, kAttnMinT = 64;
+constexpr int64_t kAttnLongL = 2048;
 constexpr int64_t kAttnSplitMaxL = (int64_t)1 << 20;
 
 // Inputs of the RoPE-fused form (kRope): the raw f32 projections and what
@@ -819,7 +830,7 @@ __device__ __forceinline__ void rope_apply(const RopeRow& r, int c, float eps, u
     for (int e = 0; e < 4; ++e) o[e] = (uint32_t)f2h(res[2 * e]) | ((uint32_t)f2h(res[2 * e + 1]) << 16);
 }
 
-template <int HD, int G, bool kRope = false>
+template <int HD, int G, bool kRope = false, int NC = kAttnChunks>
 __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__ q,
                                                     const uint16_t* __restrict__ k_cache,
                                                     const uint16_t* __restrict__ v_cache,
@@ -837,12 +848,21 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
     __shared__ float sm[PG][G], sl[PG][G];
     __shared__ float sacc[PG][G][HD + 4];
     __shared__ uint32_t rq[kRope ? G : 1][HD / 2], rk[HD / 2], rv[HD / 2];   // RoPE'd rows (fp16 pairs)
-    const int kv = blockIdx.x / kAttnChunks, chunk = blockIdx.x % kAttnChunks;
+    const int kv = blockIdx.x / NC, chunk = blockIdx.x % NC;
     const int64_t pos = *pos_p;
     const int n = (int)min(max(pos, (int64_t)0) + 1, (int64_t)L);
-    const int T = (n + kAttnChunks - 1) / kAttnChunks;
+    const int T = max((n + NC - 1) / NC, NC > kAttnChunks ? kAttnMinT : 0);
     const int jb = chunk * T, je = min(jb + T, n);
     const int tid = threadIdx.x, c = tid % CH, pg = tid / CH;
+    if constexpr (NC > kAttnChunks) {
+        if (jb >= n) {                       // (uniform; a chunk past the positions never owns *pos)
+            for (int t = tid; t < G * (HD + 2); t += 256) {
+                const int g = t / (HD + 2), e = t - g * (HD + 2);
+                part[((int64_t)(kv * G + g) * NC + chunk) * (HD + 2) + e] = e == 0 ? -INFINITY : 0.f;
+            }
+            return;
+        }
+    }
     // kRope: the new position's row (pos inside the cache and inside this chunk) comes from
     // LDS, not from the cache this launch is writing
     const bool own_new = kRope && pos >= 0 && pos < L && pos >= jb && pos < je;
@@ -865,16 +885,19 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
     asm volatile("" ::: "memory");
     const uint16_t* kc = k_cache + (int64_t)kv * L * HD;
     const uint16_t* vc = v_cache + (int64_t)kv * L * HD;
-    sx8_u32x4 kr[kU], vr[kU];
-    auto load_rows = [&](int j0) {
-#pragma unroll
-        for (int u = 0; u < kU; ++u)
-            kr[u] = *reinterpret_cast<const sx8_u32x4*>(kc + (int64_t)min(j0 + u * PG, je - 1) * HD + 8 * c);
-#pragma unroll
-        for (int u = 0; u < kU; ++u)
-            vr[u] = *reinterpret_cast<const sx8_u32x4*>(vc + (int64_t)min(j0 + u * PG, je - 1) * HD + 8 * c);
+    struct Rows {
+        sx8_u32x4 k[kU], v[kU];
     };
-    load_rows(jb + pg);
+    Rows r0, r1;
+    auto load_rows = [&](Rows& r, int j0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+            r.k[u] = *reinterpret_cast<const sx8_u32x4*>(kc + (int64_t)min(j0 + u * PG, je - 1) * HD + 8 * c);
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+            r.v[u] = *reinterpret_cast<const sx8_u32x4*>(vc + (int64_t)min(j0 + u * PG, je - 1) * HD + 8 * c);
+    };
+    load_rows(r0, jb + pg);
     __builtin_amdgcn_sched_barrier(0);       // no RoPE math (which waits for its rows) above here
 
     // (3) kRope: norm + RoPE of the G q rows and the new k row in parallel (one lane group
@@ -928,7 +951,9 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
 #pragma unroll
         for (int e = 0; e < 8; ++e) a[g][e] = 0.f;
     }
-    for (int j0 = jb + pg; j0 < je;) {
+    // (the rows of the next pass are requested ahead of a pass's arithmetic, where every pass
+    // used to wait for its own: 500 positions per chunk 18.7 -> 17.1 us, one pass 7.32 -> 7.14)
+    auto pass = [&](const Rows& rw, int j0) __attribute__((always_inline)) {
         float s[kU][G];
         float vf[kU][8];
 #pragma unroll
@@ -940,7 +965,7 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     // (through a scalar: a bit_cast of a vector-element lvalue reads element 0)
-                    const uint32_t kw = is_new ? knew[e] : kr[u][e];
+                    const uint32_t kw = is_new ? knew[e] : rw.k[u][e];
                     sc = __builtin_amdgcn_fdot2(__builtin_bit_cast(sx8_half2, qv[g][e]),
                                                 __builtin_bit_cast(sx8_half2, kw), sc, false);
                 }
@@ -949,7 +974,7 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const uint32_t vw = is_new ? vnew[e] : vr[u][e];
+                const uint32_t vw = is_new ? vnew[e] : rw.v[u][e];
                 vf[u][2 * e] = h2f((uint16_t)(vw & 0xFFFFu));
                 vf[u][2 * e + 1] = h2f((uint16_t)(vw >> 16));
             }
@@ -972,8 +997,14 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
             }
             m[g] = mx;
         }
-        j0 += kU * PG;
-        if (j0 < je) load_rows(j0);
+    };
+    constexpr int kStep = kU * PG;
+    for (int jr = jb; jr < je; jr += 2 * kStep) {          // jr uniform; lane group's position jr + pg
+        if (jr + kStep < je) load_rows(r1, jr + kStep + pg);
+        if (jr + pg < je) pass(r0, jr + pg);
+        if (jr + kStep >= je) break;
+        if (jr + 2 * kStep < je) load_rows(r0, jr + 2 * kStep + pg);
+        if (jr + kStep + pg < je) pass(r1, jr + kStep + pg);
     }
     if (c == 0)
 #pragma unroll
@@ -1000,7 +1031,7 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
                 den += wi * sl[i][g];
             }
         }
-        float* ph = part + ((int64_t)(kv * G + g) * kAttnChunks + chunk) * (HD + 2);
+        float* ph = part + ((int64_t)(kv * G + g) * NC + chunk) * (HD + 2);
         ph[2 + d] = num;
         if (d == 0) {
             ph[0] = M;
@@ -1009,27 +1040,48 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
     }
 }
 
-template <int HD>
-__global__ __launch_bounds__(HD) void k_attn_combine(const float* __restrict__ part,
-                                                     uint16_t* __restrict__ out) {
-    const int h = blockIdx.x, d = threadIdx.x;
-    const float* ph = part + (int64_t)h * kAttnChunks * (HD + 2);
-    float mc[kAttnChunks], lc[kAttnChunks], ac[kAttnChunks];
+// NC / 16 groups of HD threads per head, 16 chunks each, then the groups in order.
+template <int HD, int NC = kAttnChunks>
+__global__ __launch_bounds__(HD * (NC / 16)) void k_attn_combine(const float* __restrict__ part,
+                                                                 uint16_t* __restrict__ out) {
+    constexpr int kQ = NC / 16;
+    const int h = blockIdx.x, d = threadIdx.x % HD, q = kQ > 1 ? threadIdx.x / HD : 0;
+    const float* ph = part + ((int64_t)h * NC + 16 * q) * (HD + 2);
+    float mc[16], lc[16], ac[16];
 #pragma unroll
-    for (int c = 0; c < kAttnChunks; ++c) {      // every load of the head issued at once
+    for (int c = 0; c < 16; ++c) {               // every load of the head issued at once
         mc[c] = ph[c * (HD + 2)];
         lc[c] = ph[c * (HD + 2) + 1];
         ac[c] = ph[c * (HD + 2) + 2 + d];
     }
     float M = mc[0];                             // chunk 0 always holds position 0
 #pragma unroll
-    for (int c = 1; c < kAttnChunks; ++c) M = fmaxf(M, mc[c]);
+    for (int c = 1; c < 16; ++c) M = fmaxf(M, mc[c]);
+    __shared__ float gm[kQ], gl[kQ][HD], ga[kQ][HD];
+    if constexpr (kQ > 1) {
+        if (d == 0) gm[q] = M;
+        __syncthreads();
+        M = gm[0];
+#pragma unroll
+        for (int i = 1; i < kQ; ++i) M = fmaxf(M, gm[i]);
+    }
     float num = 0.f, den = 0.f;
 #pragma unroll
-    for (int c = 0; c < kAttnChunks; ++c) {
+    for (int c = 0; c < 16; ++c) {
         const float wc = __expf(mc[c] - M);      // empty chunk: e^-inf = 0, l = acc = 0
         num += wc * ac[c];
         den += wc * lc[c];
+    }
+    if constexpr (kQ > 1) {
+        ga[q][d] = num;
+        gl[q][d] = den;
+        __syncthreads();
+        if (q != 0) return;
+#pragma unroll
+        for (int i = 1; i < kQ; ++i) {
+            num += ga[i][d];
+            den += gl[i][d];
+        }
     }
     out[h * HD + d] = f2h(num / den);
 }
@@ -1810,8 +1862,37 @@ extern "C" int32_t sx8_dec_attn_prefill_packed(const uint16_t* q, const uint16_t
     return check_launch(what);
 }
 
+// partials of one call: (m, l, acc[hd]) per head and chunk
+static int64_t attn_ws_bytes(int64_t nh, int64_t hd, int64_t chunks) {
+    return nh > 0 && hd > 0 ? nh * chunks * (hd + 2) * (int64_t)sizeof(float) : 0;
+}
+
+// Chunks of a call (see kAttnLongL), as far as the workspace holds their partials.
+static int attn_chunks(int64_t L, int64_t nh, int64_t nk, int64_t hd, int64_t workspace_bytes) {
+    int nc = kAttnChunks;
+    if (L > kAttnLongL)
+        while (nc < kAttnMaxChunks && nk * nc < 256 && workspace_bytes >= attn_ws_bytes(nh, hd, 2 * nc)) nc *= 2;
+    return nc;
+}
+
+// f(integral_constant<chunks>) for a chunk count
+template <typename F>
+static void by_chunks(int nc, F&& f) {
+    if (nc == kAttnChunks) f(std::integral_constant<int, kAttnChunks>{});
+    else if (nc == 32) f(std::integral_constant<int, 32>{});
+    else f(std::integral_constant<int, kAttnMaxChunks>{});
+}
+
 extern "C" int64_t sx8_dec_attn_workspace_bytes(int32_t nh, int32_t hd) {
-    return nh > 0 && hd > 0 ? (int64_t)nh * kAttnChunks * (hd + 2) * (int64_t)sizeof(float) : 0;
+    return attn_ws_bytes(nh, hd, kAttnMaxChunks);
+}
+
+template <int HD>
+static void launch_combine(int nc, int nh, const float* part, uint16_t* out, hipStream_t st) {
+    by_chunks(nc, [&](auto c) {
+        constexpr int NC = decltype(c)::value;
+        hipLaunchKernelGGL((k_attn_combine<HD, NC>), dim3((unsigned)nh), dim3(HD * NC / 16), 0, st, part, out);
+    });
 }
 
 extern "C" int32_t sx8_dec_attn_split(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
@@ -1826,23 +1907,26 @@ extern "C" int32_t sx8_dec_attn_split(const uint16_t* q, const uint16_t* k_cache
         (hd != 64 && hd != 128) || L <= 0 || L > kAttnSplitMaxL)
         return fail(SX8_ERR_INVALID, "sx8_dec_attn_split: bad shape (nh / nk in {1, 2, 4, 8}, hd 64 or "
                                      "128, cache length <= %lld)", (long long)kAttnSplitMaxL);
-    if (workspace_bytes < sx8_dec_attn_workspace_bytes(nh, hd) || !aligned(workspace, 16))
+    if (workspace_bytes < attn_ws_bytes(nh, hd, kAttnChunks) || !aligned(workspace, 16))
         return fail(SX8_ERR_INVALID, "sx8_dec_attn_split: workspace needs %lld bytes, 16-byte aligned",
-                    (long long)sx8_dec_attn_workspace_bytes(nh, hd));
+                    (long long)attn_ws_bytes(nh, hd, kAttnChunks));
     if (!aligned(q, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16))
         return fail(SX8_ERR_INVALID, "sx8_dec_attn_split: q and caches must be 16-byte aligned");
     float* part = reinterpret_cast<float*>(workspace);
     const hipStream_t st = as_stream(stream);
-    const dim3 grid((unsigned)(nk * kAttnChunks));
-#define SX8_ATTN(HDV, GV)                                                                           \
-    hipLaunchKernelGGL((k_attn_split<HDV, GV>), grid, dim3(256), 0, st, q, k_cache, v_cache, pos,  \
-                       part, (int)L, scale)
+    const int nc = attn_chunks(L, nh, nk, hd, workspace_bytes);
+    const dim3 grid((unsigned)(nk * nc));
+#define SX8_ATTN(HDV, GV)                                                                                    \
+    by_chunks(nc, [&](auto c) {                                                                              \
+        hipLaunchKernelGGL((k_attn_split<HDV, GV, false, decltype(c)::value>), grid, dim3(256), 0, st, q,     \
+                           k_cache, v_cache, pos, part, (int)L, scale);                                      \
+    })
     if (hd == 128) {
         if (G == 1) SX8_ATTN(128, 1); else if (G == 2) SX8_ATTN(128, 2); else if (G == 4) SX8_ATTN(128, 4); else SX8_ATTN(128, 8);
-        hipLaunchKernelGGL(k_attn_combine<128>, dim3((unsigned)nh), dim3(128), 0, st, part, out);
+        launch_combine<128>(nc, nh, part, out, st);
     } else {
         if (G == 1) SX8_ATTN(64, 1); else if (G == 2) SX8_ATTN(64, 2); else if (G == 4) SX8_ATTN(64, 4); else SX8_ATTN(64, 8);
-        hipLaunchKernelGGL(k_attn_combine<64>, dim3((unsigned)nh), dim3(64), 0, st, part, out);
+        launch_combine<64>(nc, nh, part, out, st);
     }
 #undef SX8_ATTN
     return check_launch("sx8_dec_attn_split");
@@ -1864,25 +1948,28 @@ extern "C" int32_t sx8_dec_attn_rope(const float* q_raw, const float* k_raw, con
         (hd != 64 && hd != 128) || L <= 0 || L > kAttnSplitMaxL)
         return fail(SX8_ERR_INVALID, "%s: bad shape (nh / nk in {1, 2, 4, 8}, hd 64 or 128, cache length "
                                      "<= %lld)", what, (long long)kAttnSplitMaxL);
-    if (workspace_bytes < sx8_dec_attn_workspace_bytes(nh, hd) || !aligned(workspace, 16))
+    if (workspace_bytes < attn_ws_bytes(nh, hd, kAttnChunks) || !aligned(workspace, 16))
         return fail(SX8_ERR_INVALID, "%s: workspace needs %lld bytes, 16-byte aligned", what,
-                    (long long)sx8_dec_attn_workspace_bytes(nh, hd));
+                    (long long)attn_ws_bytes(nh, hd, kAttnChunks));
     if (!aligned(q_raw, 16) || !aligned(k_raw, 16) || !aligned(v_raw, 16) || !aligned(q_norm, 16) ||
         !aligned(k_norm, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16))
         return fail(SX8_ERR_INVALID, "%s: projections, norm weights and caches must be 16-byte aligned", what);
     RopeIn ri{q_raw, k_raw, v_raw, q_norm, k_norm, cos_t, sin_t, k_cache, v_cache, eps};
     float* part = reinterpret_cast<float*>(workspace);
     const hipStream_t st = as_stream(stream);
-    const dim3 grid((unsigned)(nk * kAttnChunks));
-#define SX8_ATTN(HDV, GV)                                                                               \
-    hipLaunchKernelGGL((k_attn_split<HDV, GV, true>), grid, dim3(256), 0, st, nullptr, k_cache, v_cache, \
-                       pos, part, (int)L, scale, ri)
+    const int nc = attn_chunks(L, nh, nk, hd, workspace_bytes);
+    const dim3 grid((unsigned)(nk * nc));
+#define SX8_ATTN(HDV, GV)                                                                                    \
+    by_chunks(nc, [&](auto c) {                                                                              \
+        hipLaunchKernelGGL((k_attn_split<HDV, GV, true, decltype(c)::value>), grid, dim3(256), 0, st, nullptr, \
+                           k_cache, v_cache, pos, part, (int)L, scale, ri);                                  \
+    })
     if (hd == 128) {
         if (G == 1) SX8_ATTN(128, 1); else if (G == 2) SX8_ATTN(128, 2); else if (G == 4) SX8_ATTN(128, 4); else SX8_ATTN(128, 8);
-        hipLaunchKernelGGL(k_attn_combine<128>, dim3((unsigned)nh), dim3(128), 0, st, part, out);
+        launch_combine<128>(nc, nh, part, out, st);
     } else {
         if (G == 1) SX8_ATTN(64, 1); else if (G == 2) SX8_ATTN(64, 2); else if (G == 4) SX8_ATTN(64, 4); else SX8_ATTN(64, 8);
-        hipLaunchKernelGGL(k_attn_combine<64>, dim3((unsigned)nh), dim3(64), 0, st, part, out);
+        launch_combine<64>(nc, nh, part, out, st);
     }
 #undef SX8_ATTN
     return check_launch(what);
