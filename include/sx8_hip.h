@@ -159,7 +159,7 @@ int64_t sx8_gemv_workspace_bytes(int64_t n_cb);
  * fp16 as an fp16 sum when bias is not NULL.  X (M, K) fp16 with row stride ldx >= K; K and ldx
  * may be odd, the tail of the last K block counts as zero.  Z is computed inside (its bases
  * split into two fp16 parts, about 22 bits), the core weights are those of sx8_gemm_prefill;
- * no workspace.  SX8_ERR_UNSUPPORTED past 32 rows or 2 GiB operands.  Replaces
+ * one row runs sx8_gemv's arithmetic (float32 weights; at most 640 K blocks).  No workspace.  SX8_ERR_UNSUPPORTED past 32 rows or 2 GiB operands.  Replaces
  * gemm_compact's call plus the .half() and the bias add of SX8LinearV44.forward
  * (scripts/integrate_fused_v44.py:43-77). */
 int32_t sx8_linear_f16(const uint16_t* X, int64_t M, int64_t ldx, int64_t K, const uint8_t* hdr,

@@ -611,11 +611,13 @@ extern "C" int32_t sx8_linear_f16(const uint16_t* X, int64_t M, int64_t ldx, int
     if (hdr_bytes != 6 && hdr_bytes != 8)
         return fail(SX8_ERR_INVALID, "%s: hdr_bytes must be 6 or 8, got %d", what, hdr_bytes);
     if (!aligned(hdr, hdr_bytes == 8 ? 8 : 2) || !aligned(levels, 8) || !aligned(X, 2) || !aligned(Y, 2) ||
-        !aligned(basis, 16) || !aligned(scales, 8) || !aligned(bias, 2))
+        !aligned(basis, M == 1 ? 4 : 16) || !aligned(scales, M == 1 ? 4 : 8) || !aligned(bias, 2))
         return fail(SX8_ERR_INVALID, "%s: misaligned pointer", what);
     if (M <= 0 || K <= 0 || N <= 0 || n_cb <= 0 || n_cb * 32 < K || (n_cb - 1) * 32 >= K || ldx < K || N > 0x7FFFFFFF)
         return fail(SX8_ERR_INVALID, "%s: bad shape M=%lld K=%lld ldx=%lld N=%lld n_cb=%lld", what, (long long)M,
                     (long long)K, (long long)ldx, (long long)N, (long long)n_cb);
+    if (M == 1 && N <= 0x7FFFFFFF / 2 && n_cb <= 0x7FFFFFFF / 64)
+        return gemv_linear(what, hdr_bytes, X, K, hdr, levels, basis, scales, bias, N, n_cb, Y, as_stream(stream));
     if (M > kLinearRows || M * ldx * 2 > 0x7FFFFFFF || N * n_cb * 24 > 0x7FFFFFFF || gemm_small_us(M, 1, &N, n_cb) >= 1e300)
         return fail(SX8_ERR_UNSUPPORTED, "%s: at most %lld rows and operands below 2 GiB", what, (long long)kLinearRows);
     WeightSrc w{};

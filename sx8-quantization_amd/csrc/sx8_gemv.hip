@@ -508,7 +508,10 @@ __device__ __forceinline__ void tab_store(KbInfo* info, const TabIn& t, int kb, 
 //           resid_out (the next residual; it must not alias resid or delta, which the other
 //           work-groups are still reading).
 //   kXSilu: x = fp16(silu(g) * u) = fp16(g / (1 + exp(-g)) * u).
-constexpr int kXPlain = 0, kXRms = 1, kXSilu = 2;
+//   kXLinear (one matrix): x read as fp16, of any length K <= 32 n_cb and alignment (the rest
+//           counts as zero), and the output y = fp16(W x), plus an fp16 bias as an fp16 sum: a
+//           linear layer's row without the passes that pad x, convert y and add the bias.
+constexpr int kXPlain = 0, kXRms = 1, kXSilu = 2, kXLinear = 3;
 struct XProd {
     const float* resid;
     const uint16_t* init;
@@ -740,18 +743,22 @@ template <int HB, int kMode, int NR, int TP, int kX = kXPlain, bool kOne = false
           bool kResY = false>
 __global__ __launch_bounds__(kPanelThreads) void k_gemv_panel(
     const uint8_t* __restrict__ hdr0, const uint8_t* __restrict__ lv0, const uint16_t* __restrict__ X,
-    int N0, int n_cb, const float* __restrict__ bas0, const float* __restrict__ sca0,
+    int N0, int n_cb_pad, const float* __restrict__ bas0, const float* __restrict__ sca0,
     float* __restrict__ Y0, const GemvGroup grp,
     const KbInfo* __restrict__ table, const XProd xp) {
     extern __shared__ __align__(16) unsigned char smem[];
     float* red = reinterpret_cast<float*>(smem);                 // 2 x 512 floats
     KbInfo* info = reinterpret_cast<KbInfo*>(smem + sizeof(float) * 2 * kPanelThreads);
     const int tid = threadIdx.x;
+    // kXLinear: the values missing to 32 n_cb ride in the upper half of the preloaded count
+    constexpr bool kLin = kX == kXLinear;
+    const int n_cb = kLin ? n_cb_pad & 0xFFFF : n_cb_pad;
+    const int Kx = n_cb * 32 - (kLin ? n_cb_pad >> 16 : 0);
     // The producer's inputs go out before anything else: with kPre they need no argument
     // load (a group's matrix fields are a memory round trip away).
-    XRaw xr[kX == kXPlain ? 1 : TP];
+    XRaw xr[kX == kXPlain || kLin ? 1 : TP];
     constexpr bool kBuild = kMode == 1 || kMode == 2 || kMode == 4;   // table built in-kernel
-    if constexpr (kBuild && kX != kXPlain) {
+    if constexpr (kBuild && kX != kXPlain && !kLin) {
         XRsrc xs;
         if constexpr (kPre) xs = xraw_rsrc_pre<kX>(X, hdr0, n_cb * 32);
         else xs = xraw_rsrc<kX>(xp, n_cb * 32);
@@ -802,7 +809,25 @@ __global__ __launch_bounds__(kPanelThreads) void k_gemv_panel(
     // them after the geometry).
     const int n_units = n_cb * 4;
     TabIn tin[TP];
+    const sx8_rsrc rx = make_rsrc(kLin ? xa : nullptr, kLin ? (int64_t)Kx * 2 : 0);
+    auto load_lin = [&](int u) { return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, u * 16, 0, 0)); };
+    // K odd: the last value shares its 4-byte word with the end of x (which reads zero)
+    uint32_t x_last = 0;
+    auto fix_lin = [&](uint4& x, int u) {
+        const int w = (Kx - 1 - 8 * u) >> 1;
+        if ((Kx & 1) && w >= 0 && w < 4) {
+            x.x = w == 0 ? x_last : x.x;
+            x.y = w == 1 ? x_last : x.y;
+            x.z = w == 2 ? x_last : x.z;
+            x.w = w == 3 ? x_last : x.w;
+        }
+    };
     if constexpr (kBuild) {
+        if constexpr (kLin) {
+            if (Kx & 1) x_last = __builtin_amdgcn_raw_buffer_load_b16(rx, (Kx - 1) * 2, 0, 0);
+#pragma unroll
+            for (int p = 0; p < TP; ++p) tin[p].x = load_lin(min(p * kPanelThreads + tid, n_units - 1));
+        }
 #pragma unroll
         for (int p = 0; p < TP; ++p) {
             const int u = min(p * kPanelThreads + tid, n_units - 1);
@@ -858,6 +883,12 @@ __global__ __launch_bounds__(kPanelThreads) void k_gemv_panel(
     if constexpr (kResY) {
         if (tid < CT && col_ok) yres = *(const g_float*)(Y0 + n);
     }
+    uint16_t ybias = 0;                      // kXLinear: this column's bias (in the add slot)
+    const uint16_t* bias = nullptr;
+    if constexpr (kLin) {
+        bias = reinterpret_cast<const uint16_t*>(grp.m[0].add);
+        if (bias && tid < CT && col_ok) ybias = *to_global(bias + n);
+    }
     if constexpr (kMode == 0) {
         const uint4* src = reinterpret_cast<const uint4*>(table);
         uint4* dst = reinterpret_cast<uint4*>(info);
@@ -894,15 +925,23 @@ __global__ __launch_bounds__(kPanelThreads) void k_gemv_panel(
                 tin[p].x = make_uint4(xw[0], xw[1], xw[2], xw[3]);
             }
         }
+        if constexpr (kLin) {
+#pragma unroll
+            for (int p = 0; p < TP; ++p) fix_lin(tin[p].x, min(p * kPanelThreads + tid, n_units - 1));
+        }
 #pragma unroll
         for (int p = 0; p < TP; ++p) {
             const int u = p * kPanelThreads + tid;
             tab_store<kMode>(info, tin[p], min(u, n_units - 1) >> 2, u & 3, u < n_units, n_cb);
         }
-        if constexpr (kX == kXPlain) {
+        if constexpr (kX == kXPlain || kLin) {
             for (int u0 = TP * kPanelThreads; u0 < n_units; u0 += kPanelThreads) {
                 const int u = min(u0 + tid, n_units - 1);
-                tab_load<kMode>(tin[0], Xg, basis, scales, Zin, u >> 2, u & 3);
+                tab_load<kMode, !kLin>(tin[0], Xg, basis, scales, Zin, u >> 2, u & 3);
+                if constexpr (kLin) {
+                    tin[0].x = load_lin(u);
+                    fix_lin(tin[0].x, u);
+                }
                 tab_store<kMode>(info, tin[0], u >> 2, u & 3, u0 + tid < n_units, n_cb);
             }
         }
@@ -980,11 +1019,18 @@ __global__ __launch_bounds__(kPanelThreads) void k_gemv_panel(
         // residual epilogue: h = resid + W x, each element read and written by this thread
         if constexpr (kResY) {
             t = yres + t;
-        } else {
+        } else if constexpr (!kLin) {
             const float* __restrict__ add = kOne ? grp.m[0].add : pick([](const GemvMat& g) { return g.add; });
             if (add) t = *(const g_float*)(add + n) + t;
         }
-        *(float SX8_GLOBAL_AS*)(Y + n) = t;
+        if constexpr (kLin) {
+            asm volatile("" : "+v"(t));      // rounded to float32 before the conversion
+            _Float16 h = (_Float16)t;
+            if (bias) h = h + __builtin_bit_cast(_Float16, ybias);
+            *(uint16_t SX8_GLOBAL_AS*)(reinterpret_cast<uint16_t*>(Y) + n) = __builtin_bit_cast(uint16_t, h);
+        } else {
+            *(float SX8_GLOBAL_AS*)(Y + n) = t;
+        }
         yv = t;
     }
     // argmax partials (lm_head): the panel's best column -- larger value, or equal value and
@@ -1132,7 +1178,7 @@ void launch_panel(const PanelPlan& p, size_t smem, hipStream_t st, const uint16_
     // instantiated forms: kPre with kXRms only for groups, kPre with kXSilu and kResY only
     // for single matrices
     constexpr bool kAllowOne = !(kPre && kX == kXRms);
-    constexpr bool kAllowGroup = !(kPre && kX == kXSilu) && !kResY;
+    constexpr bool kAllowGroup = !(kPre && kX == kXSilu) && !kResY && kX != kXLinear;
     const uint8_t* h0 = (kPre && kX == kXRms) ? reinterpret_cast<const uint8_t*>(xp.w) : m0.hdr;
     // a single matrix with Z given (kMode 2) takes Z in the basis slot, which is preloaded
     const float* b0 = kMode == 2 ? m0.Zin : m0.basis;
@@ -1306,6 +1352,29 @@ extern "C" int32_t sx8_compute_z(const uint16_t* X, int64_t M, int64_t ldx, cons
         return fail(SX8_ERR_INVALID, "sx8_compute_z: misaligned pointer (basis 16 B, Z 8 B)");
     return compute_z(X, M, ldx, n_cb * 32, basis, scales, n_cb, Z, false, nullptr, as_stream(stream));
 }
+
+namespace sx8 {
+
+int32_t gemv_linear(const char* what, int32_t hdr_bytes, const uint16_t* X, int64_t K, const uint8_t* hdr,
+                    const uint8_t* levels, const float* basis, const float* scales, const uint16_t* bias, int64_t N,
+                    int64_t n_cb, uint16_t* Y, hipStream_t st) {
+    const PanelPlan p = plan_panels(&N, 1, (int)n_cb);
+    if (n_cb > kLdsMaxKb || !offsets_fit(p, N, n_cb))
+        return fail(SX8_ERR_UNSUPPORTED, "%s: one row of %lld x %lld blocks (at most %d K blocks, 32-bit offsets)", what,
+                    (long long)N, (long long)n_cb, kLdsMaxKb);
+    GemvGroup g{};
+    g.n_mats = 1;
+    g.ct = p.CT;
+    g.m[0] = GemvMat{hdr, levels, basis, scales, nullptr, reinterpret_cast<float*>(Y),
+                     reinterpret_cast<const float*>(bias), (int)N, (int)p.grid};
+    const size_t smem = panel_smem((int)n_cb, true);
+    const int n_cb_pad = (int)n_cb | (int)(n_cb * 32 - K) << 16;
+    if (hdr_bytes == 8) launch_panel<8, 1, kXLinear>(p, smem, st, X, g, nullptr, n_cb_pad);
+    else launch_panel<6, 1, kXLinear>(p, smem, st, X, g, nullptr, n_cb_pad);
+    return check_launch(what);
+}
+
+}  // namespace sx8
 
 extern "C" int32_t sx8_gemv(const uint16_t* X, const uint8_t* hdr, const uint8_t* levels,
                             int32_t hdr_bytes, const float* basis, const float* scales,

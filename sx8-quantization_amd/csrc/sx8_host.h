@@ -56,6 +56,7 @@ int32_t compute_z_silu(const float* g, const float* u, int64_t M, int64_t ld, in
 // for shapes it does not take (M > kSmallRows, 32-bit record indices).  _packed: f32 outputs
 // from the prefill GEMM's packed operands.  _raw: one v4.4 matrix, at most kLinearRows plain fp16
 // rows, Z computed inside, fp16 output y = fp16(W x) (+ bias, an fp16 sum).  Launch only.
+// gemv_linear: _raw's one-row form on the GEMV (sx8_gemv.hip).
 constexpr int64_t kSmallRows = 128, kLinearRows = 32;
 struct WeightSrc;
 double gemm_small_us(int64_t M, int n_mats, const int64_t* Ns, int64_t n_cb);
@@ -65,5 +66,8 @@ int32_t gemm_small_packed(const char* what, bool split, int32_t hdr_bytes, const
 int32_t gemm_small_raw(const char* what, int32_t hdr_bytes, const uint16_t* X, int64_t M, int64_t ldx, int64_t K,
                        int64_t n_cb, const WeightSrc& w, const float* basis, const float* scales,
                        const uint16_t* bias, int64_t N, uint16_t* Y, hipStream_t st);
+int32_t gemv_linear(const char* what, int32_t hdr_bytes, const uint16_t* X, int64_t K, const uint8_t* hdr,
+                    const uint8_t* levels, const float* basis, const float* scales, const uint16_t* bias, int64_t N,
+                    int64_t n_cb, uint16_t* Y, hipStream_t st);
 
 }  // namespace sx8

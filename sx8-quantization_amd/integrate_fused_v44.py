@@ -2,8 +2,10 @@
 
 Interface of scripts/integrate_fused_v44.py (reference): ``SX8LinearV44`` and
 ``clone_model_fused_v44``.  Dispatch follows integrate_fused_v44.py:43-77:
-  * M == 1                -> decode1_v44 (HIP GEMV, kb-major v4.4 tensors);
-  * 1 < M <= 32           -> linear_sx8 (one HIP launch with the fp16 output and the bias);
+  * M <= 32               -> linear_sx8 (one HIP launch with the fp16 output and the bias: the
+                             GEMV for one row, the few-row GEMM for more);
+  * M == 1 otherwise      -> decode1_v44 (a row that is not in_f long, more than 640 K blocks,
+                             a bias that is not fp16);
   * M > 1                 -> gemm_sx8_compact (HIP MFMA prefill on the same tensors),
                              or gemm_sx8_wmma_cached on kb-major split arrays when
                              SX8_USE_WMMA=1;
@@ -50,7 +52,8 @@ class SX8LinearV44(nn.Module):
         if x.dim() != 2:
             x = x.reshape(-1, x.shape[-1])
         M = x.shape[0]
-        if 1 < M <= LINEAR_ROWS and self.qt["shape"][0] >= 64 and os.environ.get("SX8_USE_WMMA") != "1":
+        if M == 1 or (1 < M <= LINEAR_ROWS and self.qt["shape"][0] >= 64 and
+                      os.environ.get("SX8_USE_WMMA") != "1"):
             self._load_t44()
             y = linear_sx8(x, self.qt, *self._t44, self.hdr_bytes, self.bias)
             if y is not None:

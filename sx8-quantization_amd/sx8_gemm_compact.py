@@ -120,6 +120,8 @@ def linear_sx8(X, qt, hdr_t, lvl_t, bas_t, sca_t, hdr_bytes=6, bias=None):
         return None
     Xc = _x2d(X)
     M, K = Xc.shape
+    if M == 1 and K != in_f:                 # decode1_v44 pads or cuts the row
+        return None
     if K < in_f:
         raise ValueError(f"X has {K} columns, weight needs {in_f}")
     Y = torch.empty((M, out_f), dtype=torch.float16, device=Xc.device)

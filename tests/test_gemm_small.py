@@ -70,6 +70,32 @@ def test_linear_f16(hiplib, oracle, cuda, M, N, K, hb, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,K,hb,bias", [
+    (1024, 2560, 6, False), (2560, 9728, 8, True), (33, 31, 6, True), (300, 97, 8, False), (777, 1333, 6, True),
+    (4097, 4095, 8, True), (129, 4098, 6, False), (100, 16390, 6, True), (70001, 64, 6, True),
+])
+def test_one_row_equals_gemv(hiplib, cuda, N, K, hb, bias):
+    """One row through sx8_linear_f16 is bit for bit decode1_v44's float32 result converted
+    (and the bias added): widths at the panel forms' edges, K tails inside a block and odd K,
+    table passes past the up-front ones, a row 2 bytes off 16-byte alignment."""
+    import torch
+    from sx8_decode1_v3 import decode1_v44, make_tensors_v44
+    from sx8_gemm_compact import linear_sx8
+    print("one row", N, K, hb, flush=True)
+    qt, bi = _quantized(N, K, N + K, cuda)
+    t = make_tensors_v44(qt, bi, hdr_aligned=(hb == 8))
+    g = torch.Generator(device="cpu").manual_seed(K)
+    buf = torch.full((K + 1,), float("nan"), dtype=torch.float16, device=cuda)
+    buf[1:] = torch.randn(K, generator=g).half().to(cuda)
+    x = buf[1:]
+    b = torch.randn(N, generator=g).half().to(cuda) if bias else None
+    y = decode1_v44(x.clone(), qt, bi, *t, hdr_bytes=hb)[0].half()
+    assert torch.equal(linear_sx8(x[None], qt, *t, hb, b)[0], y + b if bias else y)
+    assert torch.equal(linear_sx8(x.clone()[None], qt, *t, hb, None)[0], y)
+    assert linear_sx8(buf[None], qt, *t, hb, None) is None          # not in_f long: decode1_v44's rules
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,Ns,K,hb", [
     (1, [64], 96, 6), (16, [1000], 2560, 8), (17, [129, 300, 64, 700], 80, 6), (33, [4096, 1024, 1024], 2560, 6),
     (48, [777], 1000, 6), (49, [513], 4096, 8), (64, [9728], 640, 6), (65, [640], 1333, 6), (80, [1001], 515, 8),
