@@ -113,6 +113,20 @@ int32_t sx8_v6_encode(const uint16_t* W, int64_t out_f, int64_t in_f, int64_t ld
                       uint16_t* dmin, uint16_t* dmax, uint8_t* config, uint8_t* levels_hi,
                       uint8_t* levels_lo, void* stream);
 
+/* The PCA half of the quantizer (pca_correct_gpu, scripts/quantize_qwen35_4b_sx8_v43_gpu.py:75-142)
+ * on the V6 fields of n_rows x n_cb blocks (n-major): per K block the two leading right singular
+ * vectors of the residuals (float64 Gram matrix, largest component positive) as data (n_cb, 64)
+ * f32, scales (n_cb, 2) f32 = max(lower median |c| / 3, 1e-10), coeff (n_rows * n_cb) = two signed
+ * 4-bit coefficients.  blocks (n_rows * n_cb, 32), dmin and dmax all fp16 (is_f16 = 1) or all f32;
+ * levels (.., 32) u8 8-byte aligned; workspace 16-byte aligned, sx8_quant_pca_workspace_bytes (-1
+ * for a bad shape).  Weights with NaN give NaN scales. */
+int64_t sx8_quant_pca_workspace_bytes(int64_t n_rows, int64_t n_cb);
+int32_t sx8_quant_pca(const void* blocks, const void* dmin, const void* dmax, int32_t is_f16,
+                      const uint8_t* levels, const uint8_t* config, int64_t n_rows, int64_t n_cb,
+                      uint8_t* coeff, float* data, float* scales, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+
+
 /* PCA precompute Z[m, kb, j] = scales[kb, j] * sum_t X[m, kb*32+t] * basis[kb, 32j+t]
  * for m < M, in float32 with the reference's summation tree.
  * Replaces compute_z44 (cuda/sx8_decode1_v3.cu:185-195, kernel :44-65) for M = 1 and

@@ -3,9 +3,9 @@
 // levels) and the level packing, written straight into the pkl / container split arrays.
 //
 // Role of v6_encode_6bit_gpu and pack_levels_6bit
-// (scripts/quantize_qwen35_4b_sx8_v43_gpu.py:22-47, :148-167).  The PCA half (per-K-block
-// bases from the residuals) stays a batched Gram / eigen decomposition in torch: it is a
-// few hundred 32 x 32 problems per tensor.
+// (scripts/quantize_qwen35_4b_sx8_v43_gpu.py:22-47, :148-167).  The PCA half (pca_correct_gpu,
+// :75-142: per K block the two leading right singular vectors of the residuals, the
+// coefficients and their scales) follows below, sx8_quant_pca.
 //
 // Arithmetic (binary32, every operation rounded, no contraction), per block:
 //   dmin, dmax = min, max of the 32 weights; d = max(dmax - dmin, 1e-10); q = d / 4;
@@ -29,7 +29,7 @@ constexpr int kThreads = 256;
 __global__ __launch_bounds__(kThreads) void k_v6_encode(
     const uint16_t* __restrict__ W, int64_t out_f, int64_t in_f, int64_t ld, int64_t n_cb,
     uint8_t* __restrict__ levels, uint16_t* __restrict__ dmin_out, uint16_t* __restrict__ dmax_out,
-    uint8_t* __restrict__ config_out, uint8_t* __restrict__ hi_out, uint8_t* __restrict__ lo_out) {
+    uint8_t* __restrict__ config_out, uint8_t* __restrict__ hi_out, uint8_t* __restrict__ lo_out, bool vec_out) {
 #pragma clang fp contract(off)
     const int64_t bid = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (bid >= out_f * n_cb) return;
@@ -106,15 +106,373 @@ __global__ __launch_bounds__(kThreads) void k_v6_encode(
     }
     uint8_t* ho = hi_out + bid * 16;
     uint8_t* lo = lo_out + bid * 8;
+    if (vec_out) {
+        *reinterpret_cast<uint4*>(ho) = make_uint4(h[0], h[1], h[2], h[3]);
+        *reinterpret_cast<uint2*>(lo) = make_uint2(l[0], l[1]);
+    } else {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) ho[k] = (uint8_t)(h[k >> 2] >> (8 * (k & 3)));
+        for (int k = 0; k < 16; ++k) ho[k] = (uint8_t)(h[k >> 2] >> (8 * (k & 3)));
 #pragma unroll
-    for (int k = 0; k < 8; ++k) lo[k] = (uint8_t)(l[k >> 2] >> (8 * (k & 3)));
+        for (int k = 0; k < 8; ++k) lo[k] = (uint8_t)(l[k >> 2] >> (8 * (k & 3)));
+    }
     if (levels) {
         uint8_t* lvo = levels + bid * 32;
+        uint32_t w[8];
 #pragma unroll
-        for (int t = 0; t < 32; ++t) lvo[t] = lv_best[t];
+        for (int t = 0; t < 8; ++t)
+            w[t] = (uint32_t)lv_best[4 * t] | ((uint32_t)lv_best[4 * t + 1] << 8) |
+                   ((uint32_t)lv_best[4 * t + 2] << 16) | ((uint32_t)lv_best[4 * t + 3] << 24);
+        if (vec_out) {
+            reinterpret_cast<uint4*>(lvo)[0] = make_uint4(w[0], w[1], w[2], w[3]);
+            reinterpret_cast<uint4*>(lvo)[1] = make_uint4(w[4], w[5], w[6], w[7]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 32; ++t) lvo[t] = lv_best[t];
+        }
     }
+}
+
+// ---------------------------------------------------------------- PCA of the residuals
+// Five passes over a tensor of n_rows x n_cb blocks (bid = row * n_cb + kb):
+//   k_pca_err     residuals e = x - (lo + step lv) in float32 (every operation rounded, the
+//                 steps as products with fp32(1 / 63)), stored K block by K block
+//   k_pca_gram    partial Gram matrices E^T E of row ranges, float64 on the matrix core
+//   k_pca_eig     their sum's two leading eigenvectors by cyclic Jacobi rotations
+//   k_pca_coeff   c = basis . e (float64 sums of the float32 values, rounded to float32)
+//   k_pca_scale   the lower median of |c| by radix selection; scale = max(median / 3, 1e-10)
+//   k_pca_byte    c / scale rounded to signed 4 bits
+// The eigenproblems bounded this: a few hundred 32 x 32 matrices took a library's batched solver
+// 13.3 of the 14.7 ms of a 2560 x 4096 tensor (its tridiagonalisation runs column by column,
+// ~430 us a launch) and the median 60 us.  Measured here on that tensor (128 K blocks): V6 encode
+// 37 us (byte stores: 38), residuals 14, Gram 13.5, eigenvectors 157 (latency of ~9 sweeps of 31
+// dependent rounds on 128 work-groups; with a float64 division and square roots per rotation
+// 194), coefficients 8.6, medians 6.4, bytes 4.2; the rest of a call's 0.86 ms is the copy of 9.8
+// MB to pageable host memory.
+
+constexpr int kPcaSplits = 8;        // row ranges of the Gram sums
+constexpr float kInv63 = 1.0f / 63.0f;
+
+// One thread per (block, sub-block): 8 residuals, contiguous 32-byte stores.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_pca_err(const T* __restrict__ blocks,
+                                                      const uint8_t* __restrict__ levels,
+                                                      const T* __restrict__ dmin, const T* __restrict__ dmax,
+                                                      const uint8_t* __restrict__ config, int64_t n_rows,
+                                                      int64_t n_cb, float* __restrict__ err) {
+#pragma clang fp contract(off)
+    const int64_t gid = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    const int64_t bid = gid >> 2;
+    const int sb = (int)(gid & 3);
+    if (bid >= n_rows * n_cb) return;
+    const int64_t row = bid / n_cb;
+    const int64_t kb = bid - row * n_cb;
+    const float mn = (float)dmin[bid], mx = (float)dmax[bid];
+    float d = mx - mn;
+    d = d < 1e-10f ? 1e-10f : d;                     // (NaN stays, as torch.clamp leaves it)
+    const float q = d / 4.0f;
+    const int s = (config[bid] >> (2 * sb)) & 3;
+    float w = d - 2.0f * q;
+    w = w < 1e-10f ? 1e-10f : w;
+    const float lo = s == 2 ? mx - q : s == 3 ? mn + q : mn;
+    const float step = (s == 0 ? d : s == 3 ? w : q) * kInv63;
+    const T* x = blocks + bid * 32 + 8 * sb;
+    const uint2 lv = *reinterpret_cast<const uint2*>(levels + bid * 32 + 8 * sb);
+    float e[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float l = (float)(((i < 4 ? lv.x : lv.y) >> (8 * (i & 3))) & 0xFFu);
+        const float r = lo + step * l;
+        e[i] = (float)x[i] - r;
+    }
+    float4* o = reinterpret_cast<float4*>(err + (kb * n_rows + row) * 32 + 8 * sb);
+    o[0] = make_float4(e[0], e[1], e[2], e[3]);
+    o[1] = make_float4(e[4], e[5], e[6], e[7]);
+}
+
+typedef double sx8_double4 __attribute__((ext_vector_type(4)));
+
+// Work-group (split, kb): its rows' Gram matrix as three 16 x 16 tiles (00, 01, 11) of
+// v_mfma_f64_16x16x4: lane l supplies e[row l / 16][l % 16] of four rows, so both operands
+// of a tile are the same loads (products of float32 values are exact in float64).
+__global__ __launch_bounds__(256) void k_pca_gram(const float* __restrict__ err, int n_rows, int rows_per,
+                                                  double* __restrict__ part) {
+    const int kb = blockIdx.x, split = blockIdx.y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r0 = split * rows_per, r1 = min(r0 + rows_per, n_rows);
+    const float* e = err + (int64_t)kb * n_rows * 32;
+    sx8_double4 acc[3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) acc[t] = sx8_double4{0.0, 0.0, 0.0, 0.0};
+    for (int r = r0 + wave * 4; r < r1; r += 16 * 4) {
+        float x[4], y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int row = r + 16 * u + (lane >> 4);
+            const float* p = e + (int64_t)min(row, n_rows - 1) * 32 + (lane & 15);
+            x[u] = p[0];
+            y[u] = p[16];
+            if (row >= r1) x[u] = y[u] = 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const double a = x[u], b = y[u];
+            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, a, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, b, acc[2], 0, 0, 0);
+        }
+    }
+    __shared__ sx8_double4 red[4][3][64];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) red[wave][t][lane] = acc[t];
+    __syncthreads();
+    if (threadIdx.x < 192) {
+        const int t = threadIdx.x / 64, l = threadIdx.x & 63;
+        const sx8_double4 v = ((red[0][t][l] + red[1][t][l]) + red[2][t][l]) + red[3][t][l];
+        // element i of lane l: row l / 16 + 4 i, column l % 16
+        double* o = part + (((int64_t)split * gridDim.x + kb) * 3 + t) * 256 + (l & 15);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[((l >> 4) + 4 * i) * 16] = v[i];
+    }
+}
+
+// One work-group per K block: cyclic Jacobi on the 32 x 32 Gram matrix in LDS, float64.  A sweep
+// is 31 rounds of 16 disjoint rotations (round-robin pairing); in a round thread (p, q) owns the
+// 2 x 2 block (rows of pair p, columns of pair q), so the whole two-sided update is one step
+// without conflicts, two barriers a round.  The rotation's tangent only steers convergence, so
+// it is a float32 value (of a matrix scaled to a largest diagonal near 1); cosine and sine are
+// float64 and orthogonal to its precision, and the updated off-diagonal element is computed,
+// not set to zero.  Ends when the off-diagonal norm is below 1e-13 of the diagonal's (an
+// eigenvector error of 1e-10 at the gaps of 1e-3 that nearly white residuals have), after 20
+// sweeps at the latest.
+__global__ __launch_bounds__(256) void k_pca_eig(const double* __restrict__ part, int n_splits, int n_cb,
+                                                 float* __restrict__ data) {
+    constexpr int kLd = 33;
+    __shared__ double A[32 * kLd], V[32 * kLd], cs[16], sn[16], red[2][4];
+    const int kb = blockIdx.x, tid = threadIdx.x;
+    for (int i = tid; i < 768; i += 256) {
+        const int t = i >> 8, r = (i >> 4) & 15, c = i & 15;
+        double v = 0.0;
+        for (int s = 0; s < n_splits; ++s) v += part[(((int64_t)s * n_cb + kb) * 3 + t) * 256 + (i & 255)];
+        const int rr = r + (t == 2 ? 16 : 0), cc = c + (t >= 1 ? 16 : 0);
+        A[rr * kLd + cc] = v;
+        if (t == 1) A[cc * kLd + rr] = v;
+    }
+    for (int i = tid; i < 1024; i += 256) V[(i >> 5) * kLd + (i & 31)] = (i >> 5) == (i & 31) ? 1.0 : 0.0;
+    __syncthreads();
+    // scale by a power of two (the eigenvectors stay)
+    double top = 0.0;
+    for (int i = 0; i < 32; ++i) top = fmax(top, A[i * kLd + i]);
+    const int ex = top > 0.0 && top < 1e300 ? -ilogb(top) : 0;
+    __syncthreads();
+    for (int i = tid; i < 1024; i += 256) A[(i >> 5) * kLd + (i & 31)] = ldexp(A[(i >> 5) * kLd + (i & 31)], ex);
+    __syncthreads();
+    const int p = tid >> 4, q = tid & 15;
+    auto pair = [](int r, int k, int& a, int& b) {
+        a = k == 0 ? 31 : r + k >= 31 ? r + k - 31 : r + k;
+        b = k == 0 ? r : r - k < 0 ? r - k + 31 : r - k;
+    };
+    for (int sweep = 0; sweep < 20; ++sweep) {
+        double off = 0.0, dia = 0.0;
+        for (int i = tid; i < 1024; i += 256) {
+            const double v = A[(i >> 5) * kLd + (i & 31)];
+            if ((i >> 5) == (i & 31)) dia += v * v;
+            else off += v * v;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            off += __shfl_xor(off, o);
+            dia += __shfl_xor(dia, o);
+        }
+        if ((tid & 63) == 0) {
+            red[0][tid >> 6] = off;
+            red[1][tid >> 6] = dia;
+        }
+        __syncthreads();
+        off = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+        dia = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+        if (!(off > 1e-26 * dia)) break;             // the same for every thread; also ends on NaN
+        for (int r = 0; r < 31; ++r) {
+            if (tid < 16) {
+                int a, b;
+                pair(r, tid, a, b);
+                const float x = (float)A[a * kLd + b];
+                float t = 0.f;
+                if (x != 0.f) {
+                    const float tau = (float)(A[b * kLd + b] - A[a * kLd + a]) * __builtin_amdgcn_rcpf(x + x);
+                    const float at = fabsf(tau);
+                    t = at < 1e18f ? __builtin_amdgcn_rcpf(at + __builtin_amdgcn_sqrtf(1.f + at * at)) : 0.f;
+                    t = tau < 0.f ? -t : t;
+                }
+                const double y = __builtin_fma((double)t, (double)t, 1.0);      // 1 .. 2
+                double c = __builtin_amdgcn_rsq(y);
+                c = __builtin_fma(0.5 * c, __builtin_fma(-y * c, c, 1.0), c);   // Newton steps
+                c = __builtin_fma(0.5 * c, __builtin_fma(-y * c, c, 1.0), c);
+                cs[tid] = c;
+                sn[tid] = (double)t * c;
+            }
+            __syncthreads();
+            int ip, jp, iq, jq;
+            pair(r, p, ip, jp);
+            pair(r, q, iq, jq);
+            const double cp = cs[p], sp = sn[p], cq = cs[q], sq = sn[q];
+            const double a00 = A[ip * kLd + iq], a01 = A[ip * kLd + jq];
+            const double a10 = A[jp * kLd + iq], a11 = A[jp * kLd + jq];
+            const double b00 = cp * a00 - sp * a10, b01 = cp * a01 - sp * a11;
+            const double b10 = sp * a00 + cp * a10, b11 = sp * a01 + cp * a11;
+            A[ip * kLd + iq] = cq * b00 - sq * b01;
+            A[ip * kLd + jq] = sq * b00 + cq * b01;
+            A[jp * kLd + iq] = cq * b10 - sq * b11;
+            A[jp * kLd + jq] = sq * b10 + cq * b11;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                double* v = V + (p + 16 * h) * kLd;
+                const double v0 = v[iq], v1 = v[jq];
+                v[iq] = cq * v0 - sq * v1;
+                v[jq] = sq * v0 + cq * v1;
+            }
+            __syncthreads();
+        }
+    }
+    // the two largest eigenvalues; each vector's largest-magnitude component positive
+    if (tid < 2) {
+        int best = 0, second = 1;
+        if (A[kLd + 1] > A[0]) {
+            best = 1;
+            second = 0;
+        }
+        for (int i = 2; i < 32; ++i) {
+            const double v = A[i * kLd + i];
+            if (v > A[best * kLd + best]) {
+                second = best;
+                best = i;
+            } else if (v > A[second * kLd + second]) {
+                second = i;
+            }
+        }
+        const int col = tid == 0 ? best : second;
+        int arg = 0;
+        for (int i = 1; i < 32; ++i)
+            if (fabs(V[i * kLd + col]) > fabs(V[arg * kLd + col])) arg = i;
+        const double sg = V[arg * kLd + col] < 0.0 ? -1.0 : 1.0;
+        for (int i = 0; i < 32; ++i) data[(int64_t)kb * 64 + 32 * tid + i] = (float)(sg * V[i * kLd + col]);
+    }
+}
+
+// craw[kb][k][row] = basis_k . e, one thread per row of a K block.
+__global__ __launch_bounds__(kThreads) void k_pca_coeff(const float* __restrict__ err,
+                                                        const float* __restrict__ data, int n_rows,
+                                                        float* __restrict__ craw) {
+    const int kb = blockIdx.y;
+    const int row = (int)blockIdx.x * kThreads + (int)threadIdx.x;
+    if (row >= n_rows) return;
+    const float4* e = reinterpret_cast<const float4*>(err + ((int64_t)kb * n_rows + row) * 32);
+    const float* b = data + (int64_t)kb * 64;
+    double c0 = 0.0, c1 = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float4 v = e[i];
+        const float x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            c0 = __builtin_fma((double)b[4 * i + j], (double)x[j], c0);
+            c1 = __builtin_fma((double)b[32 + 4 * i + j], (double)x[j], c1);
+        }
+    }
+    craw[((int64_t)kb * 2) * n_rows + row] = (float)c0;
+    craw[((int64_t)kb * 2 + 1) * n_rows + row] = (float)c1;
+}
+
+// The lower median of |craw| over the rows of one (kb, k), by radix selection on the float bits
+// (non-negative floats order as integers): three passes of 11, 11 and 10 bits.  NaN sorts last
+// here and is then the answer, as in torch.median.
+__global__ __launch_bounds__(1024) void k_pca_scale(const float* __restrict__ craw, int n_rows,
+                                                    float* __restrict__ scales) {
+    __shared__ uint32_t hist[2048];
+    __shared__ uint32_t sel_prefix, sel_rank, any_nan;
+    __shared__ uint32_t wsum[16];
+    const int tid = threadIdx.x;
+    const float* c = craw + (int64_t)blockIdx.x * n_rows;
+    uint32_t prefix = 0, rank = (uint32_t)(n_rows - 1) / 2;
+    if (tid == 0) any_nan = 0;
+#pragma unroll
+    for (int pass = 0; pass < 3; ++pass) {
+        const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0;
+        const uint32_t mask = pass == 2 ? 0x3FFu : 0x7FFu;
+        for (int i = tid; i < 2048; i += 1024) hist[i] = 0;
+        __syncthreads();
+        for (int i = tid; i < n_rows; i += 1024) {
+            const uint32_t v = __builtin_bit_cast(uint32_t, c[i]) & 0x7FFFFFFFu;
+            if (pass == 0 && v > 0x7F800000u) any_nan = 1;
+            const bool in = pass == 0 || (v >> (pass == 1 ? 21 : 10)) == prefix;
+            if (in) atomicAdd(&hist[(v >> shift) & mask], 1u);
+        }
+        __syncthreads();
+        // bin of the rank: two bins per thread, sums over the waves, then the owner says
+        const uint32_t h0 = hist[2 * tid], h1 = hist[2 * tid + 1];
+        uint32_t incl = h0 + h1;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t t = __shfl_up(incl, o);
+            if ((tid & 63) >= o) incl += t;
+        }
+        if ((tid & 63) == 63) wsum[tid >> 6] = incl;
+        __syncthreads();
+        uint32_t base = 0;
+        for (int w = 0; w < (tid >> 6); ++w) base += wsum[w];
+        const uint32_t lo = base + incl - (h0 + h1);
+        if (rank >= lo && rank < lo + h0 + h1) {
+            const bool second = rank >= lo + h0;
+            sel_prefix = (prefix << (pass == 2 ? 10 : 11)) | (uint32_t)(2 * tid + (second ? 1 : 0));
+            sel_rank = rank - (second ? lo + h0 : lo);
+        }
+        __syncthreads();
+        prefix = sel_prefix;
+        rank = sel_rank;
+        __syncthreads();
+    }
+    if (tid == 0) {
+        const float med = any_nan ? __builtin_nanf("") : __builtin_bit_cast(float, prefix);
+        const float s = med * (1.0f / 3.0f);          // (torch's form of a division by a number)
+        scales[blockIdx.x] = s < 1e-10f ? 1e-10f : s;
+    }
+}
+
+// Coefficient bytes, four K blocks of a row per thread, rows along the lanes.
+__global__ __launch_bounds__(kThreads) void k_pca_byte(const float* __restrict__ craw,
+                                                       const float* __restrict__ scales, int n_rows, int n_cb,
+                                                       uint8_t* __restrict__ coeff) {
+    const int row = (int)blockIdx.x * kThreads + (int)threadIdx.x;
+    if (row >= n_rows) return;
+    const int kb0 = blockIdx.y * 4;
+    uint32_t w = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int kb = min(kb0 + j, n_cb - 1);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            float v = __builtin_rintf(craw[((int64_t)kb * 2 + k) * n_rows + row] / scales[kb * 2 + k]);
+            v = v < -8.f ? -8.f : (v > 7.f ? 7.f : v);
+            w |= ((uint32_t)(int)v & 0xFu) << (8 * j + 4 * k);
+        }
+    }
+    uint8_t* o = coeff + (int64_t)row * n_cb + kb0;
+    if (kb0 + 4 <= n_cb && (reinterpret_cast<uintptr_t>(o) & 3) == 0) {
+        *reinterpret_cast<uint32_t*>(o) = w;
+    } else {
+        for (int j = 0; j < 4 && kb0 + j < n_cb; ++j) o[j] = (uint8_t)(w >> (8 * j));
+    }
+}
+
+struct PcaLayout {
+    int64_t err, part, craw, total;
+};
+PcaLayout pca_layout(int64_t n_rows, int64_t n_cb) {
+    PcaLayout l;
+    l.err = 0;
+    l.part = l.err + n_rows * n_cb * 128;
+    l.craw = l.part + (int64_t)kPcaSplits * n_cb * 768 * 8;
+    l.total = l.craw + n_rows * n_cb * 8;
+    return l;
 }
 
 }  // namespace
@@ -133,7 +491,62 @@ extern "C" int32_t sx8_v6_encode(const uint16_t* W, int64_t out_f, int64_t in_f,
     const int64_t n_cb = (in_f + 31) / 32;
     const int64_t grid = (out_f * n_cb + kThreads - 1) / kThreads;
     if (grid > 0x7FFFFFFF) return fail(SX8_ERR_UNSUPPORTED, "sx8_v6_encode: tensor too large");
+    const bool vec_out = aligned(levels_hi, 16) && aligned(levels_lo, 8) && aligned(levels, 16);
     hipLaunchKernelGGL(k_v6_encode, dim3((unsigned)grid), dim3(kThreads), 0, as_stream(stream), W,
-                       out_f, in_f, ld, n_cb, levels, dmin, dmax, config, levels_hi, levels_lo);
+                       out_f, in_f, ld, n_cb, levels, dmin, dmax, config, levels_hi, levels_lo, vec_out);
     return check_launch("sx8_v6_encode");
+}
+
+extern "C" int64_t sx8_quant_pca_workspace_bytes(int64_t n_rows, int64_t n_cb) {
+    if (n_rows <= 0 || n_cb <= 0 || n_rows > ((int64_t)1 << 36) / n_cb) return -1;
+    return pca_layout(n_rows, n_cb).total;
+}
+
+extern "C" int32_t sx8_quant_pca(const void* blocks, const void* dmin, const void* dmax, int32_t is_f16,
+                                 const uint8_t* levels, const uint8_t* config, int64_t n_rows, int64_t n_cb,
+                                 uint8_t* coeff, float* data, float* scales, void* workspace,
+                                 int64_t workspace_bytes, void* stream) {
+    using namespace sx8;
+    const char* what = "sx8_quant_pca";
+    if (!blocks || !dmin || !dmax || !levels || !config || !coeff || !data || !scales || !workspace)
+        return fail(SX8_ERR_INVALID, "%s: null pointer argument", what);
+    const int64_t need = sx8_quant_pca_workspace_bytes(n_rows, n_cb);
+    if (need < 0) return fail(SX8_ERR_INVALID, "%s: bad shape n_rows=%lld n_cb=%lld", what, (long long)n_rows,
+                              (long long)n_cb);
+    const int esz = is_f16 ? 2 : 4;
+    if (!aligned(blocks, esz) || !aligned(dmin, esz) || !aligned(dmax, esz) || !aligned(levels, 8) ||
+        !aligned(data, 4) || !aligned(scales, 4) || !aligned(workspace, 16))
+        return fail(SX8_ERR_INVALID, "%s: misaligned pointer", what);
+    if (workspace_bytes < need)
+        return fail(SX8_ERR_INVALID, "%s: workspace needs %lld bytes, got %lld", what, (long long)need,
+                    (long long)workspace_bytes);
+    const int64_t err_grid = (n_rows * n_cb * 4 + kThreads - 1) / kThreads;
+    const int64_t row_grid = (n_rows + kThreads - 1) / kThreads;
+    // grid limits: 65535 work-groups in y; 32-bit row numbers
+    if (err_grid > 0x7FFFFFFF || n_rows > 0x3FFFFFFF || n_cb > 65535 || 2 * n_cb > 0x7FFFFFFF)
+        return fail(SX8_ERR_UNSUPPORTED, "%s: tensor too large", what);
+    const PcaLayout l = pca_layout(n_rows, n_cb);
+    uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
+    float* err = reinterpret_cast<float*>(ws + l.err);
+    double* part = reinterpret_cast<double*>(ws + l.part);
+    float* craw = reinterpret_cast<float*>(ws + l.craw);
+    const hipStream_t st = as_stream(stream);
+    if (is_f16)
+        hipLaunchKernelGGL(k_pca_err<_Float16>, dim3((unsigned)err_grid), dim3(kThreads), 0, st,
+                           reinterpret_cast<const _Float16*>(blocks), levels, reinterpret_cast<const _Float16*>(dmin),
+                           reinterpret_cast<const _Float16*>(dmax), config, n_rows, n_cb, err);
+    else
+        hipLaunchKernelGGL(k_pca_err<float>, dim3((unsigned)err_grid), dim3(kThreads), 0, st,
+                           reinterpret_cast<const float*>(blocks), levels, reinterpret_cast<const float*>(dmin),
+                           reinterpret_cast<const float*>(dmax), config, n_rows, n_cb, err);
+    const int rows_per = (int)((n_rows + kPcaSplits - 1) / kPcaSplits);
+    hipLaunchKernelGGL(k_pca_gram, dim3((unsigned)n_cb, kPcaSplits), dim3(256), 0, st, err, (int)n_rows, rows_per,
+                       part);
+    hipLaunchKernelGGL(k_pca_eig, dim3((unsigned)n_cb), dim3(256), 0, st, part, kPcaSplits, (int)n_cb, data);
+    hipLaunchKernelGGL(k_pca_coeff, dim3((unsigned)row_grid, (unsigned)n_cb), dim3(kThreads), 0, st, err, data,
+                       (int)n_rows, craw);
+    hipLaunchKernelGGL(k_pca_scale, dim3((unsigned)(2 * n_cb)), dim3(1024), 0, st, craw, (int)n_rows, scales);
+    hipLaunchKernelGGL(k_pca_byte, dim3((unsigned)row_grid, (unsigned)((n_cb + 3) / 4)), dim3(kThreads), 0, st, craw,
+                       scales, (int)n_rows, (int)n_cb, coeff);
+    return check_launch(what);
 }

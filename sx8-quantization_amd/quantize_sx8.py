@@ -9,7 +9,8 @@ reference, which runs at module import time and cannot be imported:
     median(|c|)/3; the first two are kept (1 coeff byte, 2 bases, 2 scales).
   * ``pack_levels_6bit`` -- :148-167.
   * on a GPU the V6 encode and the packing run as one HIP kernel (``v6_encode_hip``,
-    sx8_v6_encode), bit-identical to ``v6_encode_6bit``; the PCA stays in torch.
+    sx8_v6_encode), bit-identical to ``v6_encode_6bit``, and the gram PCA as five more
+    (sx8_quant_pca); the outputs come to the host in one copy.
   * ``quantize_tensor``  -- the tensor loop of :235-282 and the dict layout of
     :383-395.
 
@@ -70,6 +71,12 @@ def pca_correct(levels, dmin, dmax, config, blocks, n_cb, pca_method="svd"):
     dev = blocks.device
     n_blk = blocks.shape[0]
     n_rows = n_blk // n_cb
+    if pca_method == "gram" and blocks.is_cuda and n_rows >= 4:
+        out = _HostFields(n_blk, n_cb, dev)
+        _pca_hip(levels, dmin.float(), dmax.float(), config, blocks.float(), n_rows, n_cb, out)
+        f = out.to_host()
+        if f is not None:
+            return f["coeff"].reshape(n_blk, 1), f["data"], f["scales"]
     d = (dmax - dmin).clamp(min=1e-10)
     Q = d / 4.0
     lo_j = torch.stack([dmin, dmin, dmax - Q, dmin + Q], dim=0)
@@ -122,6 +129,47 @@ def pca_correct(levels, dmin, dmax, config, blocks, n_cb, pca_method="svd"):
     return coeff.cpu().numpy().reshape(n_blk, 1), data, scales
 
 
+class _HostFields:
+    """The quantizer's outputs in one device buffer, so that they reach the host in one copy
+    (numpy views of one array): data, scales, dmin, dmax, levels_hi, levels_lo, config, coeff."""
+
+    def __init__(self, n_blk, n_cb, device):
+        sizes = [("data", n_cb * 256, np.float32), ("scales", n_cb * 8, np.float32), ("dmin", n_blk * 2, np.float16),
+                 ("dmax", n_blk * 2, np.float16), ("levels_hi", n_blk * 16, np.uint8),
+                 ("levels_lo", n_blk * 8, np.uint8), ("config", n_blk, np.uint8), ("coeff", n_blk, np.uint8)]
+        self.at, off = {}, 0
+        for name, nb, dt in sizes:
+            self.at[name] = (off, nb, dt)
+            off = (off + nb + 15) // 16 * 16
+        self.n_cb = n_cb
+        self.buf = torch.empty(off, dtype=torch.uint8, device=device)
+
+    def ptr(self, name):
+        return self.buf.data_ptr() + self.at[name][0]
+
+    def to_host(self):
+        """{name: numpy array}, or None when the bases or scales are not finite (weights with
+        infinities or NaN: the caller takes the general path)."""
+        host = self.buf.cpu().numpy()
+        f = {name: host[off:off + nb].view(dt) for name, (off, nb, dt) in self.at.items()}
+        f["data"], f["scales"] = f["data"].reshape(self.n_cb, 64), f["scales"].reshape(self.n_cb, 2)
+        return f if np.isfinite(f["data"]).all() and np.isfinite(f["scales"]).all() else None
+
+
+def _pca_hip(levels, dmin, dmax, config, blocks, n_rows, n_cb, out):
+    """sx8_quant_pca of (n_rows * n_cb, 32) blocks -- all of float32 or all of float16 -- into the
+    fields coeff, data and scales of `out`."""
+    import _sx8lib as _L
+    f16 = blocks.dtype == torch.float16
+    t = [x.contiguous() for x in (blocks, dmin, dmax, levels, config.to(torch.uint8))]
+    nb = int(_L.lib().sx8_quant_pca_workspace_bytes(n_rows, n_cb))
+    if nb < 0:
+        raise RuntimeError(f"sx8_quant_pca_workspace_bytes: bad shape {n_rows} x {n_cb}")
+    ws = torch.empty(nb, dtype=torch.uint8, device=blocks.device)
+    _L.call("sx8_quant_pca", _L.ptr(t[0]), _L.ptr(t[1]), _L.ptr(t[2]), int(f16), _L.ptr(t[3]), _L.ptr(t[4]), n_rows,
+            n_cb, out.ptr("coeff"), out.ptr("data"), out.ptr("scales"), _L.ptr(ws), nb, _L.stream(blocks.device))
+
+
 def pack_levels_6bit(levels: np.ndarray):
     """(n_blk, 32) u8 levels -> (levels_hi (n_blk*16,), levels_lo (n_blk*8,))."""
     lv = np.asarray(levels, dtype=np.uint8)
@@ -142,12 +190,15 @@ def quantize_tensor(W, device=None, pca_method=None, degenerate_frac=0.0, seed=N
     step = 1e-10 floor (dmin == dmax) exactly as the measurement plan asks.
     Returns (qt, bases_info) with numpy arrays, in the reference's pkl layout.
     """
-    W = torch.as_tensor(W)
+    W = torch.as_tensor(W).detach()
     if device is None:
         device = W.device
     if pca_method is None:
         pca_method = "gram" if torch.device(device).type == "cuda" else "svd"
-    Wd = W.to(device=device, dtype=torch.float16).float()
+    hip = torch.device(device).type == "cuda"
+    Wd = W.to(device=device, dtype=torch.float16)
+    if not hip:
+        Wd = Wd.float()
     out_f, in_f = Wd.shape
     n_cb = (in_f + B - 1) // B
     pad = n_cb * B - in_f
@@ -155,12 +206,25 @@ def quantize_tensor(W, device=None, pca_method=None, degenerate_frac=0.0, seed=N
         Wd = torch.nn.functional.pad(Wd, (0, pad))
     blocks = Wd.reshape(out_f * n_cb, B).contiguous()
     if degenerate_frac > 0:
+        if blocks.data_ptr() == W.data_ptr():
+            blocks = blocks.clone()                  # never the caller's weights
         g = torch.Generator(device="cpu")
         g.manual_seed(int(seed or 0))
         n_deg = int(round(degenerate_frac * blocks.shape[0]))
         idx = torch.randperm(blocks.shape[0], generator=g)[:n_deg].to(device)
         blocks[idx] = blocks[idx, :1].expand(-1, B)
+    meta = {"shape": (out_f, in_f), "orig_shape": (out_f, in_f), "n_blocks": out_f * n_cb, "n_cb": n_cb}
+    if hip and pca_method == "gram" and out_f >= 4:
+        out = _HostFields(out_f * n_cb, n_cb, blocks.device)
+        lv, dmin16, dmax16, cfg8 = _v6_encode_into(blocks, out)
+        _pca_hip(lv, dmin16, dmax16, cfg8, blocks, out_f, n_cb, out)
+        f = out.to_host()
+        if f is not None:
+            qt = dict(meta, dmin=f["dmin"], dmax=f["dmax"], config=f["config"], levels_hi=f["levels_hi"],
+                      levels_lo=f["levels_lo"], coeff=f["coeff"].reshape(-1, 1))
+            return qt, {"n_cb": n_cb, "data": f["data"], "scales": f["scales"]}
     if blocks.is_cuda:
+        blocks = blocks.float()
         lv, dmin16, dmax16, cfg, hi_t, lo_t = v6_encode_hip(blocks)
         dmin, dmax = dmin16.float(), dmax16.float()
         hi, lo = hi_t.cpu().numpy(), lo_t.cpu().numpy()
@@ -171,13 +235,8 @@ def quantize_tensor(W, device=None, pca_method=None, degenerate_frac=0.0, seed=N
         dmin_np = dmin.cpu().numpy().astype(np.float16)
         dmax_np = dmax.cpu().numpy().astype(np.float16)
     coeff, data, scales = pca_correct(lv, dmin, dmax, cfg, blocks, n_cb, pca_method)
-    qt = {
-        "shape": (out_f, in_f), "orig_shape": (out_f, in_f),
-        "n_blocks": out_f * n_cb, "n_cb": n_cb,
-        "dmin": dmin_np, "dmax": dmax_np,
-        "config": cfg.cpu().numpy().astype(np.uint8),
-        "levels_hi": hi, "levels_lo": lo, "coeff": coeff,
-    }
+    qt = dict(meta, dmin=dmin_np, dmax=dmax_np, config=cfg.cpu().numpy().astype(np.uint8), levels_hi=hi,
+              levels_lo=lo, coeff=coeff)
     return qt, {"n_cb": n_cb, "data": data, "scales": scales}
 
 
@@ -199,3 +258,15 @@ def v6_encode_hip(blocks: torch.Tensor):
     _L.call("sx8_v6_encode", _L.ptr(b16), n, 32, 32, _L.ptr(lv), _L.ptr(dmin), _L.ptr(dmax), _L.ptr(cfg),
             _L.ptr(hi), _L.ptr(lo), _L.stream(dev))
     return lv, dmin, dmax, cfg.int(), hi, lo
+
+
+def _v6_encode_into(b16: torch.Tensor, out: _HostFields):
+    """v6_encode_hip of (n, 32) fp16 blocks with its host fields written into `out`: levels (n,
+    32) u8 and views of dmin, dmax and config."""
+    import _sx8lib as _L
+    n = b16.shape[0]
+    lv = torch.empty(n, 32, dtype=torch.uint8, device=b16.device)
+    _L.call("sx8_v6_encode", _L.ptr(b16), n, 32, 32, _L.ptr(lv), out.ptr("dmin"), out.ptr("dmax"), out.ptr("config"),
+            out.ptr("levels_hi"), out.ptr("levels_lo"), _L.stream(b16.device))
+    view = lambda name, dt: out.buf[out.at[name][0]:out.at[name][0] + out.at[name][1]].view(dt)  # noqa: E731
+    return lv, view("dmin", torch.float16), view("dmax", torch.float16), view("config", torch.uint8)

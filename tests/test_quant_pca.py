@@ -1,0 +1,100 @@
+"""sx8_quant_pca (residuals, Gram matrices, Jacobi eigenvectors, coefficients, medians) against
+numpy on the same blocks: the residuals restated in float32 with the kernel's roundings, the
+Gram matrix and its eigenvectors in float64, the coefficients from the float32 bases.  Row
+counts at the edges of the Gram ranges and of the 256-row passes, K blocks at those of the
+byte pass (four per thread)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+
+def _reference(x, lv, mn, mx, cfg, n_rows, n_cb):
+    f = np.float32
+    r63 = f(1) / f(63)
+    d = np.maximum(mx - mn, f(1e-10))
+    q = d / f(4)
+    w = np.maximum(d - f(2) * q, f(1e-10))
+    lo = np.stack([mn, mn, mx - q, mn + q], 1)
+    st = np.stack([d * r63, q * r63, q * r63, w * r63], 1)
+    s = np.stack([(cfg >> (2 * i)) & 3 for i in range(4)], 1)
+    lo, st = np.take_along_axis(lo, s, 1), np.take_along_axis(st, s, 1)
+    rec = lo[:, :, None] + st[:, :, None] * lv.reshape(-1, 4, 8).astype(f)
+    e = (x - rec.reshape(-1, 32)).reshape(n_rows, n_cb, 32).astype(np.float64)
+    G = np.einsum("rci,rcj->cij", e, e)
+    lam, vec = np.linalg.eigh(G)
+    return e, G, lam, vec
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_rows,n_cb,f16", [
+    (4, 1, True), (5, 3, False), (32, 4, True), (63, 5, True), (64, 2, False), (65, 7, True), (255, 1, True),
+    (256, 8, False), (257, 6, True), (1000, 9, True), (4099, 3, True),
+])
+def test_pca_against_numpy(hiplib, cuda, n_rows, n_cb, f16):
+    import torch
+    from quantize_sx8 import pca_correct, quantize_tensor, v6_encode_hip
+    print("pca", n_rows, n_cb, f16, flush=True)
+    g = torch.Generator().manual_seed(n_rows * 10 + n_cb)
+    W = (torch.randn(n_rows, n_cb * 32, generator=g) * 0.02).half()
+    W[1, :32] = W[1, 0]                                # a constant block
+    blocks = W.reshape(-1, 32).to(cuda)
+    lv, dmin, dmax, cfg, _, _ = v6_encode_hip(blocks)
+    if f16:
+        qt, bi = quantize_tensor(W, device=cuda)       # the fp16 form
+        coeff, data, scales = qt["coeff"], bi["data"], bi["scales"]
+        assert np.array_equal(qt["config"], cfg.cpu().numpy().astype(np.uint8))
+    else:
+        coeff, data, scales = pca_correct(lv, dmin.float(), dmax.float(), cfg, blocks.float(), n_cb, "gram")
+    assert coeff.shape == (n_rows * n_cb, 1) and data.shape == (n_cb, 64) and scales.shape == (n_cb, 2)
+    h = lambda t: t.cpu().numpy()
+    e, G, lam, vec = _reference(h(blocks).astype(np.float32), h(lv), h(dmin).astype(np.float32),
+                                h(dmax).astype(np.float32), h(cfg), n_rows, n_cb)
+    for kb in range(n_cb):
+        for k in range(2):
+            v = data[kb, 32 * k:32 * k + 32].astype(np.float64)
+            assert v[np.abs(v).argmax()] > 0
+            # float64 Jacobi, stored in float32: an eigenvector to a float32 rounding, of the
+            # right eigenvalue, and numpy's vector up to sign where the gap resolves it
+            assert abs(v @ v - 1) <= 1e-6
+            assert np.abs(G[kb] @ v - lam[kb, -1 - k] * v).max() <= 1e-6 * lam[kb, -1]
+            others = np.delete(lam[kb], 31 - k)
+            gap = np.abs(others - lam[kb, -1 - k]).min() / lam[kb, -1]
+            if gap > 1e-6:
+                u = vec[kb][:, -1 - k]
+                assert min(np.abs(v - u).max(), np.abs(v + u).max()) <= 1e-6 + 1e-12 / gap
+            c = (e[:, kb] @ v).astype(np.float32)
+            sc = max(np.sort(np.abs(c))[(n_rows - 1) // 2] / np.float32(3), np.float32(1e-10))
+            assert abs(scales[kb, k] - sc) <= 1e-6 * sc
+            ratio = c / scales[kb, k]
+            want = np.clip(np.rint(ratio), -8, 7).astype(int)
+            byte = coeff.reshape(n_rows, n_cb)[:, kb]
+            got = ((byte >> (4 * k)) & 15).astype(int)
+            got = np.where(got > 7, got - 16, got)
+            tie = np.abs(np.abs(ratio - np.floor(ratio)) - 0.5) < 1e-4   # c differs in its last bit
+            assert (got == want)[~tie].all()
+
+
+@pytest.mark.gpu
+def test_pca_not_finite_takes_general_path(hiplib, cuda):
+    """Weights with an infinity keep the torch path's outcome (whatever it is), not zeros."""
+    import torch
+    from quantize_sx8 import _HostFields, _pca_hip, v6_encode_hip
+    W = (torch.randn(64, 64, generator=torch.Generator().manual_seed(1)) * 0.02).half().to(cuda)
+    W[3, 40] = float("inf")
+    blocks = W.reshape(-1, 32)
+    lv, dmin, dmax, cfg, _, _ = v6_encode_hip(blocks)
+    out = _HostFields(128, 2, W.device)
+    _pca_hip(lv, dmin, dmax, cfg, blocks, 64, 2, out)
+    assert out.to_host() is None
+
+
+def test_pca_refusals(hiplib):
+    L, p, N0 = hiplib, ctypes.c_void_p(4096), ctypes.c_void_p(None)
+    assert L.sx8_quant_pca_workspace_bytes(0, 4) == -1 and L.sx8_quant_pca_workspace_bytes(1 << 37, 4) == -1
+    need = L.sx8_quant_pca_workspace_bytes(64, 4)
+    call = lambda **k: L.sx8_quant_pca(k.get("x", p), p, p, 1, p, p, k.get("r", 64), 4, p, p, p, k.get("ws", p),
+                                       k.get("nb", need), N0)
+    assert call(x=N0) == 1 and call(ws=N0) == 1 and call(nb=need - 1) == 1 and call(r=0) == 1
+    assert call(x=ctypes.c_void_p(4097)) == 1 and call(ws=ctypes.c_void_p(4104)) == 1
+    assert b"misaligned" in L.sx8_last_error()
