@@ -1,21 +1,31 @@
 // sx8_dequant.hip -- canonical (R64, bit-exact) dequantization kernels:
-//   * k_dequant_split: whole tensor from the pkl/container split arrays (n-major);
+//   * k_dequant_wave, k_dequant_split: whole tensor from the pkl/container split arrays (n-major);
 //     role of kernel_sx8_v43.decode_tensor_gpu_fast (scripts/kernel_sx8_v43.py:109-145).
-//   * k_gather_v44: selected rows from the kb-major v4.4 layout; role of the embedding
+//   * k_dequant_wave, k_gather_v44: selected rows from the kb-major v4.4 layout; role of the embedding
 //     gather sx8_embed_v44 (cuda/sx8_embed_v44.cu:21-94) and, with identity ids, of a
 //     whole-tensor dequant from the v4.4 layout.
 //
-// Both give one thread per (row, block, sub-block): 8 weights, one 16-byte store.
-// Threads are ordered sub-block fastest, then block along K, then row, so a wave
-// writes 64 x 16 contiguous bytes of one output row.  The inputs are read with
-// dword/short loads; these kernels move 30 B in and 64 B out per block, so the fp16
-// write stream sets their speed.
+// What bounds them: 30 B in and 64 B out per block, with the binary64 arithmetic (three fused
+// multiply-adds and a conversion a weight) close behind.  A wave takes 16 K blocks of four rows
+// at a time: lane (c, t) loads the whole record of (row t, block c), one load per field for 64
+// records, and the records cross the wave's four 16-lane rows (v_permlane32_swap,
+// v_permlane16_swap) so that lane (c, g) decodes sub-block g of block c for each of the four
+// rows: its 8 + 8 basis values and scales stay in registers as binary64 for all the wave's
+// rows, and every store instruction writes 1 KB of one output row.  One thread per (block,
+// sub-block) issues four times the load instructions, re-reads and converts the basis for
+// every 16 bytes of output: 9728 x 2560 20.9 us, here 17.8 (a 73 MB copy takes 14.2; with the
+// decode replaced by plain moves the kernel takes 14.4).  It stays for tensors too small to fill the
+// GPU with waves of four rows.
+#include <algorithm>
+#include <type_traits>
+
 #include "sx8_device.h"
 #include "sx8_host.h"
 
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / 64;
 
 // Store 8 fp16 values for columns [col, col+8) of an output row.  Vector store when
 // the row pitch allows it, element stores (and the in_f cut) otherwise.
@@ -44,6 +54,144 @@ __device__ __forceinline__ void load_basis(const float* __restrict__ basis,
     const float2 sc = *reinterpret_cast<const float2*>(scales + kb * 2);
     s0 = sc.x;
     s1 = sc.y;
+}
+
+// A whole record: dmin | dmax << 16, config | coeff << 8, hi nibbles, lo quads.
+struct Rec {
+    uint32_t lohi, cc;
+    uint32_t h[4];
+    uint32_t qx, qy;
+};
+
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+// Fields of (row, kb) from the n-major split arrays (block row n_cb + kb).
+struct SplitSrc {
+    const uint16_t* dmin;
+    const uint16_t* dmax;
+    const uint8_t* config;
+    const uint8_t* coeff;
+    const uint8_t* hi;
+    const uint8_t* lo;
+    int64_t n_cb;
+    __device__ __forceinline__ void load(Rec& o, int64_t row, int kb) const {
+        const int64_t bid = row * n_cb + kb;
+        o.lohi = (uint32_t)dmin[bid] | ((uint32_t)dmax[bid] << 16);
+        o.cc = (uint32_t)config[bid] | ((uint32_t)coeff[bid] << 8);
+        const u32x4_a4 h = *reinterpret_cast<const u32x4_a4*>(hi + bid * 16);
+        const u32x2_a2 q = *reinterpret_cast<const u32x2_a2*>(lo + bid * 8);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o.h[i] = h[i];
+        o.qx = q[0];
+        o.qy = q[1];
+    }
+};
+
+// The same from the kb-major v4.4 layout (block kb N + row).
+template <int HB>
+struct V44Src {
+    const uint8_t* hdr;
+    const uint8_t* levels;
+    int64_t N;
+    __device__ __forceinline__ void load(Rec& o, int64_t row, int kb) const {
+        const int64_t bid = kb * N + row;
+        uint32_t d0, d1, cfg, cf;
+        sx8_load_hdr<HB>(hdr, bid, d0, d1, cfg, cf);
+        o.lohi = d0 | (d1 << 16);
+        o.cc = cfg | (cf << 8);
+        const u32x4_a4 h = *reinterpret_cast<const u32x4_a4*>(levels + bid * 24);
+        const uint2 q = *reinterpret_cast<const uint2*>(levels + bid * 24 + 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o.h[i] = h[i];
+        o.qx = q.x;
+        o.qy = q.y;
+    }
+};
+
+// v in the lanes of 16-lane row i -> o[i] in every row (all four rows' values of a lane column)
+__device__ __forceinline__ void gather_rows(uint32_t v, uint32_t (&o)[4]) {
+    uint32_t a = v, b = v;
+    sx8_swap32(a, b);            // a: rows 0, 1, 0, 1; b: rows 2, 3, 2, 3
+    o[0] = o[1] = a;
+    sx8_swap16(o[0], o[1]);
+    o[2] = o[3] = b;
+    sx8_swap16(o[2], o[3]);
+}
+
+// Output rows 4 quad + t (quad = this wave's) of T: row ids[.] of the weight, or row row0 + .
+// without ids; rows outside [0, N) are skipped.  blockIdx.x: 16-block column group.
+template <typename Src, bool kIds, bool kVec>
+__global__ __launch_bounds__(kThreads) void k_dequant_wave(const Src src, const int64_t* __restrict__ ids,
+                                                           const float* __restrict__ basis,
+                                                           const float* __restrict__ scales, int64_t T, int64_t N,
+                                                           int n_cb, int64_t in_f, uint16_t* __restrict__ out, int64_t row0) {
+    const int lane = threadIdx.x & 63;
+    const int c = lane & 15, g = lane >> 4;
+    const int kb = (int)blockIdx.x * 16 + c;
+    const int kbc = min(kb, n_cb - 1);
+    const int64_t quad = (int64_t)blockIdx.y * kWaves + (threadIdx.x >> 6);
+    if (quad * 4 >= T) return;
+    // this lane's record: row g of the quad (-1: none)
+    const int64_t t = quad * 4 + g;
+    int64_t row = t < T ? (kIds ? ids[t] : row0 + t) : -1;
+    if (row >= N) row = -1;
+    Rec r;
+    src.load(r, row < 0 ? 0 : row, kbc);
+    double b0[8], b1[8], s0, s1;
+    load_basis(basis, scales, kbc, g, b0, b1, s0, s1);
+    const unsigned long long ok = __ballot(row >= 0);       // lane 16 i holds row i's
+    uint32_t lohi[4], cc[4], p[4];
+    gather_rows(r.lohi, lohi);
+    gather_rows(r.cc, cc);
+    sx8_transpose4(r.h);
+    uint32_t a = r.qx, b = r.qy;
+    sx8_swap32(a, b);
+    p[0] = p[1] = a;
+    sx8_swap16(p[0], p[1]);
+    p[2] = p[3] = b;
+    sx8_swap16(p[2], p[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (!((ok >> (16 * i)) & 1)) continue;          // uniform
+        uint32_t w[4];
+        sx8_r64_subblock(sx8_h2f(lohi[i]), sx8_h2f(lohi[i] >> 16), cc[i] & 0xFFu, cc[i] >> 8, g, r.h[i],
+                         (g & 1) ? p[i] >> 16 : p[i] & 0xFFFFu, b0, b1, s0, s1, w);
+        uint16_t* o = out + (quad * 4 + i) * in_f;
+        const int64_t col = (int64_t)kb * 32 + 8 * g;
+        if constexpr (kVec) {
+            if (col < in_f) *reinterpret_cast<uint4*>(o + col) = make_uint4(w[0], w[1], w[2], w[3]);
+        } else {
+            if (kb < n_cb) store8(o, col, in_f, false, w);
+        }
+    }
+}
+
+// The wave kernel where it has at least four waves per SIMD to run, false otherwise: a wave's four
+// rows are a chain that few waves do not hide (1024 x 2560: 1280 waves 5.5 us against 4.3; 4096 rows of
+// 2560 gathered, 5120 waves: 19.8 against 21.0), and where at most a fifth of its lanes idle in the last
+// 16-block group (5000 x 333, 11 blocks: 7.7 against 5.4 us).
+template <typename Src>
+bool launch_wave(const Src& src, const int64_t* ids, const float* basis, const float* scales, int64_t T, int64_t N,
+                 int64_t n_cb, int64_t in_f, bool vec_ok, uint16_t* out, hipStream_t st) {
+    const int64_t quads = (T + 3) / 4, cols = (n_cb + 15) / 16;
+    if (quads * cols < 4096 || n_cb * 5 < cols * 16 * 4 || cols > 0x7FFFFFFF / 16) return false;
+    // blockIdx.y takes at most 65535 work-groups: more rows go in several launches
+    constexpr int64_t kRows = (int64_t)65535 * kWaves * 4;
+    for (int64_t t0 = 0; t0 < T; t0 += kRows) {
+        const int64_t Tc = std::min(kRows, T - t0);
+        const dim3 grid((unsigned)cols, (unsigned)((Tc + kWaves * 4 - 1) / (kWaves * 4)));
+        auto go = [&](auto with_ids, auto vec) {
+            hipLaunchKernelGGL((k_dequant_wave<Src, decltype(with_ids)::value, decltype(vec)::value>), grid,
+                               dim3(kThreads), 0, st, src, ids ? ids + t0 : nullptr, basis, scales, Tc, N, (int)n_cb,
+                               in_f, out + t0 * in_f, t0);
+        };
+        if (ids && vec_ok) go(std::true_type{}, std::true_type{});
+        else if (ids) go(std::true_type{}, std::false_type{});
+        else if (vec_ok) go(std::false_type{}, std::true_type{});
+        else go(std::false_type{}, std::false_type{});
+    }
+    return true;
 }
 
 __global__ __launch_bounds__(kThreads) void k_dequant_split(
@@ -116,6 +264,9 @@ extern "C" int32_t sx8_dequant_f16(const uint16_t* dmin, const uint16_t* dmax,
         return fail(SX8_ERR_INVALID, "sx8_dequant_f16: misaligned pointer");
     const int64_t n_blocks = out_f * n_cb;
     const bool vec_ok = aligned(out, 16) && (in_f % 8 == 0);
+    if (launch_wave(SplitSrc{dmin, dmax, config, coeff, levels_hi, levels_lo, n_cb}, nullptr, basis, scales, out_f,
+                    out_f, n_cb, in_f, vec_ok, out, as_stream(stream)))
+        return check_launch("sx8_dequant_f16");
     const int64_t threads = n_blocks * 4;
     const int64_t grid = (threads + kThreads - 1) / kThreads;
     if (grid > 0x7FFFFFFF) return fail(SX8_ERR_UNSUPPORTED, "sx8_dequant_f16: tensor too large");
@@ -143,6 +294,10 @@ extern "C" int32_t sx8_embed_gather(const int64_t* ids, int64_t T, const uint8_t
         return fail(SX8_ERR_INVALID, "sx8_embed_gather: misaligned pointer");
     if (T == 0) return ok();
     const bool vec_ok = aligned(out, 16) && (K % 8 == 0);
+    const hipStream_t st = as_stream(stream);
+    if (hdr_bytes == 8 ? launch_wave(V44Src<8>{hdr, levels, N}, ids, basis, scales, T, N, n_cb, K, vec_ok, out, st)
+                       : launch_wave(V44Src<6>{hdr, levels, N}, ids, basis, scales, T, N, n_cb, K, vec_ok, out, st))
+        return check_launch("sx8_embed_gather");
     const int64_t threads = T * n_cb * 4;
     const int64_t grid = (threads + kThreads - 1) / kThreads;
     if (grid > 0x7FFFFFFF) return fail(SX8_ERR_UNSUPPORTED, "sx8_embed_gather: too many rows");

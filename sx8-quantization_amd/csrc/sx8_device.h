@@ -78,11 +78,9 @@ __host__ __device__ __forceinline__ void sx8_r64_subblock(float lo_f, float hi_f
     const double q = (double)d32 * 0.25;
     const double lo64 = (double)lo_f, hi64 = (double)hi_f;
     const uint32_t s = (cfg >> (2 * sb)) & 3u;
-    double rlo, rhi;
-    if (s == 0u)      { rlo = lo64;     rhi = hi64; }
-    else if (s == 1u) { rlo = lo64;     rhi = lo64 + q; }
-    else if (s == 2u) { rlo = hi64 - q; rhi = hi64; }
-    else              { rlo = lo64 + q; rhi = hi64 - q; }
+    const double lq = lo64 + q, hq = hi64 - q;
+    const double rlo = s == 2u ? hq : s == 3u ? lq : lo64;
+    const double rhi = s == 1u ? lq : s == 3u ? hq : hi64;
     double step = (rhi - rlo) * 0.015873;
     if (step < 1e-10) step = 1e-10;
     const double p0 = (1.0 * (double)sx8_sext4(coeff)) * s0;
@@ -93,7 +91,9 @@ __host__ __device__ __forceinline__ void sx8_r64_subblock(float lo_f, float hi_f
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int i = 2 * j + e;
-            double w = __builtin_fma(step, (double)sx8_level(H, P, i), rlo);
+            // (the level as 2^52 + lv minus 2^52: exact, and cheaper than an integer conversion)
+            const double lv = __builtin_bit_cast(double, 0x4330000000000000ull | sx8_level(H, P, i)) - 4503599627370496.0;
+            double w = __builtin_fma(step, lv, rlo);
             if constexpr (kPca) {
                 w = __builtin_fma(p0, b0[i], w);
                 w = __builtin_fma(p1, b1[i], w);
@@ -141,6 +141,27 @@ __device__ __forceinline__ float sx8_silu_mul(float g, float u) {
     float x = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
     asm volatile("" : "+v"(x));
     return x;
+}
+
+// v_permlane32_swap / v_permlane16_swap: the upper half (the odd 16-lane rows) of a against
+// the lower half (the even rows) of b.
+__device__ __forceinline__ void sx8_swap32(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void sx8_swap16(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+// v[i] of 16-lane row t -> v[t] of row i
+__device__ __forceinline__ void sx8_transpose4(uint32_t (&v)[4]) {
+    sx8_swap32(v[0], v[2]);
+    sx8_swap32(v[1], v[3]);
+    sx8_swap16(v[0], v[1]);
+    sx8_swap16(v[2], v[3]);
 }
 
 // v with lanes 0-31 and 32-63 swapped (v_permlane32_swap).

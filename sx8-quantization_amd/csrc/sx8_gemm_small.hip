@@ -113,27 +113,6 @@ __device__ __forceinline__ void load_record(Rec& r, const RecSrc& s, uint32_t bi
     }
 }
 
-// v_permlane32_swap / v_permlane16_swap: the upper half (the odd 16-lane rows) of a against
-// the lower half (the even rows) of b.
-__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = r[0];
-    b = r[1];
-}
-__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    a = r[0];
-    b = r[1];
-}
-
-// v[i] of 16-lane row t -> v[t] of row i
-__device__ __forceinline__ void transpose4(uint32_t (&v)[4]) {
-    swap32(v[0], v[2]);
-    swap32(v[1], v[3]);
-    swap16(v[0], v[1]);
-    swap16(v[2], v[3]);
-}
-
 typedef sx8_u32x4 u32x4;
 
 // One column fragment's four blocks, ready to decode.  kT (transposed): element t is this
@@ -169,19 +148,19 @@ __device__ __forceinline__ void frag_prep(Frag& f, const Rec& r) {
     f.h[2] = r.h.z;
     f.h[3] = r.h.w;
     if constexpr (kT) {
-        transpose4(f.h);
-        transpose4(f.rlo);
-        transpose4(f.step);
+        sx8_transpose4(f.h);
+        sx8_transpose4(f.rlo);
+        sx8_transpose4(f.step);
         // quads: words x (sub-blocks 0, 1) and y (2, 3); rows g < 2 need x, g >= 2 y, of every
         // block: one half swap, then each register copied across its row pair
         uint32_t a = r.q.x, b = r.q.y;
-        swap32(a, b);
+        sx8_swap32(a, b);
         f.p[0] = a;
         f.p[1] = a;
-        swap16(f.p[0], f.p[1]);
+        sx8_swap16(f.p[0], f.p[1]);
         f.p[2] = b;
         f.p[3] = b;
-        swap16(f.p[2], f.p[3]);
+        sx8_swap16(f.p[2], f.p[3]);
     } else {
         f.p[0] = f.p[1] = r.q.x;
         f.p[2] = f.p[3] = r.q.y;
