@@ -20,6 +20,7 @@ LIB_NAME = "libsx8_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = ["sx8_abi.hip", "sx8_dequant.hip", "sx8_layout.hip", "sx8_quant.hip", "sx8_gemv.hip",
            "sx8_gemm.hip", "sx8_gemm_small.hip", "sx8_decoder.hip"]
+PY_SOURCE, PY_PATH = "sx8_py.cpp", os.path.join(PKG_DIR, "_sx8py.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # hipcc flags: gfx950 only, no packed-fp32 instruction selection (those forms have
@@ -117,12 +118,13 @@ SIGNATURES = [
 ABI_VERSION = 5
 
 _lib = None
+_py = None
 _lock = threading.Lock()
 
 
 def build(verbose: bool = False) -> str:
     """Compile every HIP source for gfx950 with hipcc (one object per source, in parallel)
-    and link LIB_PATH (always rebuilds)."""
+    and link LIB_PATH, and compile the host module PY_PATH with g++ (always rebuilds)."""
     from concurrent.futures import ThreadPoolExecutor
     import tempfile
     with tempfile.TemporaryDirectory(prefix="sx8_build_") as d:
@@ -132,9 +134,13 @@ def build(verbose: bool = False) -> str:
             cmd = [HIPCC, *flags, "-I", CSRC_DIR, "-I", INCLUDE_DIR, "-c", "-o", obj,
                    os.path.join(CSRC_DIR, name)]
             return obj, subprocess.run(cmd, capture_output=True, text=True)
-        jobs = min(len(SOURCES), max(1, (os.cpu_count() or 1)), 8)
+        jobs = min(len(SOURCES) + 1, max(1, (os.cpu_count() or 1)), 8)
         with ThreadPoolExecutor(jobs) as ex:
+            py = ex.submit(_build_py)
             results = list(ex.map(compile_one, SOURCES))
+            res = py.result()
+        if res.returncode != 0:
+            raise RuntimeError(f"{PY_SOURCE}: the compiler failed:\n" + res.stdout + res.stderr)
         errs = [r.stdout + r.stderr for _, r in results if r.returncode != 0]
         if errs:
             raise RuntimeError("hipcc failed:\n" + "\n".join(errs))
@@ -147,7 +153,24 @@ def build(verbose: bool = False) -> str:
         if res.returncode != 0:
             raise RuntimeError("hipcc link failed:\n" + res.stdout + res.stderr)
     os.replace(tmp, LIB_PATH)
+    os.replace(PY_PATH + ".tmp", PY_PATH)
     return LIB_PATH
+
+
+def _build_py():
+    """Compile PY_SOURCE to PY_PATH.tmp against torch's headers and libraries."""
+    import sysconfig
+    import torch
+    T = os.path.dirname(os.path.abspath(torch.__file__))
+    inc = [os.path.join(T, "include"), os.path.join(T, "include", "torch", "csrc", "api", "include"),
+           os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    libs = os.path.join(T, "lib")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(a for i in inc for a in ("-isystem", i)),
+           os.path.join(CSRC_DIR, PY_SOURCE), "-o", PY_PATH + ".tmp", "-L", libs, "-ltorch", "-ltorch_cpu",
+           "-ltorch_python", "-lc10", "-lc10_hip", "-Wl,-rpath," + libs]
+    return subprocess.run(cmd, capture_output=True, text=True)
 
 
 def lib_path() -> str:
@@ -193,6 +216,27 @@ def lib():
                 raise RuntimeError(f"{path}: ABI version {L.sx8_abi_version()} != {ABI_VERSION}")
             _lib = L
     return _lib
+
+
+def py():
+    """The host module of sx8_py.cpp, bound to the library that lib() loaded; RuntimeError if
+    it is missing."""
+    global _py
+    if _py is not None:
+        return _py
+    L = lib()
+    with _lock:
+        if _py is None:
+            import importlib.util
+            if not os.path.exists(PY_PATH):
+                raise RuntimeError(f"S-X8 host module not found at {PY_PATH}; run "
+                                   "__graft_entry__.build() (or _sx8lib.build()) first")
+            spec = importlib.util.spec_from_file_location("_sx8py", PY_PATH)
+            m = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(m)
+            m.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name, _, _ in SIGNATURES})
+            _py = m
+    return _py
 
 
 def call(name: str, *args) -> None:

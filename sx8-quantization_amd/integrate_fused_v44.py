@@ -19,6 +19,7 @@ import os
 import torch
 import torch.nn as nn
 
+import _sx8lib as _L
 from sx8_decode1_v3 import decode1_v44, best_split_k, make_tensors_v44
 from sx8_embed_v44 import SX8EmbeddingV44
 from sx8_fused_wmma import gemm_sx8_wmma_cached, make_tensors, to_kbmajor
@@ -47,6 +48,11 @@ class SX8LinearV44(nn.Module):
                                          hdr_aligned=(self.hdr_bytes == 8))
 
     def forward(self, x):
+        if self._t44 is not None:
+            qt = self.qt
+            y = _L.py().linear(x, self._t44, self.hdr_bytes, self.bias, self.out_f, *qt["shape"], qt["n_cb"])
+            if y is not None:
+                return y
         x = x.contiguous()
         orig_shape = x.shape
         if x.dim() != 2:

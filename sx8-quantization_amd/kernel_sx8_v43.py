@@ -61,8 +61,13 @@ def decode_tensor_gpu_fast(qt, bases_info, out=None):
             return _dequant_into(qt, bases_info, out, out.device)
         out.copy_(_dequant_into(qt, bases_info, torch.empty_like(out, memory_format=torch.contiguous_format), out.device))
         return out
-    W = torch.empty((out_f, in_f), dtype=torch.float16, device=DEV)
-    _dequant_into(qt, bases_info, W, DEV)
+    W = None
+    if int(qt["n_blocks"]) == out_f * int(qt["n_cb"]):
+        W = _L.py().dequant(qt["dmin"], qt["dmax"], qt["config"], qt["coeff"], qt["levels_hi"], qt["levels_lo"],
+                            bases_info["data"], bases_info["scales"], out_f, in_f, int(qt["n_cb"]))
+    if W is None:
+        W = torch.empty((out_f, in_f), dtype=torch.float16, device=DEV)
+        _dequant_into(qt, bases_info, W, DEV)
     orig = qt.get("orig_shape")
     if orig is not None and tuple(orig) != (out_f, in_f):
         W = W.reshape(orig)

@@ -150,7 +150,9 @@ class _HostFields:
     def to_host(self):
         """{name: numpy array}, or None when the bases or scales are not finite (weights with
         infinities or NaN: the caller takes the general path)."""
-        host = self.buf.cpu().numpy()
+        import _sx8lib as _L
+        host = _L.py().to_host(self.buf)
+        host = (self.buf.cpu() if host is None else host).numpy()
         f = {name: host[off:off + nb].view(dt) for name, (off, nb, dt) in self.at.items()}
         f["data"], f["scales"] = f["data"].reshape(self.n_cb, 64), f["scales"].reshape(self.n_cb, 2)
         return f if np.isfinite(f["data"]).all() and np.isfinite(f["scales"]).all() else None

@@ -139,6 +139,8 @@ def decode1_v44(X, qt, bases_info, hdr_t=None, lvl_t=None, bas_t=None, sca_t=Non
     # The reference passes a pooled Z scratch to decode1_v44_combined; nothing reads it
     # afterwards, so the Z output is skipped here, which lets the HIP GEMV build its
     # activation table inside the single launch.
+    if _L.py().gemv(X, hdr_t, lvl_t, bas_t, sca_t, hdr_bytes, N, n_cb, Y):
+        return Y, (hdr_t, lvl_t, bas_t, sca_t)
     Xc = _x_for_kernel(X, n_cb)
     ws = _workspace(n_cb, Xc.device) if n_cb > _LDS_MAX_KB else None
     _L.call("sx8_gemv", _L.ptr(Xc), _L.ptr(hdr_t), _L.ptr(lvl_t), int(hdr_bytes), _L.ptr(bas_t),

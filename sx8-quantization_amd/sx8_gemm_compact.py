@@ -93,6 +93,9 @@ def gemm_sx8_compact(X, qt, bases_info, hdr_t=None, lvl_t=None, bas_t=None, sca_
         from sx8_decode1_v3 import make_tensors_v44
         hdr_t, lvl_t, bas_t, sca_t = make_tensors_v44(qt, bases_info,
                                                       hdr_aligned=(hdr_bytes == 8))
+    Y = _L.py().gemm(X, hdr_t, lvl_t, bas_t, sca_t, hdr_bytes, out_f, in_f, n_cb)
+    if Y is not None:
+        return Y
     Xc = _x2d(X)
     M, K = Xc.shape
     if K < in_f:

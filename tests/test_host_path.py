@@ -1,0 +1,181 @@
+"""The native per-call path of the wrappers (sx8_py.cpp) against their general path: the same
+bits, shapes and types for every form of input, whichever of the two takes it."""
+import numpy as np
+import pytest
+import torch
+
+
+class _Decline:
+    """A host module that takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+@pytest.fixture
+def both(hiplib, monkeypatch):
+    """Run f through the native path, then through the general one; the native calls taken."""
+    import _sx8lib
+
+    def run(f):
+        real, taken = _sx8lib.py(), []
+
+        class Watch:
+            def __getattr__(self, name):
+                def g(*a):
+                    r = getattr(real, name)(*a)
+                    taken.append((name, r is not None))
+                    return r
+                return g
+        monkeypatch.setattr(_sx8lib, "_py", Watch())
+        def result():
+            try:
+                return f().clone()
+            except (RuntimeError, ValueError) as e:
+                return type(e)
+        a = result()
+        monkeypatch.setattr(_sx8lib, "_py", _Decline())
+        b = result()
+        monkeypatch.setattr(_sx8lib, "_py", real)
+        return a, b, [n for n, t in taken if t]
+    return run
+
+
+def _same(a, b):
+    if isinstance(b, type):                              # refused
+        assert a is b
+        return
+    assert a.shape == b.shape and a.dtype == b.dtype and a.device == b.device and a.stride() == b.stride()
+    a, b = a.detach(), b.detach()
+    assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+def _weight(N, K, seed=3):
+    from quantize_sx8 import quantize_tensor
+    g = torch.Generator().manual_seed(seed)
+    return quantize_tensor((torch.randn(N, K, generator=g) * 0.02).half(), device="cpu", degenerate_frac=0.01, seed=1)
+
+
+def test_host_tensors_are_left_to_the_general_path(hiplib):
+    import _sx8lib
+    py = _sx8lib.py()
+    h, f = torch.zeros(1, 64, dtype=torch.float16), torch.zeros(64)
+    u = torch.zeros(128, 6, dtype=torch.uint8)
+    assert py.linear(h, (u, u, f, f), 6, None, 64, 64, 64, 2) is None
+    assert py.gemv(h[0], u, u, f, f, 6, 64, 2, f) is None
+    assert py.gemm(h, u, u, f, f, 6, 64, 64, 2) is None
+    assert py.gemm_split(h, f, f, u, u, u, u, f, f, 2) is None
+    assert py.dequant(h, h, u, u, u, u, f, f, 64, 64, 2) is None
+    assert py.dequant(*[np.zeros(4)] * 8, 64, 64, 2) is None
+    assert py.embed(torch.zeros(1, dtype=torch.long), u, u, f, f, 64, 64, 2, h) is None
+    assert py.to_host(u) is None
+    with pytest.raises(TypeError):
+        py.linear(h)
+    with pytest.raises(KeyError):
+        py.bind({})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hdr", [6, 8])
+@pytest.mark.parametrize("N,K", [(96, 100), (40, 64)])
+def test_linear_forms(both, cuda, N, K, hdr):
+    from integrate_fused_v44 import SX8LinearV44
+    qt, bi = _weight(N, K)
+    g = torch.Generator().manual_seed(5)
+    X = torch.randn(80, K + 3, generator=g).half().to(cuda)
+    bias = torch.nn.Parameter(torch.randn(N, generator=g).half().to(cuda))
+    forms = {"rows1": X[:1, :K].contiguous(), "vec": X[3, :K].contiguous(), "offset": X.reshape(-1)[1:1 + K],
+             "strided": X[:7, :K], "transposed": X[:5, :K].t().contiguous().t(),
+             "batch": X[:6, :K].reshape(2, 3, K), "rows32": X[:32, :K].contiguous(), "rows33": X[:33, :K].contiguous(),
+             "empty_batch_dims": X[:1, :K].reshape(1, 1, 1, K), "float": X[:2, :K].float(), "longer": X[:2].contiguous()}
+    for b, grad in ((None, False), (bias, False), (bias, True), (bias.detach().float(), False)):
+        m = SX8LinearV44(qt, bi, b, hdr_bytes=hdr)
+        m._load_t44()
+        for name, x in forms.items():
+            with torch.set_grad_enabled(grad):
+                y, ref, taken = both(lambda: m(x))
+            _same(y, ref)
+            if isinstance(y, torch.Tensor):
+                assert y.requires_grad == ref.requires_grad, name
+            if name in ("rows1", "vec", "offset") and b is None:
+                assert taken == ["linear"], name
+
+
+@pytest.mark.gpu
+def test_wrappers(both, cuda, monkeypatch):
+    from kernel_sx8_v43 import decode_tensor_gpu_fast
+    from sx8_decode1_v3 import decode1_v44, make_tensors_v44
+    from sx8_embed_v44 import SX8EmbeddingV44
+    from sx8_fused_wmma import gemm_sx8_wmma_cached, make_tensors, to_kbmajor
+    from sx8_gemm_compact import gemm_sx8_compact
+    N, K = 130, 96
+    qt, bi = _weight(N, K)
+    g = torch.Generator().manual_seed(6)
+    X = torch.randn(140, K + 8, generator=g).half().to(cuda)
+    t = make_tensors_v44(qt, bi)
+    split = make_tensors(to_kbmajor(qt, bi)[0], bi, cuda)
+    for x in (X[:1, :K].contiguous(), X[:77, :K].contiguous(), X[:3, :K], X[:5].contiguous(), X[:2, :K].float()):
+        y, ref, taken = both(lambda: gemm_sx8_compact(x, qt, bi, *t))
+        _same(y, ref)
+        assert (taken == ["gemm"]) == (x.is_contiguous() and x.dtype == torch.float16)
+        y, ref, _ = both(lambda: gemm_sx8_wmma_cached(x, split, qt["n_cb"]))
+        _same(y, ref)
+    with pytest.raises(ValueError):
+        gemm_sx8_compact(X[:4, :K - 1].contiguous(), qt, bi, *t)
+    for x in (X[0, :K].contiguous(), X[0, :K - 4], X.reshape(-1)[3:3 + K], X[:1, :K].float(), X[1]):
+        y, ref, _ = both(lambda: decode1_v44(x, qt, bi, *t)[0])
+        _same(y, ref)
+    dq = {k: torch.as_tensor(np.ascontiguousarray(v).view(np.int16 if v.dtype == np.float16 else v.dtype)).to(cuda)
+          if isinstance(v, np.ndarray) else v for k, v in qt.items()}
+    db = dict(bi, data=torch.as_tensor(bi["data"]).to(cuda), scales=torch.as_tensor(bi["scales"]).to(cuda))
+    for q, b, want in ((dq, db, ["dequant"]), (dict(dq, dmin=dq["dmin"].view(torch.float16)), db, ["dequant"]),
+                       (qt, bi, []), (dict(dq, orig_shape=(N // 2, 2 * K)), db, ["dequant"]),
+                       (dict(dq, config=dq["config"].int()), db, [])):
+        y, ref, taken = both(lambda: decode_tensor_gpu_fast(q, b))
+        _same(y, ref)
+        assert taken == want
+    with pytest.raises(ValueError):
+        decode_tensor_gpu_fast(dict(dq, n_blocks=1), db)
+    with pytest.raises(ValueError):
+        decode_tensor_gpu_fast(dq, dict(db, scales=db["scales"][:1]))
+    emb = SX8EmbeddingV44(qt, bi)
+    ids = torch.randint(0, N, (4, 9), generator=g).to(cuda)
+    for i in (ids, ids[0], ids[0, 0], ids[:, ::2], ids.int(), ids[:0]):
+        y, ref, taken = both(lambda: emb(i))
+        _same(y, ref)
+
+
+@pytest.mark.gpu
+def test_stream_and_capture(hiplib, cuda):
+    """The native path launches on the current stream, and a graph that captured it replays."""
+    from integrate_fused_v44 import SX8LinearV44
+    qt, bi = _weight(128, 256)
+    m = SX8LinearV44(qt, bi)
+    x = torch.randn(4, 256, dtype=torch.float16, device=cuda)
+    m(x)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        y = m(x)
+    for i in range(3):
+        x.normal_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, m(x))
+        with torch.cuda.stream(s):
+            z = m(x)
+        s.synchronize()
+        assert torch.equal(y, z)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 1 << 20, (1 << 20) + 1, (2 << 20) + 5, (7 << 20) - 3])
+def test_to_host(hiplib, cuda, n):
+    import _sx8lib
+    x = torch.randint(0, 256, (n,), dtype=torch.uint8, device=cuda)
+    for _ in range(2):
+        y = _sx8lib.py().to_host(x)
+        assert (y is None) == (n <= 1 << 20)
+        assert y is None or (not y.is_cuda and torch.equal(y, x.cpu()))
+        x.bitwise_not_()
