@@ -137,17 +137,15 @@ __global__ __launch_bounds__(kThreads) void k_v6_encode(
 //   k_pca_err     residuals e = x - (lo + step lv) in float32 (every operation rounded, the
 //                 steps as products with fp32(1 / 63)), stored K block by K block
 //   k_pca_gram    partial Gram matrices E^T E of row ranges, float64 on the matrix core
-//   k_pca_eig     their sum's two leading eigenvectors by cyclic Jacobi rotations
+//   k_pca_eig     their sum's two leading eigenvectors by repeated squaring on the matrix core
 //   k_pca_coeff   c = basis . e (float64 sums of the float32 values, rounded to float32)
 //   k_pca_scale   the lower median of |c| by radix selection; scale = max(median / 3, 1e-10)
 //   k_pca_byte    c / scale rounded to signed 4 bits
 // The eigenproblems bounded this: a few hundred 32 x 32 matrices took a library's batched solver
 // 13.3 of the 14.7 ms of a 2560 x 4096 tensor (its tridiagonalisation runs column by column,
 // ~430 us a launch) and the median 60 us.  Measured here on that tensor (128 K blocks): V6 encode
-// 37 us (byte stores: 38), residuals 14, Gram 13.5, eigenvectors 157 (latency of ~9 sweeps of 31
-// dependent rounds on 128 work-groups; with a float64 division and square roots per rotation
-// 194), coefficients 8.6, medians 6.4, bytes 4.2; the rest of a call's 0.86 ms is the copy of 9.8
-// MB to pageable host memory.
+// 36 us (byte stores: 38), residuals 14.5, Gram 14, eigenvectors 33, coefficients 8.4, medians
+// 6.6, bytes 3.5; the rest of a call's 0.55 ms is the copy of 9.8 MB to host memory.
 
 constexpr int kPcaSplits = 8;        // row ranges of the Gram sums
 constexpr float kInv63 = 1.0f / 63.0f;
@@ -235,126 +233,168 @@ __global__ __launch_bounds__(256) void k_pca_gram(const float* __restrict__ err,
     }
 }
 
-// One work-group per K block: cyclic Jacobi on the 32 x 32 Gram matrix in LDS, float64.  A sweep
-// is 31 rounds of 16 disjoint rotations (round-robin pairing); in a round thread (p, q) owns the
-// 2 x 2 block (rows of pair p, columns of pair q), so the whole two-sided update is one step
-// without conflicts, two barriers a round.  The rotation's tangent only steers convergence, so
-// it is a float32 value (of a matrix scaled to a largest diagonal near 1); cosine and sine are
-// float64 and orthogonal to its precision, and the updated off-diagonal element is computed,
-// not set to zero.  Ends when the off-diagonal norm is below 1e-13 of the diagonal's (an
-// eigenvector error of 1e-10 at the gaps of 1e-3 that nearly white residuals have), after 20
-// sweeps at the latest.
-__global__ __launch_bounds__(256) void k_pca_eig(const double* __restrict__ part, int n_splits, int n_cb,
-                                                 float* __restrict__ data) {
-    constexpr int kLd = 33;
-    __shared__ double A[32 * kLd], V[32 * kLd], cs[16], sn[16], red[2][4];
-    const int kb = blockIdx.x, tid = threadIdx.x;
-    for (int i = tid; i < 768; i += 256) {
-        const int t = i >> 8, r = (i >> 4) & 15, c = i & 15;
-        double v = 0.0;
-        for (int s = 0; s < n_splits; ++s) v += part[(((int64_t)s * n_cb + kb) * 3 + t) * 256 + (i & 255)];
-        const int rr = r + (t == 2 ? 16 : 0), cc = c + (t >= 1 ? 16 : 0);
-        A[rr * kLd + cc] = v;
-        if (t == 1) A[cc * kLd + rr] = v;
-    }
-    for (int i = tid; i < 1024; i += 256) V[(i >> 5) * kLd + (i & 31)] = (i >> 5) == (i & 31) ? 1.0 : 0.0;
-    __syncthreads();
-    // scale by a power of two (the eigenvectors stay)
-    double top = 0.0;
-    for (int i = 0; i < 32; ++i) top = fmax(top, A[i * kLd + i]);
-    const int ex = top > 0.0 && top < 1e300 ? -ilogb(top) : 0;
-    __syncthreads();
-    for (int i = tid; i < 1024; i += 256) A[(i >> 5) * kLd + (i & 31)] = ldexp(A[(i >> 5) * kLd + (i & 31)], ex);
-    __syncthreads();
-    const int p = tid >> 4, q = tid & 15;
-    auto pair = [](int r, int k, int& a, int& b) {
-        a = k == 0 ? 31 : r + k >= 31 ? r + k - 31 : r + k;
-        b = k == 0 ? r : r - k < 0 ? r - k + 31 : r - k;
-    };
-    for (int sweep = 0; sweep < 20; ++sweep) {
-        double off = 0.0, dia = 0.0;
-        for (int i = tid; i < 1024; i += 256) {
-            const double v = A[(i >> 5) * kLd + (i & 31)];
-            if ((i >> 5) == (i & 31)) dia += v * v;
-            else off += v * v;
-        }
+// One work-group of three waves per K block: the two leading eigenvectors of the 32 x 32 Gram
+// matrix by repeated squaring in float64.  B^(2^k) of a positive semi-definite B tends to the
+// projector on its largest eigenvalue, whose longest column is the vector; the second vector is
+// the same of the deflated matrix A - v w^T - w v^T + (v.w) v v^T, w = A v.  A squaring is one
+// 16 x 16 tile a wave (tiles 00, 01, 11 of a symmetric result; 8 f64 MFMAs whose two operands
+// are both rows of B), with one barrier: the result goes to the other of two buffers, scaled by
+// a power of two that the trace of B gives.  tr(B)^2 - tr(B^2) is twice the share of the other
+// eigenvalues to first order, so once it is below 1e-8 one more squaring leaves 1e-16; the
+// rounding errors shrink with the powers like the gap grows, so the vectors are good to a few
+// 2^-53 / (relative gap).  Gaps below 1e-12 end after 45 squarings with a vector of the two's
+// plane.  Residuals of trained or random weights take 9 to 17 squarings a vector, each ~0.4 us
+// of LDS, MFMA and barrier latency: 33 us for the 128 K blocks of a 2560 x 4096 tensor, where
+// cyclic Jacobi rotations (some 8 sweeps of 31 dependent rounds) took 157 and were good to
+// 1e-13 / gap.
+constexpr int kEigThreads = 192;
+constexpr int kEigLd = 36;           // doubles: the operand reads spread over all banks
+constexpr int kEigSquarings = 45;
+
+struct EigSmem {
+    double A[32 * kEigLd];
+    __attribute__((aligned(16))) double B[2][32 * kEigLd], dg[2][32], v[2][32], w[32];
+};
+
+__device__ __forceinline__ double eig_sum(const double* d) {
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            off += __shfl_xor(off, o);
-            dia += __shfl_xor(dia, o);
+    for (int i = 0; i < 32; ++i) s[i & 3] += d[i];
+    return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+// index of the largest of f(d[0]) .. f(d[31]), the first of equals
+template <typename F>
+__device__ __forceinline__ int eig_argmax(const double* d, F f) {
+    int j = 0;
+    double best = f(d[0]);
+#pragma unroll
+    for (int i = 1; i < 32; ++i) {
+        const double x = f(d[i]);
+        if (x > best) {
+            best = x;
+            j = i;
         }
-        if ((tid & 63) == 0) {
-            red[0][tid >> 6] = off;
-            red[1][tid >> 6] = dia;
+    }
+    return j;
+}
+
+// The leading vector of B[0] (positive trace, diagonal in dg[0], both behind a barrier), made
+// orthogonal to v[0] if second, into v[second].
+__device__ __forceinline__ void eig_lead(EigSmem& sm, int second) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int ra = wave == 2 ? 16 : 0, rb = wave == 0 ? 0 : 16;
+    const int row = lane >> 4, col = lane & 15;
+    int cur = 0;
+    double prev = 0.0;
+    bool last = false;
+    for (int k = 0; k < kEigSquarings && !last; ++k) {       // the same for every thread
+        const double* a = sm.B[cur] + (ra + col) * kEigLd + row;
+        const double* b = sm.B[cur] + (rb + col) * kEigLd + row;
+        sx8_double4 acc[2];
+        acc[0] = acc[1] = sx8_double4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            acc[s & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[4 * s], b[4 * s], acc[s & 1], 0, 0, 0);
+        const double t = eig_sum(sm.dg[cur]);
+        last = k > 0 && prev * prev - t <= 1e-8 * (prev * prev);
+        const int ex = __builtin_amdgcn_frexp_exp(t);
+        prev = __builtin_amdgcn_ldexp(t, -ex);
+        double* o = sm.B[cur ^ 1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double d = __builtin_amdgcn_ldexp(acc[0][i] + acc[1][i], -2 * ex);
+            const int r = ra + row + 4 * i, c = rb + col;
+            o[r * kEigLd + c] = d;
+            if (wave == 1) o[c * kEigLd + r] = d;
+            else if (r == c) sm.dg[cur ^ 1][r] = d;
         }
         __syncthreads();
-        off = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-        dia = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
-        if (!(off > 1e-26 * dia)) break;             // the same for every thread; also ends on NaN
-        for (int r = 0; r < 31; ++r) {
-            if (tid < 16) {
-                int a, b;
-                pair(r, tid, a, b);
-                const float x = (float)A[a * kLd + b];
-                float t = 0.f;
-                if (x != 0.f) {
-                    const float tau = (float)(A[b * kLd + b] - A[a * kLd + a]) * __builtin_amdgcn_rcpf(x + x);
-                    const float at = fabsf(tau);
-                    t = at < 1e18f ? __builtin_amdgcn_rcpf(at + __builtin_amdgcn_sqrtf(1.f + at * at)) : 0.f;
-                    t = tau < 0.f ? -t : t;
-                }
-                const double y = __builtin_fma((double)t, (double)t, 1.0);      // 1 .. 2
-                double c = __builtin_amdgcn_rsq(y);
-                c = __builtin_fma(0.5 * c, __builtin_fma(-y * c, c, 1.0), c);   // Newton steps
-                c = __builtin_fma(0.5 * c, __builtin_fma(-y * c, c, 1.0), c);
-                cs[tid] = c;
-                sn[tid] = (double)t * c;
-            }
-            __syncthreads();
-            int ip, jp, iq, jq;
-            pair(r, p, ip, jp);
-            pair(r, q, iq, jq);
-            const double cp = cs[p], sp = sn[p], cq = cs[q], sq = sn[q];
-            const double a00 = A[ip * kLd + iq], a01 = A[ip * kLd + jq];
-            const double a10 = A[jp * kLd + iq], a11 = A[jp * kLd + jq];
-            const double b00 = cp * a00 - sp * a10, b01 = cp * a01 - sp * a11;
-            const double b10 = sp * a00 + cp * a10, b11 = sp * a01 + cp * a11;
-            A[ip * kLd + iq] = cq * b00 - sq * b01;
-            A[ip * kLd + jq] = sq * b00 + cq * b01;
-            A[jp * kLd + iq] = cq * b10 - sq * b11;
-            A[jp * kLd + jq] = sq * b10 + cq * b11;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                double* v = V + (p + 16 * h) * kLd;
-                const double v0 = v[iq], v1 = v[jq];
-                v[iq] = cq * v0 - sq * v1;
-                v[jq] = sq * v0 + cq * v1;
-            }
-            __syncthreads();
-        }
+        cur ^= 1;
     }
-    // the two largest eigenvalues; each vector's largest-magnitude component positive
-    if (tid < 2) {
-        int best = 0, second = 1;
-        if (A[kLd + 1] > A[0]) {
-            best = 1;
-            second = 0;
+    if (wave == 0) {
+        const int j = eig_argmax(sm.dg[cur], [](double d) { return d; });
+        double* v = sm.v[second];
+        const int i = lane & 31;
+        double x = sm.B[cur][j * kEigLd + i];
+        auto unit = [&]() {                                   // v = x / |x|, in every lane's x
+            if (lane < 32) sm.w[i] = x * x;
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            x /= sqrt(eig_sum(sm.w));
+        };
+        unit();
+        if (second) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            if (lane < 32) sm.w[i] = x * sm.v[0][i];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            x -= eig_sum(sm.w) * sm.v[0][i];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            unit();
         }
-        for (int i = 2; i < 32; ++i) {
-            const double v = A[i * kLd + i];
-            if (v > A[best * kLd + best]) {
-                second = best;
-                best = i;
-            } else if (v > A[second * kLd + second]) {
-                second = i;
-            }
-        }
-        const int col = tid == 0 ? best : second;
-        int arg = 0;
-        for (int i = 1; i < 32; ++i)
-            if (fabs(V[i * kLd + col]) > fabs(V[arg * kLd + col])) arg = i;
-        const double sg = V[arg * kLd + col] < 0.0 ? -1.0 : 1.0;
-        for (int i = 0; i < 32; ++i) data[(int64_t)kb * 64 + 32 * tid + i] = (float)(sg * V[i * kLd + col]);
+        if (lane < 32) v[i] = x;
+    }
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(kEigThreads) void k_pca_eig(const double* __restrict__ part, int n_splits, int n_cb,
+                                                         float* __restrict__ data) {
+    __shared__ EigSmem sm;
+    const int kb = blockIdx.x, tid = threadIdx.x;
+#pragma unroll
+    for (int i = tid; i < 768; i += kEigThreads) {
+        const int t = i >> 8, r = (i >> 4) & 15, c = i & 15;
+        double v = 0.0;
+#pragma unroll 8
+        for (int s = 0; s < n_splits; ++s) v += part[(((int64_t)s * n_cb + kb) * 3 + t) * 256 + (i & 255)];
+        const int rr = r + (t == 2 ? 16 : 0), cc = c + (t >= 1 ? 16 : 0);
+        sm.A[rr * kEigLd + cc] = sm.B[0][rr * kEigLd + cc] = v;
+        if (t == 1) sm.A[cc * kEigLd + rr] = sm.B[0][cc * kEigLd + rr] = v;
+        if (rr == cc) sm.dg[0][rr] = v;
+    }
+    __syncthreads();
+    const double tr = eig_sum(sm.dg[0]);
+    float* out = data + (int64_t)kb * 64;
+    if (!(tr < 1e150)) {                              // infinities or NaN in the weights
+        if (tid < 64) out[tid] = __builtin_nanf("");
+        return;
+    }
+    if (tr > 0.0) {
+        eig_lead(sm, 0);
+    } else {                                          // no residual at all
+        if (tid < 32) sm.v[0][tid] = tid == 0 ? 1.0 : 0.0;
+        __syncthreads();
+    }
+    if (tid < 32) {
+        double w = 0.0;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) w = __builtin_fma(sm.A[tid * kEigLd + i], sm.v[0][i], w);
+        sm.w[tid] = w;
+    }
+    __syncthreads();
+    double c = 0.0;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) c = __builtin_fma(sm.w[i], sm.v[0][i], c);
+    for (int i = tid; i < 1024; i += kEigThreads) {
+        const int x = i >> 5, y = i & 31;
+        const double vx = sm.v[0][x], vy = sm.v[0][y];
+        const double d = sm.A[x * kEigLd + y] - (vx * sm.w[y] + sm.w[x] * vy) + c * vx * vy;
+        sm.B[0][x * kEigLd + y] = d;
+        if (x == y) sm.dg[0][x] = d;
+    }
+    __syncthreads();
+    if (eig_sum(sm.dg[0]) > 1e-13 * tr) {
+        eig_lead(sm, 1);
+    } else if (tid < 32) {                            // one direction only: any unit vector beside it
+        const int j = eig_argmax(sm.v[0], [](double d) { return -fabs(d); });
+        const double p = sm.v[0][j];                  // e_j - p v, of squared length 1 - p^2
+        sm.v[1][tid] = ((tid == j ? 1.0 : 0.0) - p * sm.v[0][tid]) / sqrt(1.0 - p * p);
+    }
+    __syncthreads();
+    if (tid < 64) {                                   // the largest-magnitude component positive
+        const double* v = sm.v[tid >> 5];
+        const int arg = eig_argmax(v, [](double d) { return fabs(d); });
+        out[tid] = (float)(v[arg] < 0.0 ? -v[tid & 31] : v[tid & 31]);
     }
 }
 
@@ -542,7 +582,7 @@ extern "C" int32_t sx8_quant_pca(const void* blocks, const void* dmin, const voi
     const int rows_per = (int)((n_rows + kPcaSplits - 1) / kPcaSplits);
     hipLaunchKernelGGL(k_pca_gram, dim3((unsigned)n_cb, kPcaSplits), dim3(256), 0, st, err, (int)n_rows, rows_per,
                        part);
-    hipLaunchKernelGGL(k_pca_eig, dim3((unsigned)n_cb), dim3(256), 0, st, part, kPcaSplits, (int)n_cb, data);
+    hipLaunchKernelGGL(k_pca_eig, dim3((unsigned)n_cb), dim3(kEigThreads), 0, st, part, kPcaSplits, (int)n_cb, data);
     hipLaunchKernelGGL(k_pca_coeff, dim3((unsigned)row_grid, (unsigned)n_cb), dim3(kThreads), 0, st, err, data,
                        (int)n_rows, craw);
     hipLaunchKernelGGL(k_pca_scale, dim3((unsigned)(2 * n_cb)), dim3(1024), 0, st, craw, (int)n_rows, scales);

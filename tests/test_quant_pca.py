@@ -1,4 +1,4 @@
-"""sx8_quant_pca (residuals, Gram matrices, Jacobi eigenvectors, coefficients, medians) against
+"""sx8_quant_pca (residuals, Gram matrices, eigenvectors, coefficients, medians) against
 numpy on the same blocks: the residuals restated in float32 with the kernel's roundings, the
 Gram matrix and its eigenvectors in float64, the coefficients from the float32 bases.  Row
 counts at the edges of the Gram ranges and of the 256-row passes, K blocks at those of the
@@ -54,7 +54,7 @@ def test_pca_against_numpy(hiplib, cuda, n_rows, n_cb, f16):
         for k in range(2):
             v = data[kb, 32 * k:32 * k + 32].astype(np.float64)
             assert v[np.abs(v).argmax()] > 0
-            # float64 Jacobi, stored in float32: an eigenvector to a float32 rounding, of the
+            # computed in float64, stored in float32: an eigenvector to a float32 rounding, of the
             # right eigenvalue, and numpy's vector up to sign where the gap resolves it
             assert abs(v @ v - 1) <= 1e-6
             assert np.abs(G[kb] @ v - lam[kb, -1 - k] * v).max() <= 1e-6 * lam[kb, -1]
@@ -98,3 +98,34 @@ def test_pca_refusals(hiplib):
     assert call(x=N0) == 1 and call(ws=N0) == 1 and call(nb=need - 1) == 1 and call(r=0) == 1
     assert call(x=ctypes.c_void_p(4097)) == 1 and call(ws=ctypes.c_void_p(4104)) == 1
     assert b"misaligned" in L.sx8_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["zero", "rank1", "rank2_1e-5", "identity", "tiny_identity", "gap_2e-6", "gap_1e-7",
+                                  "equal_pair", "large"])
+def test_pca_spectra(hiplib, cuda, kind):
+    """Residuals with chosen Gram spectra (levels and ranges of zero: the residual is the block):
+    unit, orthogonal vectors, each an eigenvector of its eigenvalue, whatever the gaps; the
+    subspace of the two where their common gap resolves it."""
+    import torch
+    from quantize_sx8 import pca_correct
+    rng = np.random.default_rng(7)
+    Q = np.linalg.qr(rng.standard_normal((32, 32)))[0]
+    tail = np.linspace(0.5, 0.1, 30)
+    s = {"zero": np.zeros(32), "rank1": np.r_[1, np.zeros(31)], "rank2_1e-5": np.r_[1, 1e-5, np.zeros(30)],
+         "identity": np.ones(32), "tiny_identity": np.ones(32) * 1e-18, "gap_2e-6": np.r_[1, 1 - 1e-6, tail],
+         "gap_1e-7": np.r_[1, 1 - 6e-8, tail], "equal_pair": np.r_[1, 1, tail], "large": np.r_[1, .9, tail] * 1e15}[kind]
+    E = (s[:, None] * (np.eye(32) if "identity" in kind else Q)).astype(np.float32)
+    z = torch.zeros(32, device=cuda)
+    _, data, _ = pca_correct(torch.zeros(32, 32, dtype=torch.uint8, device=cuda), z, z, z.int(),
+                             torch.from_numpy(E).to(cuda), 1, "gram")
+    G = E.astype(np.float64).T @ E.astype(np.float64)
+    lam, vec = np.linalg.eigh(G)
+    v = data.reshape(2, 32).astype(np.float64)
+    assert np.abs(v @ v.T - np.eye(2)).max() <= 1e-6           # float32 storage: 32 2^-24 at most
+    for k in range(2):
+        assert np.abs(G @ v[k] - lam[-1 - k] * v[k]).max() <= 1e-6 * lam[-1]
+        assert v[k][np.abs(v[k]).argmax()] >= 0
+    if (lam[-2] - lam[-3]) > 1e-3 * lam[-1]:
+        U = vec[:, -2:]
+        assert np.abs(v - v @ U @ U.T).max() <= 1e-6
