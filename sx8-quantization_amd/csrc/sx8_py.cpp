@@ -62,6 +62,13 @@ typedef pybind11::gil_scoped_release Unlocked;
 
 int64_t num(PyObject* o) { return PyLong_AsLongLong(o); }
 
+// A size that is no integer (a float, say) is the general path's to convert or refuse.
+#define SX8_SIZES_OK()      \
+    if (PyErr_Occurred()) { \
+        PyErr_Clear();      \
+        Py_RETURN_NONE;     \
+    }
+
 void* stream_of(const at::Tensor& x) { return c10::hip::getCurrentHIPStream(x.device().index()).stream(); }
 
 PyObject* failed(const char* name, int32_t rc) {
@@ -107,7 +114,8 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t na) {
     SX8_ARGS(8)
     const at::Tensor* x = dev(a[0], at::kHalf);
     if (!x || x->dim() < 1 || !PyTuple_Check(a[1]) || PyTuple_GET_SIZE(a[1]) != 4) Py_RETURN_NONE;
-    const int64_t out_f = num(a[4]), N = num(a[5]), K = num(a[6]), n_cb = num(a[7]);
+    const int64_t out_f = num(a[4]), N = num(a[5]), K = num(a[6]), n_cb = num(a[7]), hb = num(a[2]);
+    SX8_SIZES_OK()
     const int64_t M = K > 0 && x->size(-1) == K ? x->numel() / K : 0;
     if (M < 1 || M > kLinearRows || out_f != N) Py_RETURN_NONE;
     if (M > 1) {
@@ -124,7 +132,6 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t na) {
             (b->requires_grad() && c10::GradMode::is_enabled()))
             Py_RETURN_NONE;
     }
-    const int32_t hb = (int32_t)num(a[2]);
     c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
     shape.back() = N;
     at::Tensor y;
@@ -133,7 +140,7 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t na) {
         Unlocked u;
         const at::Tensor xc = x->is_contiguous() ? *x : x->contiguous();
         y = empty_like_device(shape, at::kHalf, *x);
-        rc = lib.linear(xc.data_ptr(), M, K, K, t[0]->data_ptr(), t[1]->data_ptr(), hb, t[2]->data_ptr(),
+        rc = lib.linear(xc.data_ptr(), M, K, K, t[0]->data_ptr(), t[1]->data_ptr(), (int32_t)hb, t[2]->data_ptr(),
                         t[3]->data_ptr(), b ? b->data_ptr() : nullptr, N, n_cb, y.data_ptr(), stream_of(*x));
     }
     if (rc == kUnsupported) Py_RETURN_NONE;
@@ -148,18 +155,18 @@ PyObject* py_gemv(PyObject*, PyObject* const* a, Py_ssize_t na) {
     SX8_ARGS(9)
     const at::Tensor* x = dense(a[0], at::kHalf);
     const at::Tensor* y = dense(a[8], at::kFloat);
-    const int64_t N = num(a[6]), n_cb = num(a[7]);
+    const int64_t N = num(a[6]), n_cb = num(a[7]), hb = num(a[5]);
+    SX8_SIZES_OK()
     if (!x || !y || n_cb > kLdsMaxKb || x->numel() != n_cb * 32 || y->numel() != N || x->device() != y->device())
         Py_RETURN_NONE;
     if (reinterpret_cast<uintptr_t>(x->data_ptr()) & 15) Py_RETURN_NONE;
     const at::Tensor* t[4];
     for (int i = 0; i < 4; ++i)
         if (!(t[i] = plain(a[1 + i]))) Py_RETURN_NONE;
-    const int32_t hb = (int32_t)num(a[5]);
     int32_t rc;
     {
         Unlocked u;
-        rc = lib.gemv(x->data_ptr(), t[0]->data_ptr(), t[1]->data_ptr(), hb, t[2]->data_ptr(), t[3]->data_ptr(), nullptr,
+        rc = lib.gemv(x->data_ptr(), t[0]->data_ptr(), t[1]->data_ptr(), (int32_t)hb, t[2]->data_ptr(), t[3]->data_ptr(), nullptr,
                       nullptr, N, n_cb, y->data_ptr(), nullptr, 0, stream_of(*x));
     }
     if (rc) return failed("sx8_gemv", rc);
@@ -196,14 +203,14 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t na) {
     for (int i = 0; i < 4; ++i)
         if (!(t[i] = plain(a[1 + i]))) Py_RETURN_NONE;
     GemmCall c;
-    const int64_t in_f = num(a[7]);
-    if (!c.make(a[0], num(a[6]), num(a[8])) || c.K < in_f) Py_RETURN_NONE;
-    const int32_t hb = (int32_t)num(a[5]);
+    const int64_t N = num(a[6]), in_f = num(a[7]), n_cb = num(a[8]), hb = num(a[5]);
+    SX8_SIZES_OK()
+    if (!c.make(a[0], N, n_cb) || c.K < in_f) Py_RETURN_NONE;
     int32_t rc;
     {
         Unlocked u;
         c.allocate();
-        rc = lib.gemm(c.x->data_ptr(), c.M, c.K, in_f, t[0]->data_ptr(), t[1]->data_ptr(), hb, t[2]->data_ptr(),
+        rc = lib.gemm(c.x->data_ptr(), c.M, c.K, in_f, t[0]->data_ptr(), t[1]->data_ptr(), (int32_t)hb, t[2]->data_ptr(),
                       t[3]->data_ptr(), c.N, c.n_cb, c.y.data_ptr(), c.ws.data_ptr(), c.ws_bytes, stream_of(*c.x));
     }
     if (rc) return failed("sx8_gemm_prefill", rc);
@@ -219,6 +226,7 @@ PyObject* py_gemm_split(PyObject*, PyObject* const* a, Py_ssize_t na) {
     for (int i = 0; i < 8; ++i)
         if (!(t[i] = plain(a[1 + i]))) Py_RETURN_NONE;
     const int64_t n_cb = num(a[9]);
+    SX8_SIZES_OK()
     GemmCall c;
     if (n_cb < 1 || !c.make(a[0], t[0]->numel() / n_cb, n_cb)) Py_RETURN_NONE;
     int32_t rc;
@@ -248,6 +256,7 @@ PyObject* py_dequant(PyObject*, PyObject* const* a, Py_ssize_t na) {
     }
     if (t[0]->device().index() != c10::hip::current_device()) Py_RETURN_NONE;
     const int64_t out_f = num(a[8]), in_f = num(a[9]), n_cb = num(a[10]);
+    SX8_SIZES_OK()
     if (t[6]->numel() != n_cb * 64 || t[7]->numel() != n_cb * 2) Py_RETURN_NONE;
     at::Tensor w;
     int32_t rc;
@@ -275,6 +284,7 @@ PyObject* py_embed(PyObject*, PyObject* const* a, Py_ssize_t na) {
     const at::Tensor* b = dense(a[3], at::kFloat);
     const at::Tensor* s = dense(a[4], at::kFloat);
     const int64_t K = num(a[5]), N = num(a[6]), n_cb = num(a[7]);
+    SX8_SIZES_OK()
     if (!ids || !out || !h || !l || !b || !s || out->dim() != 2 || out->size(1) != K || ids->device() != out->device() ||
         ids->numel() < 1 || out->size(0) < ids->numel())
         Py_RETURN_NONE;

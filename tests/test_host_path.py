@@ -69,6 +69,8 @@ def test_host_tensors_are_left_to_the_general_path(hiplib):
     assert py.dequant(*[np.zeros(4)] * 8, 64, 64, 2) is None
     assert py.embed(torch.zeros(1, dtype=torch.long), u, u, f, f, 64, 64, 2, h) is None
     assert py.to_host(u) is None
+    assert py.gemm(h, u, u, f, f, 6, 64, 64.0, 2) is None          # not an integer: no error here either
+    assert py.gemv(h[0], u, u, f, f, 6, 64, None, f) is None
     with pytest.raises(TypeError):
         py.linear(h)
     with pytest.raises(KeyError):
@@ -122,6 +124,9 @@ def test_wrappers(both, cuda, monkeypatch):
         _same(y, ref)
     with pytest.raises(ValueError):
         gemm_sx8_compact(X[:4, :K - 1].contiguous(), qt, bi, *t)
+    y, ref, taken = both(lambda: gemm_sx8_compact(X[:4, :K].contiguous(), qt, bi, *t, in_f=float(K)))
+    _same(y, ref)
+    assert isinstance(y, torch.Tensor) and not taken
     for x in (X[0, :K].contiguous(), X[0, :K - 4], X.reshape(-1)[3:3 + K], X[:1, :K].float(), X[1]):
         y, ref, _ = both(lambda: decode1_v44(x, qt, bi, *t)[0])
         _same(y, ref)
