@@ -71,9 +71,12 @@ def pca_correct(levels, dmin, dmax, config, blocks, n_cb, pca_method="svd"):
     dev = blocks.device
     n_blk = blocks.shape[0]
     n_rows = n_blk // n_cb
-    if pca_method == "gram" and blocks.is_cuda and n_rows >= 4:
+    if n_rows >= 4 and min(dmin.shape[0], dmax.shape[0]) < n_blk:
+        # (the gathers below would read past them, which on a GPU ends the process)
+        raise IndexError(f"dmin / dmax hold fewer than the {n_blk} blocks")
+    if pca_method == "gram" and blocks.is_cuda and n_rows >= 4 and _pca_plain(levels, dmin, dmax, config, blocks, n_cb):
         out = _HostFields(n_blk, n_cb, dev)
-        _pca_hip(levels, dmin.float(), dmax.float(), config, blocks.float(), n_rows, n_cb, out)
+        _pca_hip(levels, dmin, dmax, config, blocks.float(), n_rows, n_cb, out)
         f = out.to_host()
         if f is not None:
             return f["coeff"].reshape(n_blk, 1), f["data"], f["scales"]
@@ -156,6 +159,19 @@ class _HostFields:
         f = {name: host[off:off + nb].view(dt) for name, (off, nb, dt) in self.at.items()}
         f["data"], f["scales"] = f["data"].reshape(self.n_cb, 64), f["scales"].reshape(self.n_cb, 2)
         return f if np.isfinite(f["data"]).all() and np.isfinite(f["scales"]).all() else None
+
+
+def _pca_plain(levels, dmin, dmax, config, blocks, n_cb):
+    """Whether pca_correct's arguments are what sx8_quant_pca reads: plain tensors of one device
+    without gradients, (n_cb n, 32) blocks and one field value (32 uint8 levels) for each.  Other
+    types, devices and shapes are torch's to convert or refuse."""
+    n = blocks.shape[0]
+    t = (levels, dmin, dmax, config, blocks)
+    return (all(type(x) is torch.Tensor and x.device == blocks.device and not x.requires_grad for x in t)
+            and blocks.shape == (n, B) and n % n_cb == 0 and blocks.dtype in (torch.float32, torch.float16)
+            and levels.shape == (n, B) and levels.dtype == torch.uint8
+            and dmin.shape == dmax.shape == config.shape == (n,) and dmin.dtype == dmax.dtype == torch.float32
+            and not config.is_floating_point() and not config.is_complex())
 
 
 def _pca_hip(levels, dmin, dmax, config, blocks, n_rows, n_cb, out):

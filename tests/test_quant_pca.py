@@ -129,3 +129,54 @@ def test_pca_spectra(hiplib, cuda, kind):
     if (lam[-2] - lam[-3]) > 1e-3 * lam[-1]:
         U = vec[:, -2:]
         assert np.abs(v - v @ U @ U.T).max() <= 1e-6
+
+
+def _fields(n_rows, n_cb, device):
+    import torch
+    from quantize_sx8 import v6_encode_6bit
+    blocks = (torch.randn(n_rows * n_cb, 32, generator=torch.Generator().manual_seed(3)) * 0.02).half().float()
+    return [t.to(device) for t in (*v6_encode_6bit(blocks), blocks)]
+
+
+def test_pca_forms_left_to_torch():
+    """The kernels read raw pointers: only the exact types, shapes and one device go there."""
+    import torch
+    from quantize_sx8 import _pca_plain
+    lv, mn, mx, cfg, x = _fields(8, 3, "cpu")
+    assert _pca_plain(lv, mn, mx, cfg, x, 3) and _pca_plain(lv, mn, mx, cfg.to(torch.uint8), x.half(), 3)
+    for bad in ((lv.int(), mn, mx, cfg, x, 3), (lv.float(), mn, mx, cfg, x, 3), (lv.to("meta"), mn, mx, cfg, x, 3),
+                (lv, mn.to("meta"), mx, cfg, x, 3), (lv, mn, mx, cfg.to("meta"), x, 3), (lv, mn.half(), mx.half(), cfg, x, 3),
+                (lv, mn.double(), mx, cfg, x, 3), (lv, mn, mx, cfg.float(), x, 3), (lv, mn, mx, cfg, x.double(), 3),
+                (lv, mn, mx, cfg, x, 5), (lv[:-1], mn, mx, cfg, x, 3), (lv.view(-1, 16), mn, mx, cfg, x, 3),
+                (lv, mn[:-1], mx, cfg, x, 3), (lv, mn, mx, cfg[:-1], x, 3), (lv, mn, mx, cfg, x[:, :16], 3),
+                (lv, mn[:, None], mx, cfg, x, 3), (lv, mn, mx, cfg, x.clone().requires_grad_(), 3)):
+        assert not _pca_plain(*bad)
+
+
+@pytest.mark.gpu
+def test_pca_other_forms(hiplib, cuda):
+    """Levels and fields of other types give what uint8 levels and float32 fields give; host
+    levels, uneven block counts and short fields raise on the host."""
+    import torch
+    from quantize_sx8 import pca_correct
+    n_rows, n_cb = 64, 3
+    lv, mn, mx, cfg, x = _fields(n_rows, n_cb, cuda)
+    want = pca_correct(lv, mn, mx, cfg, x, n_cb, "gram")
+    for f in ((lv.int(), mn, mx, cfg, x), (lv.float(), mn, mx, cfg, x), (lv, mn, mx, cfg.cpu(), x),
+              (lv, torch.cat([mn, mn]), torch.cat([mx, mx]), cfg, x)):
+        got = pca_correct(*f, n_cb, "gram")
+        # the same residuals, float64 Gram matrices on both sides; the coefficients are float32 sums of 32
+        assert np.abs(got[1] - want[1]).max() <= 1e-6 and np.abs(got[2] / want[2] - 1).max() <= 1e-5
+        assert (got[0] != want[0]).mean() <= 1e-2          # coefficients on a rounding tie
+    with pytest.raises(RuntimeError):
+        pca_correct(lv.cpu(), mn, mx, cfg, x, n_cb, "gram")
+    with pytest.raises(RuntimeError):
+        pca_correct(lv, mn.cpu(), mx.cpu(), cfg, x, n_cb, "gram")
+    with pytest.raises(RuntimeError):
+        pca_correct(lv, mn, mx, cfg, x, 5, "gram")
+    with pytest.raises(IndexError):
+        pca_correct(lv, mn[:-1], mx, cfg, x, n_cb, "gram")
+    with pytest.raises((RuntimeError, IndexError)):
+        pca_correct(lv, mn, mx, cfg[:-1], x, n_cb, "gram")
+    with pytest.raises(RuntimeError):
+        pca_correct(lv[:-1], mn, mx, cfg, x, n_cb, "gram")
