@@ -76,8 +76,7 @@ def pca_correct(levels, dmin, dmax, config, blocks, n_cb, pca_method="svd"):
         raise IndexError(f"dmin / dmax hold fewer than the {n_blk} blocks")
     if pca_method == "gram" and blocks.is_cuda and n_rows >= 4 and _pca_plain(levels, dmin, dmax, config, blocks, n_cb):
         out = _HostFields(n_blk, n_cb, dev)
-        _pca_hip(levels, dmin, dmax, config, blocks.float(), n_rows, n_cb, out)
-        f = out.to_host()
+        f = out.to_host() if _pca_hip(levels, dmin, dmax, config, blocks.float(), n_rows, n_cb, out) else None
         if f is not None:
             return f["coeff"].reshape(n_blk, 1), f["data"], f["scales"]
     d = (dmax - dmin).clamp(min=1e-10)
@@ -176,16 +175,22 @@ def _pca_plain(levels, dmin, dmax, config, blocks, n_cb):
 
 def _pca_hip(levels, dmin, dmax, config, blocks, n_rows, n_cb, out):
     """sx8_quant_pca of (n_rows * n_cb, 32) blocks -- all of float32 or all of float16 -- into the
-    fields coeff, data and scales of `out`."""
+    fields coeff, data and scales of `out`.  False, with nothing launched, for a tensor past the
+    kernels' sizes (65535 K blocks): torch's path takes it."""
     import _sx8lib as _L
     f16 = blocks.dtype == torch.float16
     t = [x.contiguous() for x in (blocks, dmin, dmax, levels, config.to(torch.uint8))]
     nb = int(_L.lib().sx8_quant_pca_workspace_bytes(n_rows, n_cb))
     if nb < 0:
-        raise RuntimeError(f"sx8_quant_pca_workspace_bytes: bad shape {n_rows} x {n_cb}")
+        return False
     ws = torch.empty(nb, dtype=torch.uint8, device=blocks.device)
-    _L.call("sx8_quant_pca", _L.ptr(t[0]), _L.ptr(t[1]), _L.ptr(t[2]), int(f16), _L.ptr(t[3]), _L.ptr(t[4]), n_rows,
-            n_cb, out.ptr("coeff"), out.ptr("data"), out.ptr("scales"), _L.ptr(ws), nb, _L.stream(blocks.device))
+    rc = _L.lib().sx8_quant_pca(_L.ptr(t[0]), _L.ptr(t[1]), _L.ptr(t[2]), int(f16), _L.ptr(t[3]), _L.ptr(t[4]), n_rows,
+                                n_cb, out.ptr("coeff"), out.ptr("data"), out.ptr("scales"), _L.ptr(ws), nb,
+                                _L.stream(blocks.device))
+    if rc == _L.ERR_UNSUPPORTED:
+        return False
+    _L.check("sx8_quant_pca", rc)
+    return True
 
 
 def pack_levels_6bit(levels: np.ndarray):
@@ -235,8 +240,7 @@ def quantize_tensor(W, device=None, pca_method=None, degenerate_frac=0.0, seed=N
     if hip and pca_method == "gram" and out_f >= 4:
         out = _HostFields(out_f * n_cb, n_cb, blocks.device)
         lv, dmin16, dmax16, cfg8 = _v6_encode_into(blocks, out)
-        _pca_hip(lv, dmin16, dmax16, cfg8, blocks, out_f, n_cb, out)
-        f = out.to_host()
+        f = out.to_host() if _pca_hip(lv, dmin16, dmax16, cfg8, blocks, out_f, n_cb, out) else None
         if f is not None:
             qt = dict(meta, dmin=f["dmin"], dmax=f["dmax"], config=f["config"], levels_hi=f["levels_hi"],
                       levels_lo=f["levels_lo"], coeff=f["coeff"].reshape(-1, 1))

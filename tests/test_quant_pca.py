@@ -98,6 +98,8 @@ def test_pca_refusals(hiplib):
     assert call(x=N0) == 1 and call(ws=N0) == 1 and call(nb=need - 1) == 1 and call(r=0) == 1
     assert call(x=ctypes.c_void_p(4097)) == 1 and call(ws=ctypes.c_void_p(4104)) == 1
     assert b"misaligned" in L.sx8_last_error()
+    big = L.sx8_quant_pca_workspace_bytes(4, 65536)               # one K block past the kernels' grids
+    assert L.sx8_quant_pca(p, p, p, 1, p, p, 4, 65536, p, p, p, p, big, N0) == 3
 
 
 @pytest.mark.gpu
@@ -180,3 +182,27 @@ def test_pca_other_forms(hiplib, cuda):
         pca_correct(lv, mn, mx, cfg[:-1], x, n_cb, "gram")
     with pytest.raises(RuntimeError):
         pca_correct(lv[:-1], mn, mx, cfg, x, n_cb, "gram")
+
+
+@pytest.mark.gpu
+def test_pca_past_the_kernels_sizes(hiplib, cuda, monkeypatch):
+    """Where sx8_quant_pca reports a tensor too large, both callers take torch's path."""
+    import torch
+    import _sx8lib
+    from quantize_sx8 import pca_correct, quantize_tensor
+    W = (torch.randn(64, 96, generator=torch.Generator().manual_seed(2)) * 0.02).half().to(cuda)
+    qt, bi = quantize_tensor(W)
+    f = _fields(64, 3, cuda)
+    want = pca_correct(*f, 3, "gram")
+
+    class Small:
+        def __getattr__(self, name):
+            return (lambda *a: _sx8lib.ERR_UNSUPPORTED) if name == "sx8_quant_pca" else getattr(hiplib, name)
+    monkeypatch.setattr(_sx8lib, "_lib", Small())
+    q2, b2 = quantize_tensor(W)
+    got = pca_correct(*f, 3, "gram")
+    for k in ("dmin", "dmax", "config", "levels_hi", "levels_lo"):
+        assert np.array_equal(qt[k], q2[k])
+    for a, b in ((bi["data"], b2["data"]), (want[1], got[1])):
+        assert np.abs(a - b).max() <= 1e-6
+    assert (qt["coeff"] != q2["coeff"]).mean() <= 1e-2 and (want[0] != got[0]).mean() <= 1e-2
