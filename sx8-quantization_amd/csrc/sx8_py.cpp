@@ -45,8 +45,16 @@ struct Lib {
 constexpr int32_t kUnsupported = 3;
 constexpr int64_t kLinearRows = 32, kLdsMaxKb = 640;
 
-// A plain tensor (or Parameter), else null: subclasses go through the general path.
-const at::Tensor* plain(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+// A plain tensor (or Parameter) whose memory holds its values, else null: subclasses, the wrappers of
+// function transforms (vmap, jvp) and views that negate on reading go through the general path.
+const at::Tensor* plain(PyObject* o) {
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    using K = c10::DispatchKey;
+    const at::Tensor& x = THPVariable_Unpack(o);
+    const c10::DispatchKeySet other({K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched, K::Functionalize, K::Python,
+                                     K::Conjugate, K::Negative, K::ZeroTensor});
+    return x.key_set().has_any(other) ? nullptr : &x;
+}
 
 const at::Tensor* dev(PyObject* o, at::ScalarType t) {
     const at::Tensor* x = plain(o);
@@ -128,8 +136,9 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t na) {
     const at::Tensor* b = nullptr;
     if (a[3] != Py_None) {
         b = dense(a[3], at::kHalf);
+        // (a bias that either mode of autograd follows is added by torch)
         if (!b || b->device() != x->device() || b->dim() != 1 || b->size(0) != N ||
-            (b->requires_grad() && c10::GradMode::is_enabled()))
+            (b->requires_grad() && c10::GradMode::is_enabled()) || b->_fw_grad(0).defined())
             Py_RETURN_NONE;
     }
     c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());

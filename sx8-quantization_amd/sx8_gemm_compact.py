@@ -112,14 +112,23 @@ def gemm_sx8_compact(X, qt, bases_info, hdr_t=None, lvl_t=None, bas_t=None, sca_
 LINEAR_ROWS = 32
 
 
+def _fusable_bias(bias, out_f, device):
+    """Whether the kernel can add this bias as torch's `y + bias` would: a plain contiguous fp16
+    (out_f,) tensor on the device whose memory holds its values, with no gradient of either mode
+    to follow and no function transform around it."""
+    return (type(bias) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(bias)
+            and bias.dtype == torch.float16 and bias.device == device and bias.shape == (out_f,)
+            and bias.is_contiguous() and not bias.is_neg() and not (bias.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad.unpack_dual(bias).tangent is None)
+
+
 def linear_sx8(X, qt, hdr_t, lvl_t, bas_t, sca_t, hdr_bytes=6, bias=None):
     """fp16(X @ W^T) (+ bias) for up to LINEAR_ROWS rows X (M, K) CUDA in one launch
     (sx8_linear_f16; no counterpart upstream, whose module runs the GEMM, .half() and the bias
-    add).  None when the call is not one it takes: a bias that is not a contiguous fp16 (N,)
-    tensor on X's device or that autograd tracks, or operands past 2 GiB."""
+    add).  None when the call is not one it takes: a bias that only torch can add (see
+    _fusable_bias), or operands past 2 GiB."""
     out_f, in_f = qt["shape"]
-    if bias is not None and (bias.dtype != torch.float16 or bias.device != X.device or bias.shape != (out_f,)
-                             or not bias.is_contiguous() or (bias.requires_grad and torch.is_grad_enabled())):
+    if bias is not None and not _fusable_bias(bias, out_f, X.device):
         return None
     Xc = _x2d(X)
     M, K = Xc.shape

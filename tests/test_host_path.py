@@ -184,3 +184,59 @@ def test_to_host(hiplib, cuda, n):
         assert (y is None) == (n <= 1 << 20)
         assert y is None or (not y.is_cuda and torch.equal(y, x.cpu()))
         x.bitwise_not_()
+
+
+def test_bias_left_to_torch():
+    """Only a bias whose sum is the kernel's fp16 addition is fused."""
+    import torch.autograd.forward_ad as fwd
+    from sx8_gemm_compact import _fusable_bias
+
+    class Sub(torch.Tensor):
+        pass
+    cpu = torch.device("cpu")
+    b = torch.randn(8).half()
+    assert _fusable_bias(b, 8, cpu) and _fusable_bias(torch.nn.Parameter(b, requires_grad=False), 8, cpu)
+    for bad in (b.float(), b[::2], b[:4], b[None], torch.nn.Parameter(b), b.as_subclass(Sub), torch._neg_view(b), 1.0,
+                b.to("meta")):
+        assert not _fusable_bias(bad, 8, cpu)
+    with torch.no_grad():
+        assert _fusable_bias(torch.nn.Parameter(b), 8, cpu)
+    seen = []
+    with fwd.dual_level():
+        assert not _fusable_bias(fwd.make_dual(b, b), 8, cpu) and _fusable_bias(b, 8, cpu)
+    torch.func.vmap(lambda v: (seen.append(_fusable_bias(v, 8, cpu)), v)[1])(b.expand(2, 8).contiguous())
+    torch.func.jvp(lambda v: (seen.append(_fusable_bias(v, 8, cpu)), v)[1], (b,), (b,))
+    assert seen == [False, False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 4])
+def test_bias_transforms(hiplib, cuda, M):
+    """Tangents, vmap, subclasses and negating views of the bias reach torch's sum."""
+    import torch.autograd.forward_ad as fwd
+    from integrate_fused_v44 import SX8LinearV44
+    from sx8_decode1_v3 import make_tensors_v44
+
+    class Sub(torch.Tensor):
+        pass
+    N, K = 96, 100
+    qt, bi = _weight(N, K)
+    t = make_tensors_v44(qt, bi)
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(M, K, generator=g).half().to(cuda)
+    b, db = (torch.randn(N, generator=g).half().to(cuda) for _ in range(2))
+
+    def f(bias, x=x):
+        m = SX8LinearV44(qt, bi, bias)
+        m._t44 = t
+        return m(x)
+    y = f(b)
+    for form in (x, x.t().contiguous().t(), x.float()):          # native path, copied rows, general path
+        with fwd.dual_level():
+            d = fwd.unpack_dual(f(fwd.make_dual(b, db), form))
+            assert torch.equal(d.tangent, db.expand(M, N)) and torch.allclose(d.primal, y, atol=1e-2)
+        out = torch.func.vmap(lambda v: f(v, form))(torch.stack([b, db]))
+        assert out.shape == (2, M, N) and torch.allclose(out[0], y, atol=1e-2)
+        assert type(f(b.as_subclass(Sub), form)) is Sub
+        assert torch.allclose(f(torch._neg_view(b), form), f(-b, form), atol=1e-2)
+        assert torch.allclose(f(0.5, form), f(torch.full_like(b, 0.5), form), atol=1e-2)
