@@ -171,11 +171,12 @@ int64_t sx8_gemv_workspace_bytes(int64_t n_cb);
 
 /* A linear layer on up to 32 rows in one launch: Y (M, N) fp16 = fp16(X . W^T), plus bias (N)
  * fp16 as an fp16 sum when bias is not NULL.  X (M, K) fp16 with row stride ldx >= K; K and ldx
- * may be odd, the tail of the last K block counts as zero.  Z is computed inside (its bases
- * split into two fp16 parts, about 22 bits), the core weights are those of sx8_gemm_prefill;
- * one row runs sx8_gemv's arithmetic (float32 weights; at most 640 K blocks).  No workspace.  SX8_ERR_UNSUPPORTED past 32 rows or 2 GiB operands.  Replaces
- * gemm_compact's call plus the .half() and the bias add of SX8LinearV44.forward
- * (scripts/integrate_fused_v44.py:43-77). */
+ * may be odd, the tail of the last K block counts as zero.  Z is computed inside (each basis
+ * vector in two fp16 parts, 22 bits of its largest element, scaled by a power of two where that
+ * is not in [2^-3, 2^15)), the core weights are those of sx8_gemm_prefill; one row runs sx8_gemv's arithmetic
+ * (float32 weights; at most 640 K blocks).  No workspace.  SX8_ERR_UNSUPPORTED past 32 rows or
+ * 2 GiB operands.  Replaces gemm_compact's call plus the .half() and the bias add of
+ * SX8LinearV44.forward (scripts/integrate_fused_v44.py:43-77). */
 int32_t sx8_linear_f16(const uint16_t* X, int64_t M, int64_t ldx, int64_t K, const uint8_t* hdr,
                        const uint8_t* levels, int32_t hdr_bytes, const float* basis,
                        const float* scales, const uint16_t* bias, int64_t N, int64_t n_cb,

@@ -25,8 +25,8 @@
 //     in flight per wave, and meet once in LDS (fixed order: deterministic).
 // Two forms of input: the packed operands of the prefill GEMM (packed X + Zhl, written by the
 // pack pass or by a producer kernel), or plain fp16 rows (kRaw), for which Z is computed on
-// the matrix core too: the block's two basis vectors, split into fp16 hi + lo (about 22 bits),
-// are four rows of an A operand, so the product with the block's X lands, for every row of X,
+// the matrix core too: the block's two basis vectors, split into fp16 hi + lo (22 bits of the
+// largest element), are four rows of an A operand, so the product with the block's X lands, for every row of X,
 // in the lane that feeds it to the PCA MFMA.
 // Measured (kernel alone, packed, against k_gemm + k_reduce): 9728 x 2560 at 8 rows 9.9 against
 // 17.7 us, 2560 x 9728 at 16 rows 11.6 against 22.5, 4096 x 2560 at 16 / 64 / 128 rows 5.6 / 9.1 /
@@ -178,6 +178,22 @@ __device__ __forceinline__ int xcd_order_small(int b, int G) {
 
 constexpr uint32_t kOob = 0x80000000u;     // past every buffer (all below 2 GiB): reads zero
 
+// v of lane 4 g + k of this lane's 16-lane row g (row_newbcast, one row at a time)
+template <int k>
+__device__ __forceinline__ uint32_t from_own_block(uint32_t v) {
+    int r = __builtin_amdgcn_update_dpp(0, (int)v, 0x150 + k, 0x1, 0xF, false);
+    r = __builtin_amdgcn_update_dpp(r, (int)v, 0x154 + k, 0x2, 0xF, false);
+    r = __builtin_amdgcn_update_dpp(r, (int)v, 0x158 + k, 0x4, 0xF, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp(r, (int)v, 0x15C + k, 0x8, 0xF, false);
+}
+
+// max(|a|, |b|, |c|), NaN left out
+__device__ __forceinline__ float abs_max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 constexpr int kMaxWaves = 8;
 
 // Work-group: 64 S threads (S waves); 16 CF columns, 16 MT rows (row block mb = blockIdx / NB).
@@ -289,6 +305,42 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
         }
     };
 
+    // Two fp16 parts hold 22 bits of a basis vector's largest element while that lies in [2^-3,
+    // 2^15); unit vectors of 32 do (2^-2.5 at least).  z_far: the group in z4 has a vector outside
+    // (uniform).  z_scale: each vector times a power of two that puts its largest element in [2^14,
+    // 2^15), undone in its scale.  Scaling every group costs ~45 instructions, 2560 x 9728 at 2 rows
+    // 14.0 -> 15.6 us; the test after the wait for z4 14.5, with the record arithmetic ahead of it to
+    // hide its chain 14.1 (1024 x 2560 at 2 / 32 rows 5.58 / 9.10 -> 5.68 / 9.08).
+    auto b_max = [&]() __attribute__((always_inline)) {
+        float b[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) b[i] = __builtin_bit_cast(float, (uint32_t)z4[kRaw ? i >> 2 : 0][i & 3]);
+        return abs_max3(abs_max3(b[0], b[1], b[2]), abs_max3(b[3], b[4], b[5]), abs_max3(b[6], b[7], 0.f));
+    };
+    auto z_far = [&]() __attribute__((always_inline)) {
+        const float mx = b_max();
+        unsigned long long reach = __ballot(mx >= 0.125f);
+        reach |= reach >> 32;
+        reach |= reach >> 16;
+        return (reach & 0xFFFF) != 0xFFFF || __ballot(mx >= 32768.f) != 0;
+    };
+    auto z_scale = [&]() __attribute__((always_inline)) {
+        uint32_t a = __builtin_bit_cast(uint32_t, b_max()), b = a;      // (non-negative: ordered as integers)
+        sx8_swap32(a, b);
+        a = b = max(a, b);
+        sx8_swap16(a, b);
+        const uint32_t ex = min(max(max(a, b) >> 23, 15u), 254u);
+        const float down = __builtin_bit_cast(float, (268u - ex) << 23);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            uint32_t w = z4[kRaw ? i >> 2 : 0][i & 3];
+            z4[kRaw ? i >> 2 : 0][i & 3] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, w) * down);
+        }
+        // this lane's scales are of its own block g: lanes 4 g and 4 g + 1 hold its vectors' exponents
+        sc.x *= __builtin_bit_cast(float, (from_own_block<0>(ex) - 14u) << 23);
+        sc.y *= __builtin_bit_cast(float, (from_own_block<1>(ex) - 14u) << 23);
+    };
+
     sx8_float4 acc[CF][MT];
 #pragma unroll
     for (int cf = 0; cf < CF; ++cf)
@@ -307,6 +359,12 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
     asm volatile("" ::: "memory");
 
     auto step = [&](Rec (&r)[CF]) __attribute__((always_inline)) {
+        Frag fr[CF];
+        if constexpr (kRaw) {
+#pragma unroll
+            for (int cf = 0; cf < CF; ++cf) frag_prep<kSplit, kRaw>(fr[cf], r[cf]);
+            if (z_far()) z_scale();
+        }
         // values past K (raw) or blocks past n_cb (packed) count as zero
         const int kb0 = 4 * gi;
         const bool last = kb0 * 32 + 128 > (kRaw ? K : n_cb * 32);
@@ -363,10 +421,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
             for (int mt = 0; mt < MT; ++mt) zop[mt] = u32x4{zp[mt].x, zp[mt].y, 0u, 0u};
         }
         load_z();
-        Frag fr[CF];
 #pragma unroll
         for (int cf = 0; cf < CF; ++cf) {
-            frag_prep<kSplit, kRaw>(fr[cf], r[cf]);
+            if constexpr (!kRaw) frag_prep<kSplit, kRaw>(fr[cf], r[cf]);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
                 acc[cf][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(sx8_half8, fr[cf].coef),

@@ -70,6 +70,58 @@ def test_linear_f16(hiplib, oracle, cuda, M, N, K, hb, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [2, 17, 32])
+def test_linear_f16_basis_range(hiplib, cuda, M):
+    """Bases of any length with their scales the other way: Z keeps its 22 bits, and powers of two
+    past the unscaled range change no bit between them (nothing is rounded where both are undone)."""
+    import torch
+    from sx8_decode1_v3 import make_tensors_v44
+    from sx8_gemm_compact import linear_sx8
+    print("basis range", M, flush=True)
+    N, K = 130, 640 + 35
+    qt, bi = _quantized(N, K, M, cuda)
+    hdr, lv, bas, sca = make_tensors_v44(qt, bi)
+    sca = sca * 64                                    # a PCA part as large as the core weights'
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half().to(cuda)
+    want = linear_sx8(X, qt, hdr, lv, bas, sca)
+    assert want.isfinite().all() and (want - linear_sx8(X, qt, hdr, lv, bas * 0, sca)).abs().max() > 0.1
+    def scaled(f0, f1):
+        f = torch.tensor([f0, f1], dtype=torch.float64, device=cuda)
+        b = (bas.view(-1, 2, 32).double() * f[:, None]).float().view(-1, 64).contiguous()
+        return linear_sx8(X, qt, hdr, lv, b, (sca.double() / f).float().contiguous())
+    # the PCA part, about as large as Y, to 2^-22 and two float32 factors, and one fp16 rounding of
+    # the output that may fall either way
+    near = lambda y: ((y - want).abs() <= 2.0 ** -10 * want.abs() + 4e-6 * want.abs().max()).all()
+    small = scaled(2.0 ** -12, 2.0 ** -12)
+    assert near(small)
+    for e0, e1 in ((17, 17), (-40, 30), (60, -60), (-100, 0)):
+        assert torch.equal(scaled(2.0 ** e0, 2.0 ** e1), small), (e0, e1)
+    for f in (1e-3, 3e-5, 0.2, 300.0, 7e4):
+        assert near(scaled(f, f)), f
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [4, 32])
+def test_linear_f16_not_finite(hiplib, cuda, M):
+    """Infinities and NaN of X stay in their rows, which are NaN as the tiled kernels give them
+    (Z's second fp16 part of an infinity is NaN)."""
+    import torch
+    from sx8_decode1_v3 import make_tensors_v44
+    from sx8_gemm_compact import gemm_sx8_compact, linear_sx8
+    print("not finite", M, flush=True)
+    N, K = 200, 515
+    qt, bi = _quantized(N, K, M, cuda)
+    t = make_tensors_v44(qt, bi)
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half().to(cuda)
+    want = linear_sx8(X, qt, *t)
+    X[1, 70], X[M - 1, K - 1] = float("inf"), float("nan")
+    got = linear_sx8(X, qt, *t)
+    rows = [i for i in range(M) if i not in (1, M - 1)]
+    assert torch.equal(got[rows], want[rows]) and got[[1, M - 1]].isnan().all()
+    assert torch.equal(got.isnan(), gemm_sx8_compact(X, qt, bi, *t).isnan())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,K,hb,bias", [
     (1024, 2560, 6, False), (2560, 9728, 8, True), (33, 31, 6, True), (300, 97, 8, False), (777, 1333, 6, True),
     (4097, 4095, 8, True), (129, 4098, 6, False), (100, 16390, 6, True), (70001, 64, 6, True),
