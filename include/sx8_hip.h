@@ -40,8 +40,10 @@ extern "C" {
  * 4: deferred split-K sums: sx8_gemm_prefill_group_deferred, sx8_dec_gemm_silu_deferred and
  *    the consumers sx8_dec_add_rmsnorm_parts, sx8_dec_qk_rope_cache_rows_parts
  * 5: producer-written GEMM operands: sx8_gemm_prefill_packed(_workspace_bytes),
- *    sx8_dec_attn_prefill_packed, sx8_dec_gemm_gateup_silu(_workspace_bytes) */
-#define SX8_ABI_VERSION 5
+ *    sx8_dec_attn_prefill_packed, sx8_dec_gemm_gateup_silu(_workspace_bytes)
+ * 6: sx8_linear_f16, sx8_quant_pca(_workspace_bytes); sx8_dec_attn_workspace_bytes returns the
+ *    bytes of 64 chunks (the entry points still run with those of 16) */
+#define SX8_ABI_VERSION 6
 
 #define SX8_OK 0
 #define SX8_ERR_INVALID 1      /* bad argument (null pointer, size, hdr_bytes, alignment) */

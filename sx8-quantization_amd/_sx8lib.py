@@ -115,7 +115,7 @@ SIGNATURES = [
                                          _P, _P, _P, _P]),
     ("sx8_dec_gemv_zp_add", _I32, [_P, _P, _P, _I32, _P, _P, _I64, _I64, _P, _P, _P]),
 ]
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 _lib = None
 _py = None
@@ -208,12 +208,14 @@ def lib():
             if len(runtimes) > 1:
                 raise RuntimeError("two HIP runtimes are loaded in this process: "
                                    + ", ".join(runtimes))
+            # (before the entry points: a library of another version need not have them all)
+            L.sx8_abi_version.restype, L.sx8_abi_version.argtypes = _I32, []
+            if L.sx8_abi_version() != ABI_VERSION:
+                raise RuntimeError(f"{path}: ABI version {L.sx8_abi_version()} != {ABI_VERSION}")
             for name, res, args in SIGNATURES:
                 fn = getattr(L, name)
                 fn.restype = res
                 fn.argtypes = args
-            if L.sx8_abi_version() != ABI_VERSION:
-                raise RuntimeError(f"{path}: ABI version {L.sx8_abi_version()} != {ABI_VERSION}")
             _lib = L
     return _lib
 

@@ -31,6 +31,19 @@ def test_library_exports_every_declared_symbol(hiplib):
     assert hiplib.sx8_abi_version() == _sx8lib.ABI_VERSION
 
 
+def test_library_of_another_version_is_named(tmp_path, monkeypatch):
+    """A library of an older ABI, which lacks newer entry points, is refused by its version."""
+    import subprocess
+    import _sx8lib
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int sx8_abi_version(void) { return 5; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setattr(_sx8lib, "_lib", None)
+    monkeypatch.setenv("SX8_HIP_LIB", str(so))
+    with pytest.raises(RuntimeError, match=r"ABI version 5 != \d+"):
+        _sx8lib.lib()
+
+
 NULL = ctypes.c_void_p(None)
 
 
