@@ -3,7 +3,8 @@
 The library is built in-tree (``build()`` drives hipcc) and loaded from this
 directory, or from the path in the SX8_HIP_LIB environment variable.  There is no
 fallback: if the library cannot be loaded, every GPU entry point raises
-RuntimeError.  The C signatures are declared in include/sx8_hip.h.
+RuntimeError.  The C signatures are declared in include/sx8_hip.h.  The host module (``py()``)
+only shortens the way to the library.
 """
 from __future__ import annotations
 
@@ -11,6 +12,7 @@ import ctypes
 import os
 import subprocess
 import threading
+import warnings
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
@@ -124,7 +126,9 @@ _lock = threading.Lock()
 
 def build(verbose: bool = False) -> str:
     """Compile every HIP source for gfx950 with hipcc (one object per source, in parallel)
-    and link LIB_PATH, and compile the host module PY_PATH with g++ (always rebuilds)."""
+    and link LIB_PATH, and compile the host module PY_PATH with g++ (always rebuilds).  Where the
+    host module does not compile (no Python or torch headers), a warning says so and none is
+    left: the wrappers run without it."""
     from concurrent.futures import ThreadPoolExecutor
     import tempfile
     with tempfile.TemporaryDirectory(prefix="sx8_build_") as d:
@@ -138,9 +142,7 @@ def build(verbose: bool = False) -> str:
         with ThreadPoolExecutor(jobs) as ex:
             py = ex.submit(_build_py)
             results = list(ex.map(compile_one, SOURCES))
-            res = py.result()
-        if res.returncode != 0:
-            raise RuntimeError(f"{PY_SOURCE}: the compiler failed:\n" + res.stdout + res.stderr)
+            res_py = py.result()
         errs = [r.stdout + r.stderr for _, r in results if r.returncode != 0]
         if errs:
             raise RuntimeError("hipcc failed:\n" + "\n".join(errs))
@@ -153,7 +155,14 @@ def build(verbose: bool = False) -> str:
         if res.returncode != 0:
             raise RuntimeError("hipcc link failed:\n" + res.stdout + res.stderr)
     os.replace(tmp, LIB_PATH)
-    os.replace(PY_PATH + ".tmp", PY_PATH)
+    if res_py.returncode == 0:
+        os.replace(PY_PATH + ".tmp", PY_PATH)
+    else:
+        for f in (PY_PATH, PY_PATH + ".tmp"):
+            if os.path.exists(f):
+                os.remove(f)
+        warnings.warn(f"{PY_SOURCE}: the compiler failed, the wrappers run without it:\n{res_py.stdout}{res_py.stderr}",
+                      RuntimeWarning, stacklevel=2)
     return LIB_PATH
 
 
@@ -167,10 +176,13 @@ def _build_py():
     libs = os.path.join(T, "lib")
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(a for i in inc for a in ("-isystem", i)),
-           os.path.join(CSRC_DIR, PY_SOURCE), "-o", PY_PATH + ".tmp", "-L", libs, "-ltorch", "-ltorch_cpu",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DSX8_TORCH="{torch.__version__}"',
+           *(a for i in inc for a in ("-isystem", i)), "-I", INCLUDE_DIR, os.path.join(CSRC_DIR, PY_SOURCE), "-o", PY_PATH + ".tmp", "-L", libs, "-ltorch", "-ltorch_cpu",
            "-ltorch_python", "-lc10", "-lc10_hip", "-Wl,-rpath," + libs]
-    return subprocess.run(cmd, capture_output=True, text=True)
+    try:
+        return subprocess.run(cmd, capture_output=True, text=True)
+    except OSError as e:                             # no such compiler
+        return subprocess.CompletedProcess(cmd, 1, "", str(e))
 
 
 def lib_path() -> str:
@@ -220,23 +232,45 @@ def lib():
     return _lib
 
 
+class _NoHostModule:
+    """In place of a host module that cannot be loaded: takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def _load_py(L):
+    """The host module bound to L, or the reason why there is none."""
+    import importlib.util
+    import torch
+    if not os.path.exists(PY_PATH):
+        return f"not found at {PY_PATH}; __graft_entry__.build() compiles it"
+    try:
+        spec = importlib.util.spec_from_file_location("_sx8py", PY_PATH)
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        if m.torch_version != torch.__version__:
+            return f"{PY_PATH} was built for torch {m.torch_version}, this is {torch.__version__}"
+        m.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name, _, _ in SIGNATURES})
+        return m
+    except (ImportError, AttributeError, KeyError, RuntimeError) as e:   # another interpreter, torch or library
+        return f"{PY_PATH}: {e}"
+
+
 def py():
-    """The host module of sx8_py.cpp, bound to the library that lib() loaded; RuntimeError if
-    it is missing."""
+    """The host module of sx8_py.cpp, bound to the library that lib() loaded.  Without one that
+    fits this interpreter, torch and library, a warning says so once and every wrapper takes its
+    general path (the same kernels, 5-10 us more of Python a call)."""
     global _py
     if _py is not None:
         return _py
     L = lib()
     with _lock:
         if _py is None:
-            import importlib.util
-            if not os.path.exists(PY_PATH):
-                raise RuntimeError(f"S-X8 host module not found at {PY_PATH}; run "
-                                   "__graft_entry__.build() (or _sx8lib.build()) first")
-            spec = importlib.util.spec_from_file_location("_sx8py", PY_PATH)
-            m = importlib.util.module_from_spec(spec)
-            spec.loader.exec_module(m)
-            m.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name, _, _ in SIGNATURES})
+            m = _load_py(L)
+            if isinstance(m, str):
+                warnings.warn("S-X8 host module not used: " + m, RuntimeWarning, stacklevel=3)
+                m = _NoHostModule()
             _py = m
     return _py
 

@@ -26,10 +26,13 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "sx8_hip.h"
+
 namespace {
 
 typedef const void* CP;
 struct Lib {
+    int32_t (*abi_version)();
     const char* (*last_error)();
     int32_t (*linear)(CP, int64_t, int64_t, int64_t, CP, CP, int32_t, CP, CP, CP, int64_t, int64_t, void*, void*);
     int32_t (*gemv)(CP, CP, CP, int32_t, CP, CP, CP, void*, int64_t, int64_t, void*, void*, int64_t, void*);
@@ -42,7 +45,7 @@ struct Lib {
     int32_t (*embed)(CP, int64_t, CP, CP, int32_t, CP, CP, int64_t, int64_t, int64_t, void*, void*);
 } lib;
 
-constexpr int32_t kUnsupported = 3;
+constexpr int32_t kUnsupported = SX8_ERR_UNSUPPORTED;
 constexpr int64_t kLinearRows = 32, kLdsMaxKb = 640;
 
 // A plain tensor (or Parameter) whose memory holds its values, else null: subclasses, the wrappers of
@@ -94,7 +97,7 @@ at::Tensor empty_like_device(at::IntArrayRef sizes, at::ScalarType t, const at::
         return nullptr;                                                            \
     }
 
-// bind({name: address})
+// bind({name: address}): RuntimeError for a library of another ABI version.
 PyObject* py_bind(PyObject*, PyObject* d) {
     auto get = [&](const char* name) -> void* {
         PyObject* v = PyDict_GetItemString(d, name);
@@ -103,6 +106,12 @@ PyObject* py_bind(PyObject*, PyObject* d) {
     };
 #define SX8_BIND(field, name) \
     if (!(lib.field = reinterpret_cast<decltype(lib.field)>(get(name)))) return nullptr;
+    SX8_BIND(abi_version, "sx8_abi_version")
+    if (lib.abi_version() != SX8_ABI_VERSION) {
+        PyErr_Format(PyExc_RuntimeError, "built for ABI version %d, the library has %d", SX8_ABI_VERSION,
+                     (int)lib.abi_version());
+        return nullptr;
+    }
     SX8_BIND(last_error, "sx8_last_error")
     SX8_BIND(linear, "sx8_linear_f16")
     SX8_BIND(gemv, "sx8_gemv")
@@ -377,4 +386,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_sx8py", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__sx8py() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__sx8py() {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", SX8_TORCH) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

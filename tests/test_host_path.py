@@ -1,5 +1,7 @@
 """The native per-call path of the wrappers (sx8_py.cpp) against their general path: the same
 bits, shapes and types for every form of input, whichever of the two takes it."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -75,6 +77,7 @@ def test_host_tensors_are_left_to_the_general_path(hiplib):
         py.linear(h)
     with pytest.raises(KeyError):
         py.bind({})
+    py.bind({n: ctypes.cast(getattr(hiplib, n), ctypes.c_void_p).value for n, _, _ in _sx8lib.SIGNATURES})
 
 
 @pytest.mark.gpu
@@ -184,6 +187,26 @@ def test_to_host(hiplib, cuda, n):
         assert (y is None) == (n <= 1 << 20)
         assert y is None or (not y.is_cuda and torch.equal(y, x.cpu()))
         x.bitwise_not_()
+
+
+def test_without_a_host_module(hiplib, monkeypatch, tmp_path):
+    """Missing, built for something else or for another library: one warning, no call taken."""
+    import _sx8lib
+    real = _sx8lib.py()
+    assert real.torch_version == torch.__version__ and not isinstance(real, _sx8lib._NoHostModule)
+    for path, why in ((tmp_path / "none.so", "not found"), (tmp_path / "bad.so", "bad.so")):
+        if why == "bad.so":
+            path.write_bytes(b"not a module")
+        monkeypatch.setattr(_sx8lib, "PY_PATH", str(path))
+        monkeypatch.setattr(_sx8lib, "_py", None)
+        with pytest.warns(RuntimeWarning, match=why):
+            m = _sx8lib.py()
+        assert m is _sx8lib.py() and m.linear(1, 2) is None and m.to_host(None) is None
+    old = ctypes.CFUNCTYPE(ctypes.c_int32)(lambda: _sx8lib.ABI_VERSION - 1)
+    names = {n: ctypes.cast(getattr(hiplib, n), ctypes.c_void_p).value for n, _, _ in _sx8lib.SIGNATURES}
+    with pytest.raises(RuntimeError, match="ABI version"):
+        real.bind(dict(names, sx8_abi_version=ctypes.cast(old, ctypes.c_void_p).value))
+    real.bind(names)
 
 
 def test_bias_left_to_torch():
