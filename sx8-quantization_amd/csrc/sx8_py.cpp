@@ -134,7 +134,8 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t na) {
     const int64_t out_f = num(a[4]), N = num(a[5]), K = num(a[6]), n_cb = num(a[7]), hb = num(a[2]);
     SX8_SIZES_OK()
     const int64_t M = K > 0 && x->size(-1) == K ? x->numel() / K : 0;
-    if (M < 1 || M > kLinearRows || out_f != N) Py_RETURN_NONE;
+    // (K blocks that are not the row's: decode1_v44 cuts or pads the row, the GEMM refuses)
+    if (M < 1 || M > kLinearRows || out_f != N || n_cb != (K + 31) / 32) Py_RETURN_NONE;
     if (M > 1) {
         const char* wmma = std::getenv("SX8_USE_WMMA");
         if (N < 64 || (wmma && std::strcmp(wmma, "1") == 0)) Py_RETURN_NONE;

@@ -126,8 +126,10 @@ def linear_sx8(X, qt, hdr_t, lvl_t, bas_t, sca_t, hdr_bytes=6, bias=None):
     """fp16(X @ W^T) (+ bias) for up to LINEAR_ROWS rows X (M, K) CUDA in one launch
     (sx8_linear_f16; no counterpart upstream, whose module runs the GEMM, .half() and the bias
     add).  None when the call is not one it takes: a bias that only torch can add (see
-    _fusable_bias), or operands past 2 GiB."""
+    _fusable_bias), an n_cb that is not in_f's, or operands past 2 GiB."""
     out_f, in_f = qt["shape"]
+    if qt["n_cb"] != (in_f + 31) // 32:      # decode1_v44 cuts or pads the row, the GEMM refuses
+        return None
     if bias is not None and not _fusable_bias(bias, out_f, X.device):
         return None
     Xc = _x2d(X)

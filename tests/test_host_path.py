@@ -263,3 +263,22 @@ def test_bias_transforms(hiplib, cuda, M):
         assert type(f(b.as_subclass(Sub), form)) is Sub
         assert torch.allclose(f(torch._neg_view(b), form), f(-b, form), atol=1e-2)
         assert torch.allclose(f(0.5, form), f(torch.full_like(b, 0.5), form), atol=1e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [40, 100])
+def test_k_blocks_of_another_length(both, cuda, K):
+    """A weight of three K blocks used with shorter or longer rows: one row is padded or cut as
+    decode1_v44 does it, more rows are refused."""
+    from integrate_fused_v44 import SX8LinearV44
+    from sx8_decode1_v3 import decode1_v44, make_tensors_v44
+    qt, bi = _weight(80, 96)
+    t = make_tensors_v44(qt, bi)
+    m = SX8LinearV44(dict(qt, shape=(80, K)), bi)
+    m._t44 = t
+    x = torch.randn(4, K, generator=torch.Generator().manual_seed(K)).half().to(cuda)
+    y, ref, taken = both(lambda: m(x[:1]))
+    _same(y, ref)
+    assert "linear" not in taken and torch.equal(y[0], decode1_v44(x[0], qt, bi, *t)[0].half())
+    with pytest.raises(RuntimeError, match="bad shape"):
+        m(x)
