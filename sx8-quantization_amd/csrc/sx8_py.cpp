@@ -54,7 +54,7 @@ const at::Tensor* plain(PyObject* o) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     using K = c10::DispatchKey;
     const at::Tensor& x = THPVariable_Unpack(o);
-    const c10::DispatchKeySet other({K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched, K::Functionalize, K::Python,
+    static const c10::DispatchKeySet other({K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched, K::Functionalize, K::Python,
                                      K::Conjugate, K::Negative, K::ZeroTensor});
     return x.key_set().has_any(other) ? nullptr : &x;
 }
@@ -332,22 +332,44 @@ struct Event {
 
 void hip_ok(hipError_t e) { TORCH_CHECK(e == hipSuccess, "copy to the host: ", hipGetErrorString(e)); }
 
-// to_host(x): a host copy of a dense device tensor of bytes, through two pinned pieces of 1 MB
-// (torch's caching host allocator): the GPU fills one while the host empties the other.  10 MB
-// take 0.39 ms, 3 MB 0.14; the runtime's own copy to pageable memory 0.55 and 0.17 (up to 0.9).
-// Pieces of 2 and 4 MB measured no faster: the link takes 20 us a MB, one host thread about 39 to
+// to_host(x): a host copy of a dense device tensor of bytes; to_host(x, ((offset, bytes), ...)): host
+// copies of those parts, each in memory of its own (a part kept alive keeps no other).  Through two
+// pinned pieces of 1 MB (torch's caching host allocator): the GPU fills one while the host empties the
+// other.  10 MB take 0.39 ms, 3 MB 0.14; the runtime's own copy to pageable memory 0.55 and 0.17 (up to
+// 0.9).  Pieces of 2 and 4 MB measured no faster: the link takes 20 us a MB, one host thread about 39 to
 // empty a piece.
-PyObject* py_to_host(PyObject*, PyObject* o) {
+PyObject* py_to_host(PyObject*, PyObject* const* a, Py_ssize_t na) {
     HANDLE_TH_ERRORS
     constexpr int64_t kPiece = 1 << 20;
-    const at::Tensor* x = dense(o, at::kByte);
+    if (na != 2) SX8_ARGS(1)
+    const at::Tensor* x = dense(a[0], at::kByte);
     if (!x || x->numel() <= kPiece) Py_RETURN_NONE;
-    at::Tensor y;
+    const int64_t n = x->numel(), pieces = (n + kPiece - 1) / kPiece;
+    struct Part {
+        int64_t off, n;
+        at::Tensor y;
+    };
+    c10::SmallVector<Part, 8> parts;
+    if (na == 1) {
+        parts.push_back(Part{0, n, at::Tensor()});
+    } else {
+        if (!PyTuple_Check(a[1])) Py_RETURN_NONE;
+        for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[1]); ++i) {
+            PyObject* p = PyTuple_GET_ITEM(a[1], i);
+            if (!PyTuple_Check(p) || PyTuple_GET_SIZE(p) != 2) Py_RETURN_NONE;
+            const int64_t off = num(PyTuple_GET_ITEM(p, 0)), len = num(PyTuple_GET_ITEM(p, 1));
+            SX8_SIZES_OK()
+            if (off < 0 || len < 0 || off > n || len > n - off) {
+                PyErr_SetString(PyExc_ValueError, "to_host: a part outside the tensor");
+                return nullptr;
+            }
+            parts.push_back(Part{off, len, at::Tensor()});
+        }
+    }
     {
         Unlocked u;
         c10::DeviceGuard on(x->device());
-        const int64_t n = x->numel(), pieces = (n + kPiece - 1) / kPiece;
-        y = at::empty({n}, at::TensorOptions().dtype(at::kByte));
+        for (Part& p : parts) p.y = at::empty({p.n}, at::TensorOptions().dtype(at::kByte));
         const at::Tensor pin = at::empty({2 * kPiece}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
         const hipStream_t st = c10::hip::getCurrentHIPStream(x->device().index()).stream();
         Event ev[2];
@@ -359,17 +381,22 @@ PyObject* py_to_host(PyObject*, PyObject* o) {
                                   std::min(kPiece, n - off), hipMemcpyDeviceToHost, st));
             hip_ok(hipEventRecord(ev[k & 1].e, st));
         };
-        uint8_t* const dst = static_cast<uint8_t*>(y.data_ptr());
         send(0);
         for (int64_t k = 0; k < pieces; ++k) {
             if (k + 1 < pieces) send(k + 1);
             hip_ok(hipEventSynchronize(ev[k & 1].e));
-            const int64_t off = k * kPiece;
+            const int64_t lo = k * kPiece, hi = std::min(lo + kPiece, n);
             const uint8_t* src = stage + (k & 1) * kPiece;
-            std::memcpy(dst + off, src, std::min(kPiece, n - off));
+            for (Part& p : parts) {
+                const int64_t from = std::max(lo, p.off), to = std::min(hi, p.off + p.n);
+                if (from < to) std::memcpy(static_cast<uint8_t*>(p.y.data_ptr()) + (from - p.off), src + (from - lo), to - from);
+            }
         }
     }
-    return THPVariable_Wrap(std::move(y));
+    if (na == 1) return THPVariable_Wrap(std::move(parts[0].y));
+    PyObject* list = PyList_New((Py_ssize_t)parts.size());
+    for (size_t i = 0; list && i < parts.size(); ++i) PyList_SET_ITEM(list, (Py_ssize_t)i, THPVariable_Wrap(std::move(parts[i].y)));
+    return list;
     END_HANDLE_TH_ERRORS
 }
 
@@ -381,7 +408,7 @@ PyMethodDef methods[] = {{"bind", py_bind, METH_O, nullptr},
                          {"gemm_split", SX8_FAST(py_gemm_split), nullptr},
                          {"dequant", SX8_FAST(py_dequant), nullptr},
                          {"embed", SX8_FAST(py_embed), nullptr},
-                         {"to_host", py_to_host, METH_O, nullptr},
+                         {"to_host", SX8_FAST(py_to_host), nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_sx8py", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -132,8 +132,9 @@ def pca_correct(levels, dmin, dmax, config, blocks, n_cb, pca_method="svd"):
 
 
 class _HostFields:
-    """The quantizer's outputs in one device buffer, so that they reach the host in one copy
-    (numpy views of one array): data, scales, dmin, dmax, levels_hi, levels_lo, config, coeff."""
+    """The quantizer's outputs in one device buffer, so that they reach the host in one pass of
+    copies (each an array of its own there): data, scales, dmin, dmax, levels_hi, levels_lo, config,
+    coeff."""
 
     def __init__(self, n_blk, n_cb, device):
         sizes = [("data", n_cb * 256, np.float32), ("scales", n_cb * 8, np.float32), ("dmin", n_blk * 2, np.float16),
@@ -153,9 +154,12 @@ class _HostFields:
         """{name: numpy array}, or None when the bases or scales are not finite (weights with
         infinities or NaN: the caller takes the general path)."""
         import _sx8lib as _L
-        host = _L.py().to_host(self.buf)
-        host = (self.buf.cpu() if host is None else host).numpy()
-        f = {name: host[off:off + nb].view(dt) for name, (off, nb, dt) in self.at.items()}
+        at = [(off, nb) for off, nb, _ in self.at.values()]
+        host = _L.py().to_host(self.buf, tuple(at))
+        if host is None:
+            whole = self.buf.cpu()
+            host = [whole[off:off + nb].clone() for off, nb in at]
+        f = {name: h.numpy().view(dt) for (name, (_, _, dt)), h in zip(self.at.items(), host)}
         f["data"], f["scales"] = f["data"].reshape(self.n_cb, 64), f["scales"].reshape(self.n_cb, 2)
         return f if np.isfinite(f["data"]).all() and np.isfinite(f["scales"]).all() else None
 

@@ -282,3 +282,35 @@ def test_k_blocks_of_another_length(both, cuda, K):
     assert "linear" not in taken and torch.equal(y[0], decode1_v44(x[0], qt, bi, *t)[0].half())
     with pytest.raises(RuntimeError, match="bad shape"):
         m(x)
+
+
+@pytest.mark.gpu
+def test_to_host_parts(hiplib, cuda):
+    """Parts that begin and end at, before and past the 1 MB pieces, empty and overlapping ones."""
+    import _sx8lib
+    M = 1 << 20
+    n = 3 * M + 77
+    x = torch.randint(0, 256, (n,), dtype=torch.uint8, device=cuda)
+    at = ((0, n), (0, 1), (M - 1, 2), (M, M), (5, 2 * M), (n - 1, 1), (n, 0), (2 * M + 3, M + 74))
+    for (off, nb), y in zip(at, _sx8lib.py().to_host(x, at)):
+        assert torch.equal(y, x[off:off + nb].cpu())
+    assert len(_sx8lib.py().to_host(x, at)) == len(at)
+    for bad in ((-1, 2), (0, n + 1), (n, 1)):
+        with pytest.raises(ValueError):
+            _sx8lib.py().to_host(x, (bad,))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(16, 64), (1024, 2560)])
+def test_quantizer_arrays_are_their_own(hiplib, cuda, n, k):
+    """No array of a quantized tensor keeps another one's memory alive."""
+    from quantize_sx8 import quantize_tensor
+    qt, bi = quantize_tensor((torch.randn(n, k, device=cuda) * 0.02).half())
+    sizes = {}
+    for name, a in list(qt.items()) + list(bi.items()):
+        if isinstance(a, np.ndarray):
+            root = a
+            while isinstance(root.base, np.ndarray):
+                root = root.base
+            sizes[name] = (root.nbytes, a.nbytes)
+    assert all(r == own for r, own in sizes.values()), sizes
