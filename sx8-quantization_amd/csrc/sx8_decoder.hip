@@ -726,13 +726,13 @@ __global__ __launch_bounds__(256) void k_qk_rope128(const float* __restrict__ q_
 // chunk count derived from *pos on the device was slower, 1.66: the combine's loads then
 // wait for that read.)
 // Caches longer than kAttnLongL positions get as many chunks (16, 32 or 64) as fill the 256 CUs
-// with one work-group each, never shorter than kAttnMinT positions (one pass of the lane
-// groups); work-groups past the last chunk write an empty partial and stop.  With 16 chunks and
-// 8 KV heads only half the CUs stream the cache.  Split + combine, 32/8 heads of 128, us with 16
-// / 32 / 64 chunks: position 2000 8.5 / 7.7 / 10.2, 8000 17.1 / 12.9 / 14.4, 24000 42.8 / 26.6 /
-// 25.4 (the combine reads every chunk's partials); 4 KV heads at 8000 26.1 / 17.5 / 14.3, 16 KV
-// heads of 64 at 8000 10.2 / 10.7 / 10.8.  A long cache at an early position costs at most 0.3 us
-// (position 700 of 4096: 7.2 / 7.5 / 9.9).
+// with one work-group each, never shorter than kAttnMinT positions (one pass of the lane groups at
+// head dim 128, half a pass at 64); work-groups past the last chunk write an empty partial and
+// stop.  With 16 chunks and 8 KV heads only half the CUs stream the cache.  Split + combine, us with
+// 16 / 32 / 64 chunks: 32/8 heads of 128 at position 700 6.8 / 6.9 / 6.9, 2000 7.9 / 7.0 / 6.9, 8000
+// 15.7 / 11.3 / 11.1, 16000 26.7 / 17.7 / 17.4; 32/4 heads at 700 9.4 / 9.4 / 9.6, 2000 11.5 / 9.6 / 9.8,
+// 8000 24.2 / 15.8 / 12.1; 16/2 heads at 700 9.3 / 9.3 / 9.4, 8000 24.0 / 15.7 / 11.7; 16/16 heads of 64
+// the same with all three.  So more chunks than an early position needs cost at most 0.2 us.
 constexpr int kAttnChunks = 16, kAttnMaxChunks = 64, kAttnMinT = 64;
 constexpr int64_t kAttnLongL = 2048;
 constexpr int64_t kAttnSplitMaxL = (int64_t)1 << 20;
@@ -759,6 +759,11 @@ template <int kCtrl>
 __device__ __forceinline__ float dpp_f(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, 0xF, 0xF,
                                                                  false));
+}
+
+// v of the given (uniform) lane
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
 
 // Sum over the lanes of a lane group, the same value in every lane: DPP quad swaps, then
@@ -1040,48 +1045,70 @@ __global__ __launch_bounds__(256) void k_attn_split(const uint16_t* __restrict__
     }
 }
 
-// NC / 16 groups of HD threads per head, 16 chunks each, then the groups in order.
-template <int HD, int NC = kAttnChunks>
-__global__ __launch_bounds__(HD * (NC / 16)) void k_attn_combine(const float* __restrict__ part,
-                                                                 uint16_t* __restrict__ out) {
-    constexpr int kQ = NC / 16;
-    const int h = blockIdx.x, d = threadIdx.x % HD, q = kQ > 1 ? threadIdx.x / HD : 0;
-    const float* ph = part + ((int64_t)h * NC + 16 * q) * (HD + 2);
-    float mc[16], lc[16], ac[16];
+template <int HD>
+__global__ __launch_bounds__(HD) void k_attn_combine(const float* __restrict__ part,
+                                                     uint16_t* __restrict__ out) {
+    const int h = blockIdx.x, d = threadIdx.x;
+    const float* ph = part + (int64_t)h * kAttnChunks * (HD + 2);
+    float mc[kAttnChunks], lc[kAttnChunks], ac[kAttnChunks];
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {               // every load of the head issued at once
+    for (int c = 0; c < kAttnChunks; ++c) {      // every load of the head issued at once
         mc[c] = ph[c * (HD + 2)];
         lc[c] = ph[c * (HD + 2) + 1];
         ac[c] = ph[c * (HD + 2) + 2 + d];
     }
     float M = mc[0];                             // chunk 0 always holds position 0
 #pragma unroll
-    for (int c = 1; c < 16; ++c) M = fmaxf(M, mc[c]);
-    __shared__ float gm[kQ], gl[kQ][HD], ga[kQ][HD];
-    if constexpr (kQ > 1) {
-        if (d == 0) gm[q] = M;
-        __syncthreads();
-        M = gm[0];
-#pragma unroll
-        for (int i = 1; i < kQ; ++i) M = fmaxf(M, gm[i]);
-    }
+    for (int c = 1; c < kAttnChunks; ++c) M = fmaxf(M, mc[c]);
     float num = 0.f, den = 0.f;
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
+    for (int c = 0; c < kAttnChunks; ++c) {
         const float wc = __expf(mc[c] - M);      // empty chunk: e^-inf = 0, l = acc = 0
         num += wc * ac[c];
         den += wc * lc[c];
     }
-    if constexpr (kQ > 1) {
-        ga[q][d] = num;
-        gl[q][d] = den;
-        __syncthreads();
-        if (q != 0) return;
+    out[h * HD + d] = f2h(num / den);
+}
+
+// The same for 32 or 64 chunks: a work-group per (head, 64 dims), wave q sums chunks 16 q .. 16 q + 15,
+// then the waves in order.  Every thread loading all m and l (as above) is 48 loads a wave and 8 waves on
+// one CU; here lane c holds chunk c's (v_readlane hands them out): 18 loads a wave.  32/4 heads at
+// position 700 with 64 chunks 10.6 -> 9.6 us, 32/8 heads with 32 7.3 -> 6.9.
+template <int HD, int NC>
+__global__ __launch_bounds__(4 * NC) void k_attn_combine_wide(const float* __restrict__ part,
+                                                              uint16_t* __restrict__ out) {
+    constexpr int kQ = NC / 16;
+    const int h = blockIdx.x, lane = threadIdx.x & 63, d = blockIdx.y * 64 + lane;
+    const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float* ph = part + (int64_t)h * NC * (HD + 2);
+    const float mc = ph[(lane % NC) * (HD + 2)], lc = ph[(lane % NC) * (HD + 2) + 1];
+    float ac[16];
 #pragma unroll
-        for (int i = 1; i < kQ; ++i) {
-            num += ga[i][d];
-            den += gl[i][d];
-        }
+    for (int c = 0; c < 16; ++c) ac[c] = ph[(16 * q + c) * (HD + 2) + 2 + d];
+    float M = mc;                                // chunk 0 always holds position 0
+    M = fmaxf(M, dpp_f<0xB1>(M));                // quad_perm [1, 0, 3, 2]
+    M = fmaxf(M, dpp_f<0x4E>(M));                // quad_perm [2, 3, 0, 1]
+    M = fmaxf(M, dpp_f<0x141>(M));               // row_half_mirror
+    M = fmaxf(M, dpp_f<0x140>(M));               // row_mirror
+    M = fmaxf(M, __shfl_xor(M, 16));
+    M = fmaxf(M, __shfl_xor(M, 32));
+    const float wl = __expf(mc - M);             // empty chunk: e^-inf = 0, l = acc = 0
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        const float wc = lane_value(wl, 16 * q + c);
+        num += wc * ac[c];
+        den += wc * lane_value(lc, 16 * q + c);
+    }
+    __shared__ float gl[kQ], ga[kQ][64];
+    ga[q][lane] = num;
+    if (lane == 0) gl[q] = den;
+    __syncthreads();
+    if (q != 0) return;
+#pragma unroll
+    for (int i = 1; i < kQ; ++i) {
+        num += ga[i][lane];
+        den += gl[i];
     }
     out[h * HD + d] = f2h(num / den);
 }
@@ -1891,7 +1918,11 @@ template <int HD>
 static void launch_combine(int nc, int nh, const float* part, uint16_t* out, hipStream_t st) {
     by_chunks(nc, [&](auto c) {
         constexpr int NC = decltype(c)::value;
-        hipLaunchKernelGGL((k_attn_combine<HD, NC>), dim3((unsigned)nh), dim3(HD * NC / 16), 0, st, part, out);
+        if constexpr (NC == kAttnChunks)
+            hipLaunchKernelGGL((k_attn_combine<HD>), dim3((unsigned)nh), dim3(HD), 0, st, part, out);
+        else
+            hipLaunchKernelGGL((k_attn_combine_wide<HD, NC>), dim3((unsigned)nh, HD / 64), dim3(4 * NC), 0, st, part,
+                               out);
     });
 }
 

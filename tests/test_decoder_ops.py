@@ -422,7 +422,10 @@ def test_argmax_advance(hiplib, cuda, n, offset):
     (8, 4, 64, 64, [0, 63]),
     (32, 8, 128, 1500, [0, 700, 1499]),
     (16, 2, 128, 400, [0, 399]),                   # G = 8
-    (8, 2, 128, 3000, [0, 2047, 2999]),            # a longer cache (94 positions per chunk)
+    (8, 2, 128, 3000, [0, 2047, 2999]),            # a longer cache: 64 chunks of at least 64 positions
+    (32, 8, 128, 4096, [0, 63, 64, 127, 2047, 2048, 4094, 4095]),     # 32 chunks
+    (32, 4, 128, 2500, [63, 64, 1000, 2499]),      # 64 chunks, G = 8
+    (8, 8, 64, 4100, [0, 64, 128, 4099]),          # 32 chunks, half a pass each
 ])
 def test_attn_rope_matches_two_calls(hiplib, cuda, nh, nk, hd, L, positions):
     """sx8_dec_attn_rope against sx8_dec_qk_rope_cache + sx8_dec_attn_split: the new k/v rows
