@@ -1,4 +1,4 @@
-// sx8_gemm_small.hip -- Y (M, N) = X (M, K) . W^T for a few rows (M <= 64: batched decode,
+// sx8_gemm_small.hip -- Y (M, N) = X (M, K) . W^T for a few rows (M <= 128: batched decode,
 // short prompts), W in S-X8 blocks.
 //
 // What bounds it: the decode's VALU work and the packed weights (30 bytes per 32 weights, read
@@ -16,8 +16,8 @@
 //     sub-block would need four times the memory instructions -- and does the range
 //     arithmetic of its record's four sub-blocks.  MFMA j of a group of four blocks then takes
 //     sub-block j of each lane's own block: the K index only has to agree with X, whose
-//     packed copy is read in that order.  Plain rows (kRaw) take block t per MFMA instead (the
-//     Z products need whole blocks): 4 x 4 transposes across the wave's 16-lane rows
+//     packed copy is read in that order.  Plain rows (kRaw) take block t per MFMA instead, as
+//     the Z products here take their blocks: 4 x 4 transposes across the wave's 16-lane rows
 //     (v_permlane32_swap, v_permlane16_swap) hand lane (c, g) its sub-block of every block;
 //   * PCA: one extra MFMA per four blocks, K slots 8 t .. 8 t + 3 = block t's (c0, c0, c1, c1)
 //     (lane (c, t) already holds that record) against (Z0 hi, Z0 lo, Z1 hi, Z1 lo);
@@ -26,8 +26,8 @@
 // Two forms of input: the packed operands of the prefill GEMM (packed X + Zhl, written by the
 // pack pass or by a producer kernel), or plain fp16 rows (kRaw), for which Z is computed on
 // the matrix core too: the block's two basis vectors, split into fp16 hi + lo (22 bits of the
-// largest element), are four rows of an A operand, so the product with the block's X lands, for every row of X,
-// in the lane that feeds it to the PCA MFMA.
+// largest element), are four rows of an A operand, so the product with the block's X lands, for
+// every row of X, in the lane that feeds it to the PCA MFMA.
 // Measured (kernel alone, packed, against k_gemm + k_reduce): 9728 x 2560 at 8 rows 9.9 against
 // 17.7 us, 2560 x 9728 at 16 rows 11.6 against 22.5, 4096 x 2560 at 16 / 64 / 128 rows 5.6 / 9.1 /
 // 14.5 against 11.9 / 15.1 / 18.7.  One launch from plain rows to fp16 outputs (kRaw): gate
@@ -196,7 +196,7 @@ __device__ __forceinline__ float abs_max3(float a, float b, float c) {
 
 constexpr int kMaxWaves = 8;
 
-// Work-group: 64 S threads (S waves); 16 CF columns, 16 MT rows (row block mb = blockIdx / NB).
+// Work-group: 64 S threads (S waves); 16 CF columns, all rows (M <= 16 MT).
 template <bool kSplit, int HB, bool kRaw, int MT, int CF>
 __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* __restrict__ X, int M, int K,
                                                                int64_t ldx, int n_cb, const SmallGroup grp) {
@@ -206,15 +206,12 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int S = (int)(blockDim.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int G = grp.NB;
-    const int mb = (int)blockIdx.x / G;
-    int nb = xcd_order_small((int)blockIdx.x - mb * G, G);
+    int nb = xcd_order_small((int)blockIdx.x, grp.NB);
     int mi = 0;
     while (mi + 1 < grp.n_mats && nb >= grp.m[mi].nb) nb -= grp.m[mi++].nb;
     const SmallMat& mat = grp.m[mi];
     const int N = mat.N;
     const int n0 = nb * 16 * CF;
-    const int m0 = mb * 16 * MT;
     const int n_groups = (n_cb + 3) >> 2;
 
     const RecSrc ws = rec_src<kSplit, HB>(mat.w, (int64_t)N * n_cb);
@@ -240,7 +237,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
     auto x_imm = [](int t) { return kRaw ? 64u * t : 1024u * (t & 1) + 512u * (t >> 1); };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        const int m = m0 + 16 * mt + c;
+        const int m = 16 * mt + c;
         if constexpr (kRaw) {
             xo[mt] = m < M ? (uint32_t)(m * (int)ldx * 2 + 16 * g) + 256u * wave : kOob;
         } else {
@@ -255,7 +252,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
     if constexpr (kRaw) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const int m = min(m0 + 16 * mt + c, M - 1);
+            const int m = min(16 * mt + c, M - 1);
             x_last[mt] = (K & 1) ? __builtin_amdgcn_raw_buffer_load_b16(xs, (uint32_t)(m * (int)ldx + K - 1) * 2, 0, 0) : 0;
         }
     }
@@ -477,7 +474,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
         sx8_float4 v = red[o];
         for (int w = 1; w < S; ++w) v += red[w * kOut + o];
         const int l = o & 63, f = o >> 6;
-        const int m = m0 + 16 * (f % MT) + (l & 15);
+        const int m = 16 * (f % MT) + (l & 15);
         const int n = n0 + 16 * (f / MT) + 4 * (l >> 4);
         if (m >= M || n >= N) continue;
         if constexpr (kRaw) {
@@ -519,8 +516,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
 // launch, prologue and sum.  Fitted on packed calls, CF = 1: 1024 x 2560 at 16 / 64 / 128 rows 5.1
 // / 8.65 / 13.8 us, 2560 x 9728 at 16 / 64 rows 11.3 / 23.7, 512 x 512 at 64 rows 4.5.  More
 // fragments only pay where they save a round of work-groups over the CUs: gate_proj (9728
-// columns) at 32 rows 13.2 / 13.2 / 11.2 us with CF = 1 / 2 / 3 (608, 304, 203 tiles).  Raw
-// rows add the basis conversion and the Z products of every tile.
+// columns) at 32 rows 13.2 / 13.2 / 11.2 us with CF = 1 / 2 / 3 (608, 304, 203 tiles); with one
+// packed row fragment, whose time is all decode, they never do.  Raw rows add the basis
+// conversion and the Z products of every tile.
 // Eight waves per work-group (two per SIMD) hide the loads where a CU has one work-group and
 // the row fragments are few (down at 16 rows 11.6 against 14.3 us with four); else four, so
 // that two or three work-groups share a CU (gate at 64 rows 17.5 against 20.7).
@@ -529,9 +527,12 @@ struct SmallPlan {
     double us;
 };
 
+// most column fragments a wave may take: what its registers hold past two row fragments
+constexpr int max_cf(int64_t MT, bool raw) { return MT == 1 && !raw ? 1 : MT <= 2 ? 3 : MT <= 5 ? 2 : 1; }
+
 SmallPlan plan_small(int64_t MT, int n_mats, const int64_t* Ns, int64_t n_groups, bool raw) {
     SmallPlan best{1, 8, 1e300};
-    for (int cf = 1; cf <= (MT <= 2 ? 3 : MT <= 5 ? 2 : 1); ++cf) {
+    for (int cf = 1; cf <= max_cf(MT, raw); ++cf) {
         int64_t tiles = 0;
         for (int i = 0; i < n_mats; ++i) tiles += (Ns[i] + 16 * cf - 1) / (16 * cf);
         const double per = raw ? 0.1 + 0.53 * cf + 0.4 * (double)(MT - 1) : 0.38 * cf + 0.245 * (double)(MT - 1);
@@ -559,8 +560,9 @@ void launch_small(int64_t MT, const SmallPlan& p, int64_t grid, const uint16_t* 
                   int64_t ldx, int64_t n_cb, const SmallGroup& g, hipStream_t st) {
     auto go = [&](auto mt) {
         constexpr int kMT = decltype(mt)::value;
-        if (kMT <= 2 && p.cf == 3) launch_one<kSplit, HB, kRaw, kMT, kMT <= 2 ? 3 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
-        else if (kMT <= 5 && p.cf == 2) launch_one<kSplit, HB, kRaw, kMT, kMT <= 5 ? 2 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
+        constexpr int kCF = max_cf(kMT, kRaw);
+        if (kCF >= 3 && p.cf == 3) launch_one<kSplit, HB, kRaw, kMT, kCF >= 3 ? 3 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
+        else if (kCF >= 2 && p.cf == 2) launch_one<kSplit, HB, kRaw, kMT, kCF >= 2 ? 2 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
         else launch_one<kSplit, HB, kRaw, kMT, 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
     };
     if (MT == 1) go(std::integral_constant<int, 1>{});

@@ -1,6 +1,6 @@
 """Few-row GEMMs (sx8_gemm_small.hip): sx8_linear_f16 and the packed form behind the prefill
 entry points at up to 128 rows.  Sizes at the edges of the kernel's tiles: 16-row fragments,
-16 / 32 / 48-column tiles, four-block groups, K tails inside a block and odd rows (whose last
+16 / 32 / 48-column tiles (every pair of row and column fragments that a plan picks), four-block groups, K tails inside a block and odd rows (whose last
 element shares a word with the next row).  W16 is the oracle's R64 dequant; the bar against its
 float64 product is the other GEMM tests' 1e-3 of max |Y| (weights rounded to fp16), and the
 tiled kernels, forced by SX8_GEMM_TILE, multiply the same fp16 operands, so the two differ by
@@ -27,7 +27,7 @@ def _rel(a, b):
 @pytest.mark.parametrize("M,N,K,hb,bias", [
     (2, 64, 32, 6, False), (3, 80, 31, 8, True), (15, 1000, 1333, 6, True), (16, 2560, 4096, 8, False),
     (17, 1024, 2560, 6, True), (31, 9728, 515, 6, False), (32, 305, 2081, 8, True), (1, 129, 97, 6, False),
-    (8, 4099, 640, 6, True),
+    (8, 4099, 640, 6, True), (8, 9728, 515, 6, True), (12, 6000, 99, 8, False), (32, 6001, 160, 8, True),
 ])
 def test_linear_f16(hiplib, oracle, cuda, M, N, K, hb, bias):
     """fp16 outputs against the oracle (fp16 rounding on top of the GEMM bar), the bias as an
@@ -151,7 +151,9 @@ def test_one_row_equals_gemv(hiplib, cuda, N, K, hb, bias):
 @pytest.mark.parametrize("M,Ns,K,hb", [
     (1, [64], 96, 6), (16, [1000], 2560, 8), (17, [129, 300, 64, 700], 80, 6), (33, [4096, 1024, 1024], 2560, 6),
     (48, [777], 1000, 6), (49, [513], 4096, 8), (64, [9728], 640, 6), (65, [640], 1333, 6), (80, [1001], 515, 8),
-    (96, [300, 500], 2081, 6), (97, [256], 129, 6), (128, [2560], 2560, 6),
+    (96, [300, 500], 2081, 6), (97, [256], 129, 6), (128, [2560], 2560, 6), (16, [9729], 515, 6), (32, [9728], 640, 8),
+    (27, [4001, 3000, 1000, 900], 259, 6), (31, [6001], 320, 8), (45, [5003], 640, 6), (64, [4100, 2000], 515, 8),
+    (80, [5001], 320, 6),
 ])
 def test_packed_forms_match_tiles(hiplib, oracle, cuda, gemm_tuning, M, Ns, K, hb):
     """sx8_gemm_prefill_group against the oracle, against the tiled kernels, and against the
