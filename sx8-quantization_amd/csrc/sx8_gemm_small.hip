@@ -197,7 +197,10 @@ __device__ __forceinline__ float abs_max3(float a, float b, float c) {
 constexpr int kMaxWaves = 8;
 
 // Work-group: 64 S threads (S waves); 16 CF columns, all rows (M <= 16 MT).
-template <bool kSplit, int HB, bool kRaw, int MT, int CF>
+// kOdd (raw): rows that do not all begin on 4 bytes.  A 16-byte load that is 2 bytes off splits into many
+// (32 rows, 4096 columns: K = 4095 34.8 us, 4096 14.3), so these read whole words, one more than they need,
+// and shift by half a word where the row begins in the middle of one: 16.9 us (16 rows 19.9 -> 11.7).
+template <bool kSplit, int HB, bool kRaw, bool kOdd, int MT, int CF>
 __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* __restrict__ X, int M, int K,
                                                                int64_t ldx, int n_cb, const SmallGroup grp) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -216,8 +219,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
 
     const RecSrc ws = rec_src<kSplit, HB>(mat.w, (int64_t)N * n_cb);
     sx8_rsrc xs, zs, ss;
+    const uint32_t x_off = kOdd ? (uint32_t)(reinterpret_cast<uintptr_t>(X) & 3) : 0u;    // X's place in its word
     if constexpr (kRaw) {
-        xs = make_rsrc(X, ((int64_t)(M - 1) * ldx + K) * 2);
+        xs = make_rsrc(kOdd ? reinterpret_cast<const void*>(reinterpret_cast<uintptr_t>(X) & ~(uintptr_t)3) : X,
+                       ((int64_t)(M - 1) * ldx + K) * 2 + x_off);
         zs = make_rsrc(mat.basis, (int64_t)n_cb * 256);
         ss = make_rsrc(mat.scales, (int64_t)n_cb * 8);
     } else {
@@ -233,27 +238,32 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
     const uint32_t bid_step = (uint32_t)(4 * S) * (uint32_t)N;
     // X operand t: kRaw: row m, values 32 (kb0 + t) + 8 g ..; packed: chunk (row group, kb0 +
     // g), its 16-byte piece t (k-step t & 1, half t / 2) of row m
-    uint32_t xo[MT], zo[MT];
+    uint32_t xo[MT], zo[MT], x_sh[kOdd ? MT : 1];
     auto x_imm = [](int t) { return kRaw ? 64u * t : 1024u * (t & 1) + 512u * (t >> 1); };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int m = 16 * mt + c;
         if constexpr (kRaw) {
-            xo[mt] = m < M ? (uint32_t)(m * (int)ldx * 2 + 16 * g) + 256u * wave : kOob;
+            xo[mt] = m < M ? (uint32_t)(m * (int)ldx * 2 + 16 * g) + x_off + 256u * wave : kOob;
+            if constexpr (kOdd) {
+                x_sh[mt] = (xo[mt] & 2) * 8;
+                xo[mt] &= ~3u;
+            }
         } else {
             xo[mt] = (uint32_t)(((m >> 5) * n_cb + g) * 2048 + (m & 31) * 16) + 8192u * wave;
             if (m - c >= M) xo[mt] = kOob;
             zo[mt] = m < M ? (uint32_t)((m * n_cb + g) * 8) + 32u * wave : kOob;
         }
     }
-    // the last element of an odd-length row, whose 4-byte word may straddle the end of X
-    // (a buffer load of it reads zero)
+    // the last element of a row, whose 4-byte word may straddle the end of X (a buffer load of it
+    // reads zero): of an odd length, or in a row that begins in the middle of a word
     uint32_t x_last[kRaw ? MT : 1];
     if constexpr (kRaw) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int m = min(16 * mt + c, M - 1);
-            x_last[mt] = (K & 1) ? __builtin_amdgcn_raw_buffer_load_b16(xs, (uint32_t)(m * (int)ldx + K - 1) * 2, 0, 0) : 0;
+            const uint32_t at = (uint32_t)(m * (int)ldx + K - 1) * 2 + x_off;
+            x_last[mt] = kOdd || (K & 1) ? __builtin_amdgcn_raw_buffer_load_b16(xs, at, 0, 0) : 0;
         }
     }
 
@@ -261,6 +271,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
     // X operands in flight: the whole next group, or two operands ahead past four row fragments
     constexpr int kRing = MT > 4 ? 2 : 4;
     u32x4 x[MT][kRing];
+    uint32_t x_more[kOdd ? MT : 1][kRing];
     u32x4 z4[kRaw ? 2 : 1];
     uint2 zp[kRaw ? 1 : MT];
     float2 sc = make_float2(0.f, 0.f);
@@ -273,8 +284,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
     };
     auto load_x = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt) {
             x[mt][t % kRing] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xs, xo[mt] + x_imm(t), 0, 0));
+            if constexpr (kOdd) x_more[mt][t % kRing] = __builtin_amdgcn_raw_buffer_load_b32(xs, xo[mt] + x_imm(t) + 16, 0, 0);
+        }
     };
     auto next_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -362,9 +375,20 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
             for (int cf = 0; cf < CF; ++cf) frag_prep<kSplit, kRaw>(fr[cf], r[cf]);
             if (z_far()) z_scale();
         }
-        // values past K (raw) or blocks past n_cb (packed) count as zero
+        // values past K (raw) or blocks past n_cb (packed) count as zero (kOdd: and the last value is
+        // put in where its word straddles the end of X, also where no value is past K)
         const int kb0 = 4 * gi;
-        const bool last = kb0 * 32 + 128 > (kRaw ? K : n_cb * 32);
+        const bool last = kb0 * 32 + 128 + (kOdd ? 1 : 0) > (kRaw ? K : n_cb * 32);
+        if constexpr (kOdd) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        x[mt][t][i] = __builtin_amdgcn_alignbit(i < 3 ? x[mt][t][i < 3 ? i + 1 : 0] : x_more[mt][t],
+                                                                x[mt][t][i], x_sh[mt]);
+        }
         if constexpr (kRaw) {
             if (last) {
 #pragma unroll
@@ -373,8 +397,11 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            x[mt][t][i] = left >= 2 * i + 2 ? x[mt][t][i] : left == 2 * i + 1 ? x_last[mt] : 0u;
+                        for (int i = 0; i < 4; ++i) {
+                            const uint32_t w = x[mt][t][i];
+                            const uint32_t end = kOdd && left == 2 * i + 2 ? (w & 0xFFFFu) | (x_last[mt] << 16) : w;
+                            x[mt][t][i] = left >= 2 * i + 2 ? end : left == 2 * i + 1 ? x_last[mt] : 0u;
+                        }
                 }
             }
         } else if (last) {
@@ -547,23 +574,23 @@ int64_t row_frags(int64_t M) {
     return MT == 7 ? 8 : MT;
 }
 
-template <bool kSplit, int HB, bool kRaw, int MT, int CF>
+template <bool kSplit, int HB, bool kRaw, bool kOdd, int MT, int CF>
 void launch_one(int S, int64_t grid, const uint16_t* X, int64_t M, int64_t K, int64_t ldx, int64_t n_cb,
                 const SmallGroup& g, hipStream_t st) {
     const size_t lds = (size_t)S * CF * MT * 1024;
-    hipLaunchKernelGGL((k_gemm_small<kSplit, HB, kRaw, MT, CF>), dim3((unsigned)grid), dim3(64 * S), lds, st, X,
+    hipLaunchKernelGGL((k_gemm_small<kSplit, HB, kRaw, kOdd, MT, CF>), dim3((unsigned)grid), dim3(64 * S), lds, st, X,
                        (int)M, (int)K, ldx, (int)n_cb, g);
 }
 
-template <bool kSplit, int HB, bool kRaw>
+template <bool kSplit, int HB, bool kRaw, bool kOdd = false>
 void launch_small(int64_t MT, const SmallPlan& p, int64_t grid, const uint16_t* X, int64_t M, int64_t K,
                   int64_t ldx, int64_t n_cb, const SmallGroup& g, hipStream_t st) {
     auto go = [&](auto mt) {
         constexpr int kMT = decltype(mt)::value;
         constexpr int kCF = max_cf(kMT, kRaw);
-        if (kCF >= 3 && p.cf == 3) launch_one<kSplit, HB, kRaw, kMT, kCF >= 3 ? 3 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
-        else if (kCF >= 2 && p.cf == 2) launch_one<kSplit, HB, kRaw, kMT, kCF >= 2 ? 2 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
-        else launch_one<kSplit, HB, kRaw, kMT, 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
+        if (kCF >= 3 && p.cf == 3) launch_one<kSplit, HB, kRaw, kOdd, kMT, kCF >= 3 ? 3 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
+        else if (kCF >= 2 && p.cf == 2) launch_one<kSplit, HB, kRaw, kOdd, kMT, kCF >= 2 ? 2 : 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
+        else launch_one<kSplit, HB, kRaw, kOdd, kMT, 1>(p.S, grid, X, M, K, ldx, n_cb, g, st);
     };
     if (MT == 1) go(std::integral_constant<int, 1>{});
     else if (kRaw || MT == 2) go(std::integral_constant<int, 2>{});
@@ -633,7 +660,13 @@ int32_t gemm_small_raw(const char* what, int32_t hdr_bytes, const uint16_t* X, i
     g.m[0].scales = scales;
     g.m[0].bias = bias;
     g.m[0].Y = Y;
-    if (hdr_bytes == 8) launch_small<false, 8, true>(MT, p, NB, X, M, K, ldx, n_cb, g, st);
+    // word loads where at least two rows begin off 4 bytes; one such row costs less than the extra words
+    // (K = 4095, 4096 columns, 2 / 3 / 4 / 8 rows 9.0 / 9.4 / 10.2 / 13.0 us without them, 9.9 / 9.9 / 9.9 / 9.8 with)
+    const int64_t off = !aligned(X, 4);
+    const bool odd = ((ldx & 1) ? (M + off) / 2 : off * M) >= 2;
+    if (hdr_bytes == 8 && odd) launch_small<false, 8, true, true>(MT, p, NB, X, M, K, ldx, n_cb, g, st);
+    else if (hdr_bytes == 8) launch_small<false, 8, true>(MT, p, NB, X, M, K, ldx, n_cb, g, st);
+    else if (odd) launch_small<false, 6, true, true>(MT, p, NB, X, M, K, ldx, n_cb, g, st);
     else launch_small<false, 6, true>(MT, p, NB, X, M, K, ldx, n_cb, g, st);
     return check_launch(what);
 }

@@ -70,6 +70,41 @@ def test_linear_f16(hiplib, oracle, cuda, M, N, K, hb, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [2, 16, 31])
+@pytest.mark.parametrize("K", [31, 96, 128, 129, 510, 512, 2047])
+def test_linear_f16_row_starts(hiplib, cuda, M, K):
+    """Rows that begin anywhere in their 4-byte words, with NaN before, between and after them, give
+    bit for bit what the same rows at 16 bytes give."""
+    import torch
+    import _sx8lib as L
+    from sx8_decode1_v3 import make_tensors_v44
+    print("row starts", M, K, flush=True)
+    N = 70
+    qt, bi = _quantized(N, K, M + K, cuda)
+    t = make_tensors_v44(qt, bi)
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)).half().to(cuda)
+    P = L.ptr
+
+    def call(x, ld):
+        Y = torch.full((M, N), 7.0, dtype=torch.float16, device=cuda)
+        L.call("sx8_linear_f16", P(x), M, ld, K, P(t[0]), P(t[1]), 6, P(t[2]), P(t[3]), None, N, qt["n_cb"], P(Y),
+               L.stream(cuda))
+        return Y
+    pad = (K + 7) // 8 * 8
+    even = torch.full((M, pad), float("nan"), dtype=torch.float16, device=cuda)
+    even[:, :K] = X
+    want = call(even, pad)
+    assert want.isfinite().all()
+    for ld in (K, K + 1, K + 2):
+        for off in (0, 1, 2, 3):
+            for tail in (0, 1):                       # X ends where its buffer ends, and before
+                buf = torch.full((off + (M - 1) * ld + K + tail,), float("nan"), dtype=torch.float16, device=cuda)
+                x = buf[off:].as_strided((M, K), (ld, 1))
+                x.copy_(X)
+                assert torch.equal(call(x, ld), want), (ld, off, tail)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [2, 17, 32])
 def test_linear_f16_basis_range(hiplib, cuda, M):
     """Bases of any length with their scales the other way: Z keeps its 22 bits, and powers of two
