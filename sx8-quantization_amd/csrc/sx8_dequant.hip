@@ -14,10 +14,9 @@
 // rows, and every store instruction writes 1 KB of one output row.  One thread per (block,
 // sub-block) issues four times the load instructions, re-reads and converts the basis for
 // every 16 bytes of output: 9728 x 2560 20.9 us, here 17.8 (a 73 MB copy takes 14.2; with the
-// decode replaced by plain moves the kernel takes 14.4).  It stays for tensors too small to fill the
-// GPU with waves of four rows.
+// decode replaced by plain moves the kernel takes 14.4).  It stays where it is the faster one
+// (wave_wins).
 #include <algorithm>
-#include <type_traits>
 
 #include "sx8_device.h"
 #include "sx8_host.h"
@@ -121,7 +120,7 @@ __device__ __forceinline__ void gather_rows(uint32_t v, uint32_t (&o)[4]) {
 
 // Output rows 4 quad + t (quad = this wave's) of T: row ids[.] of the weight, or row row0 + .
 // without ids; rows outside [0, N) are skipped.  blockIdx.x: 16-block column group.
-template <typename Src, bool kIds, bool kVec>
+template <typename Src, bool kIds>
 __global__ __launch_bounds__(kThreads) void k_dequant_wave(const Src src, const int64_t* __restrict__ ids,
                                                            const float* __restrict__ basis,
                                                            const float* __restrict__ scales, int64_t T, int64_t N,
@@ -159,39 +158,46 @@ __global__ __launch_bounds__(kThreads) void k_dequant_wave(const Src src, const 
                          (g & 1) ? p[i] >> 16 : p[i] & 0xFFFFu, b0, b1, s0, s1, w);
         uint16_t* o = out + (quad * 4 + i) * in_f;
         const int64_t col = (int64_t)kb * 32 + 8 * g;
-        if constexpr (kVec) {
-            if (col < in_f) *reinterpret_cast<uint4*>(o + col) = make_uint4(w[0], w[1], w[2], w[3]);
-        } else {
-            if (kb < n_cb) store8(o, col, in_f, false, w);
-        }
+        if (col < in_f) *reinterpret_cast<uint4*>(o + col) = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }
 
-// The wave kernel where it has at least four waves per SIMD to run, false otherwise: a wave's four
-// rows are a chain that few waves do not hide (1024 x 2560: 1280 waves 5.5 us against 4.3; 4096 rows of
-// 2560 gathered, 5120 waves: 19.8 against 21.0), and where at most a fifth of its lanes idle in the last
-// 16-block group (5000 x 333, 11 blocks: 7.7 against 5.4 us).
-template <typename Src>
-bool launch_wave(const Src& src, const int64_t* ids, const float* basis, const float* scales, int64_t T, int64_t N,
-                 int64_t n_cb, int64_t in_f, bool vec_ok, uint16_t* out, hipStream_t st) {
+// Whether the wave kernel is the faster one.  A wave's four rows are a chain that few waves do not hide, and
+// the lanes past n_cb of the last 16-block group idle.  us, one thread per (block, sub-block) / wave kernel:
+//   any rows, output rows off 16 bytes (element stores, which its lane order scatters): 9728 x 2557 38.5 / 50.0
+//   rows in order, split arrays: 4096 x 1664 (81% of the lanes used) 7.6 / 8.7; 3300 x 2560 8.9 / 9.4; 6500 x 1472
+//     9.7 / 9.5; 9728 x 2560 20.6 / 17.9
+//   rows in order, v4.4: 4096 x 1664 9.3 / 9.0; 9728 x 2560 30.3 / 18.2
+//   rows by ids, v4.4 (each record a memory access of its own either way): 4096 x 2560 18.7 / 18.9, 8192 x 3584
+//     47.3 / 50.6; ahead only for whole sets of four column groups (4096 x 2048 15.4 / 14.9) or many waves (16384
+//     x 3072 83.1 / 80.0)
+enum class Rows { kSplit, kV44, kV44Ids };
+bool wave_wins(Rows r, int64_t T, int64_t n_cb, bool vec_ok) {
     const int64_t quads = (T + 3) / 4, cols = (n_cb + 15) / 16;
-    if (quads * cols < 4096 || n_cb * 5 < cols * 16 * 4 || cols > 0x7FFFFFFF / 16) return false;
+    if (!vec_ok || cols > 0x7FFFFFFF / 16) return false;
+    switch (r) {
+        case Rows::kSplit: return n_cb * 8 >= cols * 16 * 7 && quads * n_cb >= 16 * 4600;
+        case Rows::kV44: return n_cb * 5 >= cols * 16 * 4 && quads * cols >= 4096;
+        default: return (n_cb % 64 == 0 && quads * cols >= 4096) || quads * n_cb >= 16 * 23000;
+    }
+}
+
+template <typename Src>
+void launch_wave(const Src& src, const int64_t* ids, const float* basis, const float* scales, int64_t T, int64_t N,
+                 int64_t n_cb, int64_t in_f, uint16_t* out, hipStream_t st) {
+    const int64_t cols = (n_cb + 15) / 16;
     // blockIdx.y takes at most 65535 work-groups: more rows go in several launches
     constexpr int64_t kRows = (int64_t)65535 * kWaves * 4;
     for (int64_t t0 = 0; t0 < T; t0 += kRows) {
         const int64_t Tc = std::min(kRows, T - t0);
         const dim3 grid((unsigned)cols, (unsigned)((Tc + kWaves * 4 - 1) / (kWaves * 4)));
-        auto go = [&](auto with_ids, auto vec) {
-            hipLaunchKernelGGL((k_dequant_wave<Src, decltype(with_ids)::value, decltype(vec)::value>), grid,
-                               dim3(kThreads), 0, st, src, ids ? ids + t0 : nullptr, basis, scales, Tc, N, (int)n_cb,
-                               in_f, out + t0 * in_f, t0);
-        };
-        if (ids && vec_ok) go(std::true_type{}, std::true_type{});
-        else if (ids) go(std::true_type{}, std::false_type{});
-        else if (vec_ok) go(std::false_type{}, std::true_type{});
-        else go(std::false_type{}, std::false_type{});
+        if (ids)
+            hipLaunchKernelGGL((k_dequant_wave<Src, true>), grid, dim3(kThreads), 0, st, src, ids + t0, basis, scales, Tc,
+                               N, (int)n_cb, in_f, out + t0 * in_f, t0);
+        else
+            hipLaunchKernelGGL((k_dequant_wave<Src, false>), grid, dim3(kThreads), 0, st, src, nullptr, basis, scales, Tc,
+                               N, (int)n_cb, in_f, out + t0 * in_f, t0);
     }
-    return true;
 }
 
 __global__ __launch_bounds__(kThreads) void k_dequant_split(
@@ -264,9 +270,11 @@ extern "C" int32_t sx8_dequant_f16(const uint16_t* dmin, const uint16_t* dmax,
         return fail(SX8_ERR_INVALID, "sx8_dequant_f16: misaligned pointer");
     const int64_t n_blocks = out_f * n_cb;
     const bool vec_ok = aligned(out, 16) && (in_f % 8 == 0);
-    if (launch_wave(SplitSrc{dmin, dmax, config, coeff, levels_hi, levels_lo, n_cb}, nullptr, basis, scales, out_f,
-                    out_f, n_cb, in_f, vec_ok, out, as_stream(stream)))
+    if (wave_wins(Rows::kSplit, out_f, n_cb, vec_ok)) {
+        launch_wave(SplitSrc{dmin, dmax, config, coeff, levels_hi, levels_lo, n_cb}, nullptr, basis, scales, out_f, out_f,
+                    n_cb, in_f, out, as_stream(stream));
         return check_launch("sx8_dequant_f16");
+    }
     const int64_t threads = n_blocks * 4;
     const int64_t grid = (threads + kThreads - 1) / kThreads;
     if (grid > 0x7FFFFFFF) return fail(SX8_ERR_UNSUPPORTED, "sx8_dequant_f16: tensor too large");
@@ -295,9 +303,11 @@ extern "C" int32_t sx8_embed_gather(const int64_t* ids, int64_t T, const uint8_t
     if (T == 0) return ok();
     const bool vec_ok = aligned(out, 16) && (K % 8 == 0);
     const hipStream_t st = as_stream(stream);
-    if (hdr_bytes == 8 ? launch_wave(V44Src<8>{hdr, levels, N}, ids, basis, scales, T, N, n_cb, K, vec_ok, out, st)
-                       : launch_wave(V44Src<6>{hdr, levels, N}, ids, basis, scales, T, N, n_cb, K, vec_ok, out, st))
+    if (wave_wins(ids ? Rows::kV44Ids : Rows::kV44, T, n_cb, vec_ok)) {
+        if (hdr_bytes == 8) launch_wave(V44Src<8>{hdr, levels, N}, ids, basis, scales, T, N, n_cb, K, out, st);
+        else launch_wave(V44Src<6>{hdr, levels, N}, ids, basis, scales, T, N, n_cb, K, out, st);
         return check_launch("sx8_embed_gather");
+    }
     const int64_t threads = T * n_cb * 4;
     const int64_t grid = (threads + kThreads - 1) / kThreads;
     if (grid > 0x7FFFFFFF) return fail(SX8_ERR_UNSUPPORTED, "sx8_embed_gather: too many rows");
