@@ -541,7 +541,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
 // of four blocks costs a SIMD ~0.38 us per column fragment (the decode) plus 0.245 us per
 // further row fragment (X comes through the vector cache once per wave), on top of 3.3 us of
 // launch, prologue and sum.  Fitted on packed calls, CF = 1: 1024 x 2560 at 16 / 64 / 128 rows 5.1
-// / 8.65 / 13.8 us, 2560 x 9728 at 16 / 64 rows 11.3 / 23.7, 512 x 512 at 64 rows 4.5.  More
+// / 8.65 / 13.8 us, 2560 x 9728 at 16 / 64 rows 11.3 / 23.7, 512 x 512 at 64 rows 4.5.  Eight row
+// fragments in three rounds of work-groups take 3-4 us more than that (12288 x 512 at 128 rows 13.9
+// us, the tiled kernel 12.8).  More
 // fragments only pay where they save a round of work-groups over the CUs: gate_proj (9728
 // columns) at 32 rows 13.2 / 13.2 / 11.2 us with CF = 1 / 2 / 3 (608, 304, 203 tiles); with one
 // packed row fragment, whose time is all decode, they never do.  Raw rows add the basis
@@ -563,7 +565,8 @@ SmallPlan plan_small(int64_t MT, int n_mats, const int64_t* Ns, int64_t n_groups
         int64_t tiles = 0;
         for (int i = 0; i < n_mats; ++i) tiles += (Ns[i] + 16 * cf - 1) / (16 * cf);
         const double per = raw ? 0.1 + 0.53 * cf + 0.4 * (double)(MT - 1) : 0.38 * cf + 0.245 * (double)(MT - 1);
-        const double us = 3.3 + (double)((tiles + 255) / 256) * (double)((n_groups + 3) / 4) * per;
+        const int64_t rounds = (tiles + 255) / 256;
+        const double us = 3.3 + (double)rounds * (double)((n_groups + 3) / 4) * per + (MT == 8 && rounds > 2 ? 3.5 : 0.0);
         if (us < best.us) best = SmallPlan{cf, tiles <= 256 && MT <= 2 ? 8 : 4, us};
     }
     return best;
