@@ -121,13 +121,13 @@ int32_t sx8_v6_encode(const uint16_t* W, int64_t out_f, int64_t in_f, int64_t ld
  * f32, scales (n_cb, 2) f32 = max(lower median |c| / 3, 1e-10), coeff (n_rows * n_cb) = two signed
  * 4-bit coefficients.  blocks (n_rows * n_cb, 32), dmin and dmax all fp16 (is_f16 = 1) or all f32;
  * levels (.., 32) u8 8-byte aligned; workspace 16-byte aligned, sx8_quant_pca_workspace_bytes (-1
- * for a bad shape).  Weights with NaN give NaN scales. */
+ * for a bad shape).  Weights with infinities or NaN give NaN bases or scales.
+ * SX8_ERR_UNSUPPORTED past 65535 K blocks. */
 int64_t sx8_quant_pca_workspace_bytes(int64_t n_rows, int64_t n_cb);
 int32_t sx8_quant_pca(const void* blocks, const void* dmin, const void* dmax, int32_t is_f16,
                       const uint8_t* levels, const uint8_t* config, int64_t n_rows, int64_t n_cb,
                       uint8_t* coeff, float* data, float* scales, void* workspace,
                       int64_t workspace_bytes, void* stream);
-
 
 /* PCA precompute Z[m, kb, j] = scales[kb, j] * sum_t X[m, kb*32+t] * basis[kb, 32j+t]
  * for m < M, in float32 with the reference's summation tree.

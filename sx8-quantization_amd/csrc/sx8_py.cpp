@@ -7,7 +7,7 @@
 // Each function here does what the wrapper of the same name does for the calls a runtime makes
 // all the time -- plain device tensors of the right type -- and returns None for every other
 // call, which the wrapper then takes through its general path (conversions, copies, padding,
-// error messages).  The library's entry points are bound by address from the copy that ctypes
+// error messages); without the module every call goes there.  The library's entry points are bound by address from the copy that ctypes
 // loaded, so both paths run the same library, and as in a ctypes call the interpreter lock is
 // given up while a launch or an allocation may wait.  Nothing is kept between calls.
 #include <Python.h>

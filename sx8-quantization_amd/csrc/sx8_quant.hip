@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kThreads) void k_v6_encode(
 }
 
 // ---------------------------------------------------------------- PCA of the residuals
-// Five passes over a tensor of n_rows x n_cb blocks (bid = row * n_cb + kb):
+// Six kernels over a tensor of n_rows x n_cb blocks (bid = row * n_cb + kb):
 //   k_pca_err     residuals e = x - (lo + step lv) in float32 (every operation rounded, the
 //                 steps as products with fp32(1 / 63)), stored K block by K block
 //   k_pca_gram    partial Gram matrices E^T E of row ranges, float64 on the matrix core

@@ -4,8 +4,8 @@ Interface of scripts/integrate_fused_v44.py (reference): ``SX8LinearV44`` and
 ``clone_model_fused_v44``.  Dispatch follows integrate_fused_v44.py:43-77:
   * M <= 32               -> linear_sx8 (one HIP launch with the fp16 output and the bias: the
                              GEMV for one row, the few-row GEMM for more);
-  * M == 1 otherwise      -> decode1_v44 (a row that is not in_f long, more than 640 K blocks,
-                             a bias that is not fp16);
+  * M == 1 otherwise      -> decode1_v44 (a row that is not in_f long or not the weight's K
+                             blocks, more than 640 of them, a bias that only torch can add);
   * M > 1                 -> gemm_sx8_compact (HIP MFMA prefill on the same tensors),
                              or gemm_sx8_wmma_cached on kb-major split arrays when
                              SX8_USE_WMMA=1;

@@ -9,8 +9,8 @@ reference, which runs at module import time and cannot be imported:
     median(|c|)/3; the first two are kept (1 coeff byte, 2 bases, 2 scales).
   * ``pack_levels_6bit`` -- :148-167.
   * on a GPU the V6 encode and the packing run as one HIP kernel (``v6_encode_hip``,
-    sx8_v6_encode), bit-identical to ``v6_encode_6bit``, and the gram PCA as five more
-    (sx8_quant_pca); the outputs come to the host in one copy.
+    sx8_v6_encode), bit-identical to ``v6_encode_6bit``, and the gram PCA as six more
+    (sx8_quant_pca); the outputs come to the host in one pass of copies.
   * ``quantize_tensor``  -- the tensor loop of :235-282 and the dict layout of
     :383-395.
 
