@@ -343,7 +343,7 @@ PyObject* py_to_host(PyObject*, PyObject* const* a, Py_ssize_t na) {
     constexpr int64_t kPiece = 1 << 20;
     if (na != 2) SX8_ARGS(1)
     const at::Tensor* x = dense(a[0], at::kByte);
-    if (!x || x->numel() <= kPiece) Py_RETURN_NONE;
+    if (!x || x->numel() < 1 || (na == 1 && x->numel() <= kPiece)) Py_RETURN_NONE;
     const int64_t n = x->numel(), pieces = (n + kPiece - 1) / kPiece;
     struct Part {
         int64_t off, n;
@@ -370,21 +370,23 @@ PyObject* py_to_host(PyObject*, PyObject* const* a, Py_ssize_t na) {
         Unlocked u;
         c10::DeviceGuard on(x->device());
         for (Part& p : parts) p.y = at::empty({p.n}, at::TensorOptions().dtype(at::kByte));
-        const at::Tensor pin = at::empty({2 * kPiece}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+        const at::Tensor pin = at::empty({std::min(n, 2 * kPiece)}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
         const hipStream_t st = c10::hip::getCurrentHIPStream(x->device().index()).stream();
-        Event ev[2];
-        for (Event& v : ev) hip_ok(hipEventCreateWithFlags(&v.e, hipEventDisableTiming));
+        Event ev[2];                      // (one piece: a copy that waits, 10-15 us less than event or stream waits)
+        if (pieces > 1)
+            for (Event& v : ev) hip_ok(hipEventCreateWithFlags(&v.e, hipEventDisableTiming));
         uint8_t* const stage = static_cast<uint8_t*>(pin.data_ptr());
         auto send = [&](int64_t k) {
             const int64_t off = k * kPiece;
-            hip_ok(hipMemcpyAsync(stage + (k & 1) * kPiece, static_cast<const uint8_t*>(x->data_ptr()) + off,
-                                  std::min(kPiece, n - off), hipMemcpyDeviceToHost, st));
-            hip_ok(hipEventRecord(ev[k & 1].e, st));
+            const auto copy = pieces > 1 ? hipMemcpyAsync : hipMemcpyWithStream;
+            hip_ok(copy(stage + (k & 1) * kPiece, static_cast<const uint8_t*>(x->data_ptr()) + off,
+                        std::min(kPiece, n - off), hipMemcpyDeviceToHost, st));
+            if (pieces > 1) hip_ok(hipEventRecord(ev[k & 1].e, st));
         };
         send(0);
         for (int64_t k = 0; k < pieces; ++k) {
             if (k + 1 < pieces) send(k + 1);
-            hip_ok(hipEventSynchronize(ev[k & 1].e));
+            if (pieces > 1) hip_ok(hipEventSynchronize(ev[k & 1].e));
             const int64_t lo = k * kPiece, hi = std::min(lo + kPiece, n);
             const uint8_t* src = stage + (k & 1) * kPiece;
             for (Part& p : parts) {

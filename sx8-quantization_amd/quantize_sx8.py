@@ -157,9 +157,11 @@ class _HostFields:
         at = [(off, nb) for off, nb, _ in self.at.values()]
         host = _L.py().to_host(self.buf, tuple(at))
         if host is None:
-            whole = self.buf.cpu()
-            host = [whole[off:off + nb].clone() for off, nb in at]
-        f = {name: h.numpy().view(dt) for (name, (_, _, dt)), h in zip(self.at.items(), host)}
+            whole = self.buf.cpu().numpy()
+            host = [whole[off:off + nb].copy() for off, nb in at]
+        else:
+            host = [h.numpy() for h in host]
+        f = {name: h.view(dt) for (name, (_, _, dt)), h in zip(self.at.items(), host)}
         f["data"], f["scales"] = f["data"].reshape(self.n_cb, 64), f["scales"].reshape(self.n_cb, 2)
         return f if np.isfinite(f["data"]).all() and np.isfinite(f["scales"]).all() else None
 

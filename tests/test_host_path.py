@@ -295,6 +295,8 @@ def test_to_host_parts(hiplib, cuda):
     for (off, nb), y in zip(at, _sx8lib.py().to_host(x, at)):
         assert torch.equal(y, x[off:off + nb].cpu())
     assert len(_sx8lib.py().to_host(x, at)) == len(at)
+    small = x[:1000]
+    assert [torch.equal(y, small[a:a + 10].cpu()) for a, y in zip((0, 990), _sx8lib.py().to_host(small, ((0, 10), (990, 10))))] == [True, True]
     for bad in ((-1, 2), (0, n + 1), (n, 1)):
         with pytest.raises(ValueError):
             _sx8lib.py().to_host(x, (bad,))
