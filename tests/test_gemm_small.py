@@ -133,6 +133,10 @@ def test_linear_f16_basis_range(hiplib, cuda, M):
         assert torch.equal(scaled(2.0 ** e0, 2.0 ** e1), small), (e0, e1)
     for f in (1e-3, 3e-5, 0.2, 300.0, 7e4):
         assert near(scaled(f, f)), f
+    # a power of two of its own for every block and vector
+    e = torch.randint(-30, 30, (bas.shape[0], 2), generator=torch.Generator().manual_seed(M)).double().to(cuda)
+    b = (bas.view(-1, 2, 32).double() * 2.0 ** e[..., None]).float().view(-1, 64).contiguous()
+    assert near(linear_sx8(X, qt, hdr, lv, b, (sca.double() * 2.0 ** -e).float().contiguous()))
 
 
 @pytest.mark.gpu
