@@ -219,7 +219,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
 
     const RecSrc ws = rec_src<kSplit, HB>(mat.w, (int64_t)N * n_cb);
     sx8_rsrc xs, zs, ss;
-    const uint32_t x_off = kOdd ? (uint32_t)(reinterpret_cast<uintptr_t>(X) & 3) : 0u;    // X's place in its word
+    // X's place in its first word, which lies in X's allocation (those begin on 256 bytes)
+    const uint32_t x_off = kOdd ? (uint32_t)(reinterpret_cast<uintptr_t>(X) & 3) : 0u;
     if constexpr (kRaw) {
         xs = make_rsrc(kOdd ? reinterpret_cast<const void*>(reinterpret_cast<uintptr_t>(X) & ~(uintptr_t)3) : X,
                        ((int64_t)(M - 1) * ldx + K) * 2 + x_off);
@@ -543,8 +544,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_gemm_small(const uint16_t* _
 // launch, prologue and sum.  Fitted on packed calls, CF = 1: 1024 x 2560 at 16 / 64 / 128 rows 5.1
 // / 8.65 / 13.8 us, 2560 x 9728 at 16 / 64 rows 11.3 / 23.7, 512 x 512 at 64 rows 4.5.  Eight row
 // fragments in three rounds of work-groups take 3-4 us more than that (12288 x 512 at 128 rows 13.9
-// us, the tiled kernel 12.8).  More
-// fragments only pay where they save a round of work-groups over the CUs: gate_proj (9728
+// us, the tiled kernel 12.8).  More column fragments only pay where they save a round of work-groups over the CUs: gate_proj (9728
 // columns) at 32 rows 13.2 / 13.2 / 11.2 us with CF = 1 / 2 / 3 (608, 304, 203 tiles); with one
 // packed row fragment, whose time is all decode, they never do.  Raw rows add the basis
 // conversion and the Z products of every tile.
